@@ -6,23 +6,21 @@
 //
 //   1. tk_enum_count / tk_enum_write: the passing ids of [0, n_base), in
 //      ascending order, via GpuRoaringView::contains (any layout, negated too).
-//   2. tk_dist: grid = chunks of the passing ids x blocks of 256 queries.  Each
-//      wave keeps 32 queries in registers as the MFMA B operand and streams
-//      64-row base tiles through LDS (double buffered, rows gathered by id) as
-//      the A operand: d = ||q||^2 + ||x||^2 - 2 q.x with
-//      v_mfma_f32_32x32x2f32.  That expansion loses relative precision for
-//      near-duplicate vectors, so it only gates: a row that may beat its
-//      query's current k-th best gets its fp32 distance sum((q - x)^2)
-//      recomputed from the LDS tile, and enters the wave's candidate buffer
-//      if it does.  A full buffer is merged into per-(chunk, query) sorted
-//      top-k lists; every stored and returned distance is the direct one.
-//   3. tk_merge: one wave per query merges its chunk lists into the answer.
-// Before tk_dist, tk_pairs and tk_select run on both paths: for a small set
-// (at most the small-set limit of passing rows) tk_pairs writes every row's
-// distance estimate and tk_select picks each query's k from them, and the list
-// path's kernels exit (or are not launched when the host knows the count);
-// for a larger set they bound each query's k-th distance from the first rows,
-// the bound tk_dist starts from.
+//   2. tk_est: distance estimates on the matrix cores, from a two-way f16 split
+//      of scaled rows and queries (three f16 MFMA products per fp32 one, with
+//      an error no larger than with an fp32 MFMA).  A set of at most `keep` rows
+//      gets every estimate written and tk_select picks each query's k from
+//      them.  A larger one runs it twice: over a strided sample, from which
+//      tk_select bounds each query's k-th distance, and then over every row,
+//      where each (query, row) whose estimate could lie at or below that bound
+//      is appended to the query's candidate lists.
+//   3. tk_select: the candidates that can be in the answer get their fp32
+//      distance sum((q - x)^2), are ranked by (distance, id), and the first k
+//      are written.  Every returned distance is the direct one.
+// The estimates only ever gate, with a bound on their error, so the answer does
+// not depend on them.  When a query's candidate lists overflow (or the
+// small-set path is turned off), tk_dist and tk_merge answer: per-chunk sorted
+// lists under an fp32 MFMA gate, merged by one wave per query.
 #include <algorithm>
 #include <atomic>
 #include <cstring>
@@ -57,24 +55,13 @@ constexpr float TK_GATE_ERR = 4e-5f;
 // distance; adding TK_SEED_ERR (qg + xg) makes it at least the fp32 distance
 // (2 E / (1 - E) with E = TK_GATE_ERR, rounded up for the fp32 arithmetic).
 constexpr float TK_SEED_ERR = 3.0f * TK_GATE_ERR;
+// The same bound for the split estimates (tk_est): 3 x 128 products summed
+// at no more than 2^-23 of |q||x| each (4.7e-5 of |q|^2 + |x|^2 with the factor
+// 2 of -2 q.x), the split's remainders (2^-22 an element on each side and the
+// dropped lo.lo product, 1e-6), the norms and the direct sum (2.3e-5).
+constexpr float TK_EST_ERR = 8e-5f;
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-// Order-preserving map of fp32 values to u32 (and back).
-__device__ __forceinline__ uint32_t tk_ordered(float f)
-{
-    const uint32_t b = __float_as_uint(f);
-    return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
-}
-
-__device__ __forceinline__ float tk_unordered(uint32_t u)
-{
-    return __uint_as_float((u & 0x80000000u) ? (u & 0x7FFFFFFFu) : ~u);
-}
-
-// Upper bound of a row's fp32 distance from its estimate (a lower bound) and
-// the scaled norms; one fused operation, so every kernel computes the same value.
-__device__ __forceinline__ float tk_upper(float est, float qg, float xg) { return __fmaf_rn(TK_SEED_ERR, qg + xg, est); }
 
 // Strict order of (distance, id) pairs: the output order.
 __device__ __forceinline__ bool tk_less(float ad, uint32_t ai, float bd, uint32_t bi)
@@ -118,54 +105,42 @@ struct TkArgs {
     uint32_t* tau;      // [n_q] bits of the smallest k-th distance any chunk has reached
     uint32_t* tau_m;    // [n_chunks][n_q] bits of each chunk's m_rank-th distance (+inf: fewer entries)
     uint32_t m_rank;    // ceil(2k / n_chunks)
-    // Small sets: with at most small_max rows the distance kernel writes every
-    // estimate (pd[q][row], lower bounds of the fp32 distances) with the scaled
-    // norms (pq[q], px[row]), and tk_select picks each query's k from them.
-    uint32_t small_max;  // 0: never
-    float* pd;           // [n_qb * TK_QB][small_max] (rows past n_q unused)
-    float* pq;           // [n_q]
-    float* px;           // [small_max]
-    uint32_t* qlo;       // [n_q] order-preserving bits of the smallest upper bound of the query's rows
-    uint32_t* qhi;       // [n_q] ... and of the largest
-    // The host knew the passing count to be within small_max (no filter and a
-    // small base, or a filter's recorded cardinality) and launched no list
-    // path; tk_select then answers any count (every row a candidate past it).
+    // The estimate path (gate != 0): sets of at most `keep` rows have every
+    // estimate written to pd[q][row], larger ones those of `sample` rows (a
+    // power of two, 1 << sample_lg) and then candidates in lists.
+    uint32_t gate;
+    uint32_t keep;
+    uint32_t sample;
+    uint32_t sample_lg;
+    uint32_t pd_stride;  // row stride of pd: at least keep and sample
+    float* pd;           // [whole query blocks][pd_stride] estimates (lower bounds of the fp32 distances)
+    uint32_t n_cw;       // candidate lists a query has: one per workgroup of its query block
+    uint32_t cap;        // entries of a list
+    uint32_t q_rows;     // queries of whole query blocks
+    uint2* cand;         // [n_cw][q_rows][cap] (estimate bits, id)
+    uint32_t* cand_n;    // [n_cw][q_rows] candidates found, beyond cap too
+    uint32_t* q_over;    // [n_q] the query's lists overflowed: tk_dist and tk_merge answer it
+    uint32_t* qb_over;   // [n_qb] ... any query of the block's
+    // What the host launched, from the passing count it knew: with no
+    // candidate kernels (or no list path), tk_select answers a set too large
+    // (or a query whose lists overflowed) from every passing row.
+    uint32_t cand_off;
     uint32_t list_off;
 };
 
-// Rows the distance kernel covers, and whether the small-set path takes them.
+// Rows the distance kernels cover, and whether every estimate of them is kept.
 __device__ __forceinline__ uint64_t tk_rows(const TkArgs& a) { return a.sel ? static_cast<uint64_t>(*a.n_sel) : a.n_base; }
-__device__ __forceinline__ bool tk_small(const TkArgs& a, uint64_t n_rows)
-{
-    return a.small_max != 0 && n_rows <= a.small_max;
-}
-// Larger sets: the small-set kernels first bound each query's k-th distance
-// from the upper bounds of the first rows (at most small_max of them), and the
-// list path starts from that bound instead of from +inf.
-constexpr uint32_t TK_SEED_ROWS = 16384;
-constexpr uint32_t TK_SEED_ROWS_PER_K = 256;
-__device__ __forceinline__ uint32_t tk_seed_rows(const TkArgs& a, uint64_t n_rows)
-{
-    if (a.small_max == 0 || tk_small(a, n_rows)) return 0;
-    const uint64_t want = std::max<uint64_t>(TK_SEED_ROWS, static_cast<uint64_t>(TK_SEED_ROWS_PER_K) * a.k);
-    return static_cast<uint32_t>(std::min<uint64_t>(std::min<uint64_t>(n_rows, a.small_max), want));
-}
+__device__ __forceinline__ bool tk_small(const TkArgs& a, uint64_t n_rows) { return a.gate != 0 && n_rows <= a.keep; }
 
-// The call's state: every query's bound (tau) and each chunk's m_rank-th
-// distance (tau_m) at +inf, and for the small-set path the range of the upper
-// bounds (qlo at the largest value, qhi at the smallest); thread i of `stride`.
+// The list path's state when nothing else sets it: every query's bound (tau)
+// and each chunk's m_rank-th distance (tau_m) at +inf; thread i of `stride`.
 __device__ __forceinline__ void tk_init_from(const TkArgs& a, uint64_t i, uint64_t stride)
 {
-    const uint64_t n = std::max<uint64_t>(static_cast<uint64_t>(a.n_chunks) * a.n_q, a.n_q);
+    if (a.gate) return;
+    const uint64_t n = static_cast<uint64_t>(a.n_chunks) * a.n_q;
     for (; i < n; i += stride) {
-        if (i < static_cast<uint64_t>(a.n_chunks) * a.n_q) a.tau_m[i] = 0x7F800000u;
-        if (i < a.n_q) {
-            a.tau[i] = 0x7F800000u;
-            if (a.small_max) {
-                a.qlo[i] = 0xFFFFFFFFu;
-                a.qhi[i] = 0u;
-            }
-        }
+        a.tau_m[i] = 0x7F800000u;
+        if (i < a.n_q) a.tau[i] = 0x7F800000u;
     }
 }
 
@@ -587,7 +562,7 @@ __global__ __launch_bounds__(TK_NT) void tk_dist(TkArgs a)
     const uint32_t qb = pidx % n_qb;
 
     const uint64_t n_rows = tk_rows(a);
-    if (tk_small(a, n_rows)) return;  // tk_pairs and tk_select answer small sets
+    if (a.gate && (n_rows <= a.keep || !a.qb_over[qb])) return;  // tk_select has answered
     const uint64_t rpc = ((n_rows + a.n_chunks - 1) / a.n_chunks + TK_ROWS - 1) / TK_ROWS * TK_ROWS;
     const uint64_t r0 = std::min<uint64_t>(n_rows, static_cast<uint64_t>(chunk) * rpc);
     const uint64_t r1 = std::min<uint64_t>(n_rows, r0 + rpc);
@@ -614,7 +589,7 @@ __global__ __launch_bounds__(TK_NT) void tk_dist(TkArgs a)
     const float qpart = tk_load_query<DP>(a, qok, q0 + j, h, qreg);
     const float qg = (1.f - TK_GATE_ERR) * (qpart + __shfl_xor(qpart, 32, 64));
 
-    // The prefetch as in tk_pairs: tile t + 1's rows (ids known since tile
+    // The prefetch as in tk_est: tile t + 1's rows (ids known since tile
     // t - 1) and tile t + 2's raw ids are issued before tile t's MFMA and
     // waited for after it.
     auto tile_r0 = [&](uint32_t i) { return r0 + static_cast<uint64_t>(i) * TK_ROWS; };
@@ -832,7 +807,7 @@ __global__ __launch_bounds__(TK_MERGE_NT) void tk_merge(TkArgs a, const float* l
                                                          size_t plane, const uint32_t* list_n, uint32_t n_chunks,
                                                          uint32_t n_q, uint32_t k, float* out_d, int64_t* out_id)
 {
-    if (tk_small(a, tk_rows(a))) return;  // tk_select answers small sets
+    if (tk_small(a, tk_rows(a))) return;  // tk_select has answered
     constexpr int W = TK_MERGE_NT / 64;
     __shared__ float ad[W][2][TK_KMAX];
     __shared__ uint32_t ai[W][2][TK_KMAX];
@@ -842,6 +817,7 @@ __global__ __launch_bounds__(TK_MERGE_NT) void tk_merge(TkArgs a, const float* l
     const uint32_t w = threadIdx.x >> 6;
     const uint32_t q = blockIdx.x * W + w;
     if (q >= n_q) return;  // whole wave; no block barrier below
+    if (a.gate && !a.q_over[q]) return;
     uint32_t n = 0;
     int cur = 0;
     // The next chunk's list is loaded into registers (k <= 256: four entries a
@@ -903,301 +879,660 @@ __global__ __launch_bounds__(TK_MERGE_NT) void tk_merge(TkArgs a, const float* l
     }
 }
 
-// ---- 2b. small sets: every estimate ------------------------------------------
-// The distance kernel's tiles and MFMA blocks without the selection: each
-// (chunk, query block) workgroup writes the estimates of its rows for its
-// queries -- (1 - TK_GATE_ERR)(|q|^2 + |x|^2) - 2 q.x, at most the fp32
-// distance -- to pd[q][row], the scaled query norms to pq (chunk 0) and the
-// scaled row norms to px (query block 0).
-// Rows whose upper bounds set the first bound: a larger sample costs reads, a
-// smaller one admits about k * rows / sample candidates, each a gathered row.
-constexpr uint32_t TK_SEL_SAMPLE = 16384;
-constexpr uint32_t TK_SEL_SAMPLE_PER_K = 1024;
-// The upper bounds' range matters only over the rows a histogram reads: the
-// selection's sample, which includes every seed row (at most 256 k of them).
-__device__ __forceinline__ uint64_t tk_hist_rows(const TkArgs& a)
-{
-    return max(TK_SEL_SAMPLE, TK_SEL_SAMPLE_PER_K * a.k);
-}
+// ---- 2b. estimates on split f16 MFMA --------------------------------------------
+// q.x from f16 halves: a row is scaled by a power of two that brings its norm
+// into [2^14, 2^15), then x = hi + lo with hi = f16(x) and lo = f16(x - hi), and
+// the same for the query; hi.hi + lo.hi + hi.lo accumulate in fp32 in one MFMA
+// chain.  The remainders are 2^-22 of an element (2^-29 of the row's norm where
+// lo is below f16's normal range), under the fp32 accumulation's own rounding;
+// v_mfma_f32_32x32x16_f16 runs at 16 times the fp32 MFMA rate, so three of them
+// cost 3/16 of the fp32 product.
+//
+// A rank-2 product (one fp32 MFMA) then brings the accumulator to
+//   sx sq (2 q.x - |x|^2 - |q|^2 + gate) / 2
+// (sx, sq the scales; the norms shrunk by 1 - TK_EST_ERR): a row can lie at or
+// below the query's gate exactly when it is >= 0, one maximum over the
+// accumulator's registers and one test per 32 x 32 pairs.  With gate = 0 it is
+// the estimate times -sx sq / 2.  The norms come last so that the products are
+// rounded at their own size, as an fp32 MFMA's are before its norms are added.
+//
+// A workgroup's eight waves are QG query groups of 32 QW queries (their halves
+// live in registers) by RG row groups of 32 rows; a tile of 32 RG rows goes
+// through LDS once for all of them, split as it is stored.  Large query counts
+// take 256 queries a workgroup (QW 2, QG 4): the MFMA work per tile covers its
+// conversion; up to 64 queries are bound by reading the rows and take 128-row
+// tiles (QW 1, QG 2).
+// Measured (10M x 128, 1M passing rows, 1024 queries): 706-741 us for the candidate
+// kernel, against 2505 us of fp32 MFMA with sorted lists; the MFMAs alone 480 us.
+// 300K x 100 unfiltered rows, 64 queries: 32 us (3.8 TB/s of rows), against 189 us and
+// 224 us more for merging 256 lists a query.
+// The estimate's error against fp64, 32 x 32 blocks of 17 to 128 dimensions
+// (normal, positive, and over 2^20 of magnitudes), rms of |q|^2 + |x|^2:
+// 5.5e-8 to 1.45e-7, with fp32 MFMA 6.4e-8 to 1.73e-7 (lower in each block).
+constexpr uint32_t TK_KEEP = 16384;         // rows whose estimates are all kept, and the sample, at most
+constexpr uint32_t TK_SCRATCH = 1u << 30;   // bytes of estimates, and of candidate lists, at most
+constexpr uint32_t TK_CAND_CAP = 2048;      // candidates a list holds where it cannot hold every row
+constexpr uint32_t TK_TWO_STAGE = 1024;     // expected candidates a query above which a second bound pays
+constexpr float TK_GATE_ROUND = 0x1p-20f;   // rounding of a stored estimate, relative to the gate
 
-constexpr int TK_ES = TK_ROWS + 4;  // estimate staging: a query's 64 rows, 16-byte aligned
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));  // (a float4 struct's load is split where two paths merge)
 
-template <int DP>
-struct TkPairsLds {
-    float tile[2][TK_ROWS * (DP + 4)];
-    float xg[2][TK_ROWS];
-    uint32_t id[2][TK_ROWS];
-    float est[TK_WAVES][TK_QW * TK_ES];  // a wave's 32 x 64 estimates
+template <int KS, int QW, int QG>
+struct TkEst {
+    static constexpr int RG = TK_WAVES / QG;
+    static constexpr int T = 32 * RG;         // rows of a tile
+    static constexpr int QB = 32 * QW * QG;   // queries of a workgroup
+    static constexpr int DP = 16 * KS;        // padded dimensions
+    // Eight threads load a row: thread l takes dimensions 8 l .. + 7 and, past
+    // 64 dimensions, 64 + 8 l .. + 7.  More threads a row would spend more on
+    // its norm and scale than on its elements.
+    static constexpr int TPR = 8;
+    static constexpr int V = DP > 64 ? 16 : 8;  // elements a thread
+    static constexpr int RPP = TK_NT / TPR;   // rows per pass
+    static constexpr int P = T / RPP;         // passes
+    static constexpr int RS = DP + 8;         // row stride in LDS: conflict-free 16-byte reads
 };
 
-template <int DP, bool SEL>
-__global__ __launch_bounds__(TK_NT) void tk_pairs(TkArgs a)
+struct alignas(16) TkRow {
+    float u, z;  // the rank-2 product's row factors: -sx |x|^2 / 2 and sx
+    float isx;   // 1 / sx
+    uint32_t id;
+};
+
+template <int KS, int QW, int QG>
+struct TkEstLds {
+    using C = TkEst<KS, QW, QG>;
+    alignas(16) _Float16 hi[2][C::T * C::RS];
+    alignas(16) _Float16 lo[2][C::T * C::RS];
+    TkRow row[2][C::T];
+    alignas(16) float isq[C::QB];
+};
+
+// What the candidates need beside it.  A wave appends its candidates to a
+// buffer and writes them to their lists when it is nearly full: a store to
+// memory in the tile loop would make the next wait for a tile's rows wait for
+// the store too (both count in order).
+template <int QB>
+struct TkGateLds {
+    static constexpr uint32_t WB = QB == 256 ? 512 : 192;  // entries a wave (LDS left by the tiles)
+    float2 gq[QB];  // an estimate is gq.x - acc gq.y / sx
+    uint32_t cnt[QB];
+    uint2 buf[TK_WAVES][WB];    // (estimate bits, id)
+    uint16_t lq[TK_WAVES][WB];  // query within the workgroup
+};
+
+// Scale for a squared norm: the power of two that brings the norm into
+// [2^14, 2^15).  Norms outside [2^-30, 2^30] (zero aside, whose scale is 1) are
+// not estimated: `odd`.
+__device__ __forceinline__ float tk_scale(float ss, float& inv, bool& odd)
 {
-    // Every row of a small set, or the seed rows of a larger one.
-    const uint64_t all_rows = tk_rows(a);
-    const uint64_t n_rows = tk_small(a, all_rows) ? all_rows : tk_seed_rows(a, all_rows);
-    if (n_rows == 0) return;
-    __shared__ TkPairsLds<DP> L;
+    const uint32_t e = __float_as_uint(ss) >> 23;  // ss >= 0: its biased exponent (NaN: past the range)
+    odd = ss != 0.f && (e < 127u - 60u || e > 127u + 60u);
+    const bool unit = odd || ss == 0.f;
+    const uint32_t sh = (e + 1u) >> 1;  // floor(log2 ss / 2) + 64, for the odd bias
+    const uint32_t se = unit ? 127u : 127u + 14u + 64u - sh;
+    inv = __uint_as_float((254u - se) << 23);
+    return __uint_as_float(se << 23);
+}
+
+// hi and lo halves of two scaled values.
+__device__ __forceinline__ void tk_split(float a, float b, f16x2& hi, f16x2& lo)
+{
+    const f32x2 v = {a, b};
+    hi = __builtin_convertvector(v, f16x2);
+    const f32x2 r = {fmaf(static_cast<float>(hi.x), -1.f, a), fmaf(static_cast<float>(hi.y), -1.f, b)};
+    lo = __builtin_convertvector(r, f16x2);
+}
+
+// Which rows a launch covers: every row or the sample (row i stands for
+// i * rows / sample), and which tiles of them.
+struct TkSpan {
+    uint64_t rows;   // the set's
+    uint64_t n;      // rows of this launch
+    uint32_t lg;     // log2 of the sample's size, 0 for every row
+};
+
+template <class C, bool SEL>
+__device__ __forceinline__ void tk_est_ids(const TkArgs& a, const TkSpan& sp, uint64_t r0, uint32_t (&raw)[C::P])
+{
+#pragma unroll
+    for (int p = 0; p < C::P; ++p) {
+        uint64_t r = std::min<uint64_t>(r0 + p * C::RPP + threadIdx.x / C::TPR, sp.n - 1);
+        if (sp.lg) r = (r * sp.rows) >> sp.lg;
+        raw[p] = SEL ? a.sel[r] : static_cast<uint32_t>(r);
+    }
+}
+
+template <class C>
+__device__ __forceinline__ void tk_est_valid(uint64_t r0, uint64_t n, uint32_t (&id)[C::P])
+{
+#pragma unroll
+    for (int p = 0; p < C::P; ++p)
+        if (r0 + p * C::RPP + threadIdx.x / C::TPR >= n) id[p] = TK_NOID;
+}
+
+// A thread's elements of its rows (dimensions past dim repeat the last; they are
+// zeroed where they are used, so that nothing waits for a load where it is issued).
+template <class C>
+__device__ __forceinline__ uint32_t tk_est_col(int e)
+{
+    return (threadIdx.x % C::TPR) * 8u + (e < 8 ? 0u : 64u) + (e & 7u);
+}
+
+template <class C>
+__device__ __forceinline__ void tk_est_rows(const TkArgs& a, const uint32_t (&id)[C::P], float (&pre)[C::P][C::V])
+{
+#pragma unroll
+    for (int p = 0; p < C::P; ++p) {
+        const float* src = a.base + static_cast<size_t>(id[p] != TK_NOID ? id[p] : 0u) * a.dim;
+        if (a.vec) {
+#pragma unroll
+            for (int e = 0; e < C::V; e += 4) {
+                const f32x4 v = *reinterpret_cast<const f32x4*>(src + min(tk_est_col<C>(e), a.dim - 4u));
+                pre[p][e] = v.x, pre[p][e + 1] = v.y, pre[p][e + 2] = v.z, pre[p][e + 3] = v.w;
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < C::V; ++e) pre[p][e] = src[min(tk_est_col<C>(e), a.dim - 1u)];
+        }
+    }
+}
+
+template <class C, class Lds>
+__device__ __forceinline__ void tk_est_store(const TkArgs& a, Lds& L, int buf, const float (&pre)[C::P][C::V],
+                                             const uint32_t (&id)[C::P])
+{
+    const uint32_t l = threadIdx.x % C::TPR;
+#pragma unroll
+    for (int p = 0; p < C::P; ++p) {
+        const int row = p * C::RPP + static_cast<int>(threadIdx.x / C::TPR);
+        float v[C::V];
+        float ss = 0.f;
+#pragma unroll
+        for (int e = 0; e < C::V; ++e) {
+            v[e] = tk_est_col<C>(e) < a.dim ? pre[p][e] : 0.f;
+            ss = fmaf(v[e], v[e], ss);
+        }
+        ss = tk_group_sum<8>(ss);
+        float inv;
+        bool odd;
+        const float sx = tk_scale(ss, inv, odd);
+        if (__ballot(odd)) {  // rows that are not estimated multiply as zeros ...
+#pragma unroll
+            for (int e = 0; e < C::V; ++e) v[e] = odd ? 0.f : v[e];
+        }
+        _Float16* H = &L.hi[buf][row * C::RS + 8 * l];
+        _Float16* W = &L.lo[buf][row * C::RS + 8 * l];
+#pragma unroll
+        for (int c = 0; c < C::V; c += 8) {
+            f16x8 hv, lv;
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                f16x2 hi, lo;
+                tk_split(v[c + e] * sx, v[c + e + 1] * sx, hi, lo);
+                hv[e] = hi.x, hv[e + 1] = hi.y, lv[e] = lo.x, lv[e + 1] = lo.y;
+            }
+            if (8 * l + 8 * c < C::DP) {
+                *reinterpret_cast<f16x8*>(H + 8 * c) = hv;
+                *reinterpret_cast<f16x8*>(W + 8 * c) = lv;
+            }
+        }
+        if (l == 0) {  // ... and their factor makes them pass every gate, or (past the last row) none
+            TkRow r;
+            r.u = id[p] == TK_NOID ? -__builtin_inff() : odd ? __builtin_inff() : -0.5f * (1.f - TK_EST_ERR) * ss * sx;
+            r.z = sx;
+            r.isx = inv;
+            r.id = id[p];
+            L.row[buf][row] = r;
+        }
+    }
+}
+
+// GATE false: estimates of a small set or of the sample, into pd.  GATE true:
+// candidates of a larger set; `stage` 0 takes every tile, 1 every 16th, 2 the
+// others (the counts then continue).
+constexpr uint32_t TK_STAGE = 16;
+
+template <int KS, int QW, int QG, bool SEL, bool GATE>
+__global__ __launch_bounds__(TK_NT) void tk_est(TkArgs a, uint32_t n_qb, uint32_t stage)
+{
+    using C = TkEst<KS, QW, QG>;
+    const uint64_t rows = tk_rows(a);
+    const bool small = rows <= a.keep;
+    if (rows == 0 || (GATE && small)) return;
+    TkSpan sp;
+    sp.rows = rows;
+    sp.lg = !GATE && !small && rows > a.sample ? a.sample_lg : 0u;
+    sp.n = sp.lg ? a.sample : rows;
+    // The workgroups of a query block take its tiles in turn.  Blocks are
+    // dispatched round-robin over the 8 XCDs: an XCD's blocks take consecutive
+    // query blocks of the same tiles, which then share the rows in its L2.
+    const uint32_t pidx = (blockIdx.x % 8u) * (gridDim.x / 8u) + blockIdx.x / 8u;
+    const uint32_t chunk = pidx / n_qb, qb = pidx % n_qb;
+    if (chunk >= a.n_cw) return;
+    const uint64_t all = (sp.n + C::T - 1) / C::T;
+    const uint64_t first = (all + TK_STAGE - 1) / TK_STAGE;  // tiles of stage 1
+    const uint64_t part = stage == 0 ? all : stage == 1 ? first : all - first;
+    const uint32_t n_tiles = chunk < part ? static_cast<uint32_t>((part - chunk + a.n_cw - 1) / a.n_cw) : 0u;
+    auto tile_r0 = [&](uint32_t i) -> uint64_t {
+        const uint64_t g = chunk + static_cast<uint64_t>(i) * a.n_cw;
+        const uint64_t t = stage == 0 ? g : stage == 1 ? g * TK_STAGE : g + g / (TK_STAGE - 1) + 1;
+        return t * C::T;
+    };
+    __shared__ TkEstLds<KS, QW, QG> L;
+    using Gate = TkGateLds<GATE ? C::QB : 1>;
+    __shared__ Gate G;
     const uint32_t lane = __lane_id();
     const uint32_t wave = threadIdx.x >> 6;
-    const uint32_t h = lane >> 5;
-    const uint32_t j = lane & 31u;
-    // The workgroups of a query block take its tiles in turn: tile c, c + n_cw,
-    // ... (the grid is n_cw x n_qb, balanced however many rows there are).
-    const uint32_t n_qb = (a.n_q + TK_QB - 1) / TK_QB;
-    const uint32_t n_cw = gridDim.x / n_qb;
-    const uint32_t chunk = blockIdx.x / n_qb;
-    const uint32_t qb = blockIdx.x % n_qb;
-    const uint64_t n_all = (n_rows + TK_ROWS - 1) / TK_ROWS;
-    const uint32_t n_tiles = chunk < n_all ? static_cast<uint32_t>((n_all - chunk + n_cw - 1) / n_cw) : 0u;
-    auto tile_r0 = [&](uint32_t i) { return (static_cast<uint64_t>(chunk) + static_cast<uint64_t>(i) * n_cw) * TK_ROWS; };
-    auto tile_r1 = [&](uint32_t i) { return std::min<uint64_t>(n_rows, tile_r0(i) + TK_ROWS); };
-    const uint32_t q0 = qb * TK_QB + wave * TK_QW;
-    const uint32_t uq0 = __builtin_amdgcn_readfirstlane(q0);  // the same, known to be wave-uniform
-    const uint32_t nq_wave = q0 < a.n_q ? std::min<uint32_t>(TK_QW, a.n_q - q0) : 0u;
-    const bool qok = j < nq_wave;
-    float qreg[DP / 2];
-    const float qpart = tk_load_query<DP>(a, qok, q0 + j, h, qreg);
-    const float qg = (1.f - TK_GATE_ERR) * (qpart + __shfl_xor(qpart, 32, 64));
-    if (chunk == 0 && h == 0 && qok) a.pq[q0 + j] = qg;
-    float4 pre[DP / 32];
-    uint32_t pid[DP / 32], nid[DP / 32];  // ids of the next tile, and (raw) of the one after it
-    const uint64_t last = n_rows - 1;
-    // A tile's loads are all issued before the previous tile's MFMA and
-    // waited for after it: the rows of tile t + 1 (their ids known since
-    // tile t - 1) and the ids of tile t + 2.  Every iteration prefetches (a tile
-    // past the last has no valid rows and is never read), so no branch skips
-    // a load and the one wait of an iteration comes after its MFMA.
-    tk_ids_raw<DP, SEL>(a, tile_r0(1), last, nid);
+    const uint32_t rg = wave % C::RG, qg = wave / C::RG;
+    const uint32_t h = lane >> 5, j = lane & 31u;
+    const uint32_t lq0 = qg * 32u * QW;  // the wave's first query within the workgroup
+    const uint32_t q0 = qb * C::QB + lq0;
+    const bool busy = q0 < a.n_q;  // wave-uniform
+
+    float pre[C::P][C::V];
+    uint32_t id[C::P], nid[C::P];
     if (n_tiles > 0) {
-        tk_load_rows<DP>(a, tile_r0(0), tile_r1(0), pre, pid);
-        tk_store_rows<DP>(L, 0, pre, pid);
+        tk_est_ids<C, SEL>(a, sp, tile_r0(0), id);
+        tk_est_ids<C, SEL>(a, sp, tile_r0(1), nid);
+        tk_est_valid<C>(tile_r0(0), sp.n, id);
+        tk_est_rows<C>(a, id, pre);
     }
+
+    // A operand: the wave's queries, split, dimensions 16 s + 8 h .. + 7 a lane.
+    f16x8 qh[QW][KS], ql[QW][KS];
+    float vw[QW];  // the rank-2 product's query factors: sq (lanes 0-31), (gate - |q|^2) sq / 2 (lanes 32-63)
 #pragma unroll
-    for (int p = 0; p < DP / 32; ++p) pid[p] = nid[p];
-    tk_ids_valid<DP>(tile_r0(1), tile_r1(1), pid);
+    for (int f = 0; f < QW; ++f) {
+        const uint32_t q = q0 + 32u * f + j;
+        const bool ok = q < a.n_q;
+        const float* src = a.queries + static_cast<size_t>(ok ? q : 0u) * a.dim;
+        float x[8 * KS];
+        if (a.qvec) {
+#pragma unroll
+            for (int e = 0; e < 8 * KS; e += 4) {
+                const f32x4 v = *reinterpret_cast<const f32x4*>(src + min(16u * (e / 8) + 8u * h + e % 8, a.dim - 4u));
+                x[e] = v.x, x[e + 1] = v.y, x[e + 2] = v.z, x[e + 3] = v.w;
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8 * KS; ++e) x[e] = src[min(16u * (e / 8) + 8u * h + e % 8, a.dim - 1u)];
+        }
+        float ss = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8 * KS; ++e) {
+            x[e] = ok && 16u * (e / 8) + 8u * h + e % 8 < a.dim ? x[e] : 0.f;
+            ss += x[e] * x[e];
+        }
+        ss += __shfl_xor(ss, 32, 64);
+        float inv;
+        bool odd;
+        const float sq = tk_scale(ss, inv, odd);
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                f16x2 hi, lo;
+                tk_split(odd ? 0.f : x[8 * s + e] * sq, odd ? 0.f : x[8 * s + e + 1] * sq, hi, lo);
+                qh[f][s][e] = hi.x, qh[f][s][e + 1] = hi.y;
+                ql[f][s][e] = lo.x, ql[f][s][e + 1] = lo.y;
+            }
+        const float gate = GATE && ok ? __uint_as_float(a.tau[q]) : 0.f;
+        const bool pass = odd || !(gate < __builtin_inff());  // every row is a candidate
+        const float qgn = (1.f - TK_EST_ERR) * ss;
+        vw[f] = h == 0 ? (ok ? sq : 0.f) : !ok ? -__builtin_inff() : pass ? __builtin_inff() : 0.5f * (gate - qgn) * sq;
+        if (rg == 0 && h == 0) {
+            L.isq[lq0 + 32u * f + j] = inv;
+            if (GATE) {
+                G.gq[lq0 + 32u * f + j] = make_float2(pass ? -__builtin_inff() : gate - TK_GATE_ROUND * gate, 2.f * inv);
+                G.cnt[lq0 + 32u * f + j] =
+                    stage == 2 ? a.cand_n[static_cast<size_t>(chunk) * a.q_rows + q] : 0u;
+            }
+        }
+    }
+    // A tile into LDS, from registers that were loaded a
+    // tile ago; then the rows of the tile after it (their ids known since the
+    // last tile) and the ids of the one after that.  Past the last tile they
+    // repeat valid rows that nothing reads.
+    auto next = [&](uint32_t t, int buf) {
+        if (t < n_tiles) tk_est_store<C>(a, L, buf, pre, id);
+#pragma unroll
+        for (int p = 0; p < C::P; ++p) id[p] = nid[p];
+        tk_est_valid<C>(tile_r0(t + 1), t + 1 < n_tiles ? sp.n : 0, id);
+        tk_est_rows<C>(a, id, pre);
+        tk_est_ids<C, SEL>(a, sp, tile_r0(t + 2), nid);
+    };
+    if (n_tiles > 0) next(0, 0);
     __syncthreads();
-    float ulo = __builtin_inff(), uhi = -__builtin_inff();  // range of the upper bounds of this lane's rows
+
+    // The workgroup's lists (TK_SCRATCH bounds them: 32-bit offsets).
+    uint2* cand = GATE ? a.cand + (static_cast<size_t>(chunk) * a.q_rows + qb * C::QB) * a.cap : nullptr;
+    uint32_t held = 0;  // candidates in the wave's buffer (uniform)
+    auto drain = [&]() {
+        wave_lds_fence();
+        for (uint32_t i = lane; i < held; i += 64) {
+            const uint32_t lq = G.lq[wave][i];
+            const uint32_t slot = atomicAdd(&G.cnt[lq], 1u);
+            if (slot < a.cap) cand[lq * a.cap + slot] = G.buf[wave][i];
+        }
+        wave_lds_fence();
+        held = 0;
+    };
+    // Waves 0-3 (one a SIMD) multiply first and convert the next tile then,
+    // waves 4-7 the other way round: a SIMD's matrix unit works for one of its
+    // two waves while its vector unit converts for the other.
+    const bool late = __builtin_amdgcn_readfirstlane(wave) >= 4;
     for (uint32_t t = 0; t < n_tiles; ++t) {
         const int b = static_cast<int>(t & 1u);
-        tk_load_rows_nb<DP>(a, pid, pre);
-        tk_ids_raw<DP, SEL>(a, tile_r0(t + 2), last, nid);
-        if (nq_wave > 0) {
-            f32x16 acc0 = {}, acc1 = {};
-            const float* A0 = &L.tile[b][j * (DP + 4) + h * (DP / 2)];
-            const float* A1 = A0 + 32 * (DP + 4);
+        if (late) next(t + 1, b ^ 1);
+        if (busy) {
+            f32x16 acc[QW];
+            const TkRow* R = &L.row[b][rg * 32u + j];
+            const float uz = h == 0 ? R->u : R->z;
 #pragma unroll
-            for (int s = 0; s < DP / 2; s += 4) {
-                const float4 x0 = *reinterpret_cast<const float4*>(A0 + s);
-                const float4 x1 = *reinterpret_cast<const float4*>(A1 + s);
-                acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(x0.x, qreg[s + 0], acc0, 0, 0, 0);
-                acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(x1.x, qreg[s + 0], acc1, 0, 0, 0);
-                acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(x0.y, qreg[s + 1], acc0, 0, 0, 0);
-                acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(x1.y, qreg[s + 1], acc1, 0, 0, 0);
-                acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(x0.z, qreg[s + 2], acc0, 0, 0, 0);
-                acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(x1.z, qreg[s + 2], acc1, 0, 0, 0);
-                acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(x0.w, qreg[s + 3], acc0, 0, 0, 0);
-                acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(x1.w, qreg[s + 3], acc1, 0, 0, 0);
+            for (int f = 0; f < QW; ++f) acc[f] = f32x16{};
+            const _Float16* H = &L.hi[b][(rg * 32u + j) * C::RS + 8u * h];
+            const _Float16* W = &L.lo[b][(rg * 32u + j) * C::RS + 8u * h];
+            // hi.hi last for few dimensions, the cross products with it for
+            // many, which saves keeping or reading the row's halves twice.
+            constexpr bool CROSS_FIRST = KS <= 4;
+            f16x8 xh[KS];
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                xh[s] = *reinterpret_cast<const f16x8*>(H + 16 * s);
+                const f16x8 xl = *reinterpret_cast<const f16x8*>(W + 16 * s);
+                if constexpr (!CROSS_FIRST) {
+#pragma unroll
+                    for (int f = 0; f < QW; ++f) acc[f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(qh[f][s], xh[s], acc[f], 0, 0, 0);
+                }
+#pragma unroll
+                for (int f = 0; f < QW; ++f) acc[f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ql[f][s], xh[s], acc[f], 0, 0, 0);
+#pragma unroll
+                for (int f = 0; f < QW; ++f) acc[f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(qh[f][s], xl, acc[f], 0, 0, 0);
             }
-            // Through LDS, so each store writes 64 consecutive rows of four
-            // queries.  Accumulator registers 4m .. 4m + 3 of a block hold four
-            // consecutive rows (tk_row), one 16-byte LDS access.
-            float* E = L.est[wave];
-            const int rows = static_cast<int>(tile_r1(t) - tile_r0(t));  // rows of this tile
-            const bool track = tile_r0(t) < tk_hist_rows(a);  // uniform
+            if constexpr (CROSS_FIRST) {
 #pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                const int ra = tk_row(4 * m, static_cast<int>(h)), rb = tk_row(16 + 4 * m, static_cast<int>(h));
-                const float4 ga = *reinterpret_cast<const float4*>(&L.xg[b][ra]);
-                const float4 gb = *reinterpret_cast<const float4*>(&L.xg[b][rb]);
-                const float4 ea = make_float4(qg + ga.x - 2.f * acc0[4 * m + 0], qg + ga.y - 2.f * acc0[4 * m + 1],
-                                              qg + ga.z - 2.f * acc0[4 * m + 2], qg + ga.w - 2.f * acc0[4 * m + 3]);
-                const float4 eb = make_float4(qg + gb.x - 2.f * acc1[4 * m + 0], qg + gb.y - 2.f * acc1[4 * m + 1],
-                                              qg + gb.z - 2.f * acc1[4 * m + 2], qg + gb.w - 2.f * acc1[4 * m + 3]);
-                *reinterpret_cast<float4*>(&E[j * TK_ES + ra]) = ea;
-                *reinterpret_cast<float4*>(&E[j * TK_ES + rb]) = eb;
-                if (track) {
-                    const float e8[8] = {ea.x, ea.y, ea.z, ea.w, eb.x, eb.y, eb.z, eb.w};
-                    const float g8[8] = {ga.x, ga.y, ga.z, ga.w, gb.x, gb.y, gb.z, gb.w};
+                for (int s = 0; s < KS; ++s)
 #pragma unroll
-                    for (int c = 0; c < 8; ++c) {
-                        const bool in = (c < 4 ? ra : rb - 4) + c < rows;  // a row of the tile
-                        const float u = tk_upper(e8[c], qg, g8[c]);
-                        ulo = fminf(ulo, in ? u : __builtin_inff());
-                        uhi = fmaxf(uhi, in ? u : -__builtin_inff());
+                    for (int f = 0; f < QW; ++f) acc[f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(qh[f][s], xh[s], acc[f], 0, 0, 0);
+            }
+#pragma unroll
+            for (int f = 0; f < QW; ++f) acc[f] = __builtin_amdgcn_mfma_f32_32x32x2f32(vw[f], uz, acc[f], 0, 0, 0);
+            // Register r of fragment f: query 32 f + 8 (r / 4) + 4 h + r % 4,
+            // row j of the row group.
+            if constexpr (GATE) {
+#pragma unroll
+                for (int f = 0; f < QW; ++f) {
+                    float m[4];
+#pragma unroll
+                    for (int g = 0; g < 4; ++g)
+                        m[g] = fmaxf(fmaxf(fmaxf(acc[f][4 * g], acc[f][4 * g + 1]), acc[f][4 * g + 2]), acc[f][4 * g + 3]);
+                    if (__ballot(fmaxf(fmaxf(fmaxf(m[0], m[1]), m[2]), m[3]) >= 0.f)) {
+                        uint32_t lq = lq0 + 32u * f + 4u * h;
+                        asm volatile("" : "+v"(lq));  // keeps the 32 queries' addresses out of the tile loop's registers
+                        const float isx = R->isx;
+                        const uint32_t row_id = R->id;
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            if (!__ballot(m[g] >= 0.f)) continue;
+#pragma unroll
+                            for (int c = 0; c < 4; ++c) {
+                                const float x = acc[f][4 * g + c];
+                                const uint64_t pass = __ballot(x >= 0.f);
+                                if (!pass) continue;
+                                if (held > Gate::WB - 64u) drain();
+                                if (x >= 0.f) {
+                                    const float2 gq = G.gq[lq + 8 * g + c];
+                                    const uint32_t at = held + static_cast<uint32_t>(__popcll(pass & lanemask_lt()));
+                                    G.buf[wave][at] = make_uint2(__float_as_uint(gq.x - x * isx * gq.y), row_id);
+                                    G.lq[wave][at] = static_cast<uint16_t>(lq + 8 * g + c);
+                                }
+                                held += static_cast<uint32_t>(__popcll(pass));
+                            }
+                        }
                     }
+                }
+            } else {
+                const uint64_t r0 = tile_r0(t) + rg * 32u;
+                const float nisx2 = -2.f * R->isx;
+                if (r0 + j < sp.n) {
+#pragma unroll
+                    for (int f = 0; f < QW; ++f)
+#pragma unroll
+                        for (int r4 = 0; r4 < 4; ++r4) {
+                            const uint32_t lq = lq0 + 32u * f + 8u * r4 + 4u * h;
+                            const float4 iq = *reinterpret_cast<const float4*>(&L.isq[lq]);
+                            float* dst = a.pd + static_cast<size_t>(qb * C::QB + lq) * a.pd_stride + r0 + j;
+                            dst[0] = acc[f][4 * r4 + 0] * nisx2 * iq.x;
+                            dst[a.pd_stride] = acc[f][4 * r4 + 1] * nisx2 * iq.y;
+                            dst[2 * static_cast<size_t>(a.pd_stride)] = acc[f][4 * r4 + 2] * nisx2 * iq.z;
+                            dst[3 * static_cast<size_t>(a.pd_stride)] = acc[f][4 * r4 + 3] * nisx2 * iq.w;
+                        }
                 }
             }
         }
-        // Tile t + 1 into the other buffer, and tile t + 2's valid ids.
-        tk_store_rows<DP>(L, b ^ 1, pre, pid);
-#pragma unroll
-        for (int p = 0; p < DP / 32; ++p) pid[p] = nid[p];
-        tk_ids_valid<DP>(tile_r0(t + 2), tile_r1(t + 2), pid);
-        // Every wave stores all 32 of its queries' rows and every lane its row
-        // (the estimate rows are allocated for whole query blocks and whole
-        // tiles; a query past n_q, or a row past the tile's last, receives a
-        // value nothing reads), after the iteration's wait: nothing waits for
-        // these stores before the next tile's MFMA has run.
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        {
-            // lane l stores rows 4 (l % 16) .. + 3 of query 4 i + l / 16
-            const float* E = L.est[wave];
-            const uint32_t ql = lane >> 4, cl = 4u * (lane & 15u);
-            float* dst = a.pd + static_cast<size_t>(uq0) * a.small_max + tile_r0(t);  // uniform
-#pragma unroll
-            for (uint32_t i = 0; i < TK_QW / 4; ++i) {
-                const float4 v = *reinterpret_cast<const float4*>(&E[(4u * i + ql) * TK_ES + cl]);
-                *reinterpret_cast<float4*>(dst + static_cast<size_t>(4u * i + ql) * a.small_max + cl) = v;
-            }
-            // the scaled norms, from every wave (the same values)
-            a.px[tile_r0(t) + lane] = L.xg[b][lane];
-        }
-        __builtin_amdgcn_wave_barrier();
+        if (!late) next(t + 1, b ^ 1);
         __syncthreads();
     }
-    ulo = fminf(ulo, __shfl_xor(ulo, 32, 64));
-    uhi = fmaxf(uhi, __shfl_xor(uhi, 32, 64));
-    if (h == 0 && qok && uhi >= ulo) {  // the lane pair saw at least one row
-        atomicMin(a.qlo + q0 + j, tk_ordered(ulo));
-        atomicMax(a.qhi + q0 + j, tk_ordered(uhi));
+    if constexpr (GATE) {
+        drain();
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < C::QB; i += TK_NT)
+            a.cand_n[static_cast<size_t>(chunk) * a.q_rows + qb * C::QB + i] = G.cnt[i];
     }
 }
 
-// ---- 3b. small sets: one workgroup per query selects from every estimate ---
-// Each row's estimate L is a lower bound of its fp32 distance and
-// U = L + TK_SEED_ERR (qg + xg) an upper bound.  The k-th smallest U bounds the
-// k-th smallest distance, so every row of the answer (ties included) has
-// L <= that bound: those rows get their fp32 direct distance, are sorted by
-// (distance, id) and the first k are written.
-constexpr uint32_t TK_SMALL = 1u << 18;  // rows the small-set path takes at most
-constexpr uint32_t TK_SMALL_BYTES = 1u << 30;  // and the estimates it may keep
-constexpr int TK_SEL_NT = 1024;
-constexpr uint32_t TK_SEL_BINS = TK_SEL_NT;  // one histogram bin per thread
-constexpr uint32_t TK_SEL_CB = 8192;         // candidates per batch
-constexpr uint32_t TK_SEL_RPT = 4;           // rows per thread per candidate chunk
-// Process-wide limit of the small-set path (cr_topk_set_small_limit).
+// ---- 3. selection: one workgroup per query --------------------------------------
+// An estimate L is a lower bound of its row's fp32 distance d, and
+// d <= L + 3 E (|q|^2 + |x|^2) with |x|^2 <= 2 |q|^2 + 2 d, so the k rows of
+// smallest L have d <= (Lk + 9.1 E |q|^2) (1 + 7 E): at least k rows lie at or
+// below that bound, and every row of the answer (ties included) has its L there.
+// Lk is taken from a histogram of the estimates, as the upper edge of the bin
+// that holds the k-th smallest (rounded up), which only loosens the bound.
+//   TK_SEL_KEPT  after the estimates: a small set's answer, or from a larger
+//                one's sample the gate of its candidates (tau)
+//   TK_SEL_BOUND a tighter gate from the candidates of stage 1
+//   TK_SEL_CAND  the answer from the candidate lists
+enum { TK_SEL_KEPT, TK_SEL_BOUND, TK_SEL_CAND };
+constexpr int TK_SEL_NT = 512;
+constexpr int TK_SEL_W = TK_SEL_NT / 64;
+constexpr uint32_t TK_SEL_BINS = 1024;
+constexpr uint32_t TK_SEL_CB = 2048;   // candidates per batch
+constexpr uint32_t TK_SEL_RANK = 512;  // ... ranked by counting (one a thread) up to here, sorted above
+constexpr int TK_SEL_V = TK_KEEP / (4 * TK_SEL_NT);  // 16-byte loads a thread that hold every kept estimate
+constexpr uint32_t TK_SEL_LISTS = 512;  // candidate lists a query has at most
+constexpr uint64_t TK_NOKEY = ~0ull;    // no candidate: after every (distance, id) key
+// Limit of the small-set path's rows (cr_topk_set_small_limit).
+constexpr uint32_t TK_SMALL = 1u << 18;
 std::atomic<uint32_t> g_topk_small{TK_SMALL};
 
-// A histogram of the upper bounds of rows [0, Sn) of the query's estimates
-// over the range of all of them: the bins spread the values, so the counting
-// atomics rarely collide.  The first bin at which the count reaches k holds the
-// k-th smallest upper bound; the largest value in the bins up to it is the
-// returned bound (at least k rows lie at or below it, so the k-th distance
-// does).  Every thread of the workgroup calls it.
-__device__ __forceinline__ float tk_hist_bound(const TkArgs& a, uint32_t q, const float* lrow, uint32_t Sn,
-                                               uint32_t* hist, uint32_t* bmax, uint32_t* lds, uint32_t& s_bin,
-                                               uint32_t& s_bound)
+struct TkSelLds {
+    uint64_t key[TK_SEL_CB];      // a batch: ids (or rows), then distance bits << 32 | id
+    uint64_t best[2][TK_KMAX];    // the running best k, ascending (two planes)
+    uint32_t hist[TK_SEL_BINS];
+    uint32_t off[TK_SEL_LISTS + 1];
+    float qv[128];
+    uint32_t lds[TK_SEL_W];
+    float redf[2][TK_SEL_W];
+    uint32_t bin, n;
+};
+
+__device__ __forceinline__ bool tk_finite(float v) { return v > -__builtin_inff() && v < __builtin_inff(); }
+
+// Block-wide minimum of lo and maximum of hi.
+__device__ __forceinline__ void tk_block_range(TkSelLds& L, float& lo, float& hi)
 {
-    const uint32_t t = threadIdx.x, lane = __lane_id();
-    const float qg = a.pq[q];
-    const float vlo = tk_unordered(a.qlo[q]), vhi = tk_unordered(a.qhi[q]);
-    const float scale = vhi > vlo ? static_cast<float>(TK_SEL_BINS) / (vhi - vlo) : 0.f;
-    hist[t] = 0;
-    bmax[t] = 0;
-    if (t == 0) s_bound = 0;
-    __syncthreads();
-    // Eight rows a thread per step, the next step's loads issued before this
-    // step's are binned (clamped to the last row, tested against Sn only where
-    // used, so nothing waits for them early).
-    const uint32_t last = Sn - 1;  // Sn > k >= 1
-    float l8[8], x8[8];
 #pragma unroll
-    for (uint32_t i = 0; i < 8; ++i) {
-        const uint32_t r = min(t + i * TK_SEL_NT, last);
-        l8[i] = lrow[r];
-        x8[i] = a.px[r];
+    for (int o = 32; o > 0; o >>= 1) {
+        lo = fminf(lo, __shfl_xor(lo, o, 64));
+        hi = fmaxf(hi, __shfl_xor(hi, o, 64));
     }
-    for (uint32_t r0 = t; r0 < Sn; r0 += 8 * TK_SEL_NT) {
-        float nl8[8], nx8[8];
-#pragma unroll
-        for (uint32_t i = 0; i < 8; ++i) {
-            const uint32_t r = min(r0 + (8 + i) * TK_SEL_NT, last);
-            nl8[i] = lrow[r];
-            nx8[i] = a.px[r];
-        }
-#pragma unroll
-        for (uint32_t i = 0; i < 8; ++i) {
-            if (r0 + i * TK_SEL_NT >= Sn) break;
-            const float u = tk_upper(l8[i], qg, x8[i]);
-            const float f = (u - vlo) * scale;
-            const uint32_t bin = f >= static_cast<float>(TK_SEL_BINS - 1) ? TK_SEL_BINS - 1
-                                                                          : static_cast<uint32_t>(fmaxf(f, 0.f));
-            atomicAdd(&hist[bin], 1u);
-            atomicMax(&bmax[bin], tk_ordered(u));
-        }
-#pragma unroll
-        for (uint32_t i = 0; i < 8; ++i) l8[i] = nl8[i], x8[i] = nx8[i];
-    }
+    if (__lane_id() == 0) L.redf[0][threadIdx.x >> 6] = lo, L.redf[1][threadIdx.x >> 6] = hi;
     __syncthreads();
-    uint32_t total;
-    const uint32_t h = hist[t];
-    const uint32_t excl = block_excl_scan<TK_SEL_NT>(h, lds, total);
-    if (excl < a.k && excl + h >= a.k) s_bin = t;
-    __syncthreads();
-    uint32_t m = t <= s_bin ? bmax[t] : 0u;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) m = max(m, static_cast<uint32_t>(__shfl_xor(m, o, 64)));
-    if (lane == 0 && m) atomicMax(&s_bound, m);
-    __syncthreads();
-    return tk_unordered(s_bound);
+    for (int w = 0; w < TK_SEL_W; ++w) lo = fminf(lo, L.redf[0][w]), hi = fmaxf(hi, L.redf[1][w]);
 }
 
-// One workgroup per query, right after tk_pairs, on both paths.  A small set
-// is answered here (below).  A larger one gets query q's bound from the upper
-// bounds of its seed rows (more than k of them), into tau for the list path:
-// at least k rows have an fp32 distance at or below it, so the k-th best does
-// (tau holds the bits of non-negative distances).
-__global__ __launch_bounds__(TK_SEL_NT) __attribute__((amdgpu_waves_per_eu(8))) void tk_select(TkArgs a, float* out_d, int64_t* out_id)
+__device__ __forceinline__ uint32_t tk_bin(float v, float lo, float scale)
 {
-    __shared__ float bd[2][TK_KMAX];  // the running best, ascending (two planes)
-    __shared__ uint32_t bi[2][TK_KMAX];
-    __shared__ float cd[TK_SEL_CB];  // a batch of candidates
-    __shared__ uint32_t ci[TK_SEL_CB];
-    __shared__ uint32_t hist[TK_SEL_BINS], bmax[TK_SEL_BINS];
-    __shared__ float qv[128];
-    __shared__ uint32_t lds[TK_SEL_NT / 64];
-    __shared__ uint32_t s_bin, s_bound, s_nbatch;
+    const float f = (v - lo) * scale;
+    return f >= static_cast<float>(TK_SEL_BINS - 1) ? TK_SEL_BINS - 1 : static_cast<uint32_t>(fmaxf(f, 0.f));
+}
+
+// The k-th smallest of the binned values, rounded up to its bin's upper edge;
+// +inf with fewer than k.
+__device__ __forceinline__ float tk_hist_kth(TkSelLds& L, uint32_t k, float lo, float hi)
+{
+    const uint32_t t = threadIdx.x;
+    static_assert(TK_SEL_BINS == 2 * TK_SEL_NT, "two bins a thread");
+    if (t == 0) L.bin = TK_NOID;
+    __syncthreads();  // the counts are complete
+    const uint32_t h0 = L.hist[2 * t], h1 = L.hist[2 * t + 1];
+    uint32_t total;
+    const uint32_t e = block_excl_scan<TK_SEL_NT>(h0 + h1, L.lds, total);
+    if (e < k && e + h0 + h1 >= k) L.bin = 2 * t + (e + h0 >= k ? 0u : 1u);
+    __syncthreads();
+    const uint32_t bin = L.bin;
+    if (bin == TK_NOID) return __builtin_inff();
+    const float edge = bin == TK_SEL_BINS - 1 ? hi : lo + static_cast<float>(bin + 1) * ((hi - lo) * (1.f / TK_SEL_BINS));
+    return fminf(hi, edge + 0x1p-20f * (fabsf(lo) + fabsf(hi)));
+}
+
+template <int MODE>
+__global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, int64_t* out_id)
+{
+    __shared__ TkSelLds L;
     const uint64_t n_rows = tk_rows(a);
-    // More rows than the small-set limit with no list path launched: only a
-    // filter whose recorded cardinality understates its set does that, and
-    // every row is then a candidate (exact, slower; no estimate is read).
-    const bool all_rows = a.list_off && !tk_small(a, n_rows);
-    if (!tk_small(a, n_rows) && !all_rows) {  // the list path answers; its seed bound
-        const uint32_t Sd = tk_seed_rows(a, n_rows);
-        if (Sd <= a.k) return;
-        const uint32_t qs = blockIdx.x;
-        const float sb = tk_hist_bound(a, qs, a.pd + static_cast<size_t>(qs) * a.small_max, Sd, hist, bmax, lds,
-                                       s_bin, s_bound);
-        if (threadIdx.x == 0) atomicMin(a.tau + qs, __float_as_uint(fmaxf(sb, 0.f)));
-        return;
-    }
-    const uint32_t S = static_cast<uint32_t>(n_rows);
+    const bool small = n_rows <= a.keep;
     const uint32_t q = blockIdx.x;
     const uint32_t t = threadIdx.x;
-    const float* lrow = a.pd + static_cast<size_t>(q) * a.small_max;
-    for (uint32_t c = t; c < 128; c += TK_SEL_NT) qv[c] = c < a.dim ? a.queries[static_cast<size_t>(q) * a.dim + c] : 0.f;
-    float bound = __builtin_inff();
-    if (S > a.k && !all_rows) {
-        // The first bound from the upper bounds of the first rows (a sample
-        // only loosens it).
-        const uint32_t Sn = min(S, max(TK_SEL_SAMPLE, TK_SEL_SAMPLE_PER_K * a.k));
-        bound = tk_hist_bound(a, q, lrow, Sn, hist, bmax, lds, s_bin, s_bound);
+    if (MODE != TK_SEL_KEPT && small) return;
+    // More rows than kept with no candidate kernels launched, or lists that
+    // overflowed with no list path launched: only a filter whose recorded
+    // cardinality understates its set does that, and every row is then a
+    // candidate (exact, slower; no estimate is read).
+    bool all_rows = MODE == TK_SEL_KEPT && !small && a.cand_off;
+    const bool bound_only = MODE == TK_SEL_BOUND || (MODE == TK_SEL_KEPT && !small && !all_rows);
+    for (uint32_t c = t; c < 128; c += TK_SEL_NT) L.qv[c] = c < a.dim ? a.queries[static_cast<size_t>(q) * a.dim + c] : 0.f;
+    for (uint32_t i = t; i < TK_SEL_BINS; i += TK_SEL_NT) L.hist[i] = 0;
+    if (t == 0) L.n = 0;
+    __syncthreads();
+    float qn = 0.f;  // |q|^2, each wave by itself
+    {
+        const float x = L.qv[t & 63u], y = L.qv[64u + (t & 63u)];
+        qn = x * x + y * y;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) qn += __shfl_xor(qn, o, 64);
     }
-    // Candidates (rows whose estimate, a lower bound, is at or below the bound)
-    // in batches: fp32 direct distances, a sort by (distance, id), and a merge
-    // into the running best k.
-    uint32_t nb = 0, cur = 0, nbatch = 0;
-    auto flush = [&]() {
-        __syncthreads();  // the batch's rows are in ci
-        for (uint32_t c0 = 0; c0 < nbatch; c0 += TK_SEL_NT / 8) {  // eight threads per candidate
+
+    // The estimates: a small set's or the sample's in registers, the
+    // candidate lists' through the running counts.
+    const uint32_t S = MODE == TK_SEL_KEPT ? static_cast<uint32_t>(small ? n_rows : std::min<uint64_t>(n_rows, a.sample)) : 0u;
+    float4 v[MODE == TK_SEL_KEPT ? TK_SEL_V : 1];
+    uint32_t C = 0;  // candidates in the lists
+    const uint2* lists = a.cand + static_cast<size_t>(q) * a.cap;
+    const size_t list_step = static_cast<size_t>(a.q_rows) * a.cap;
+    float lo = __builtin_inff(), hi = -__builtin_inff();
+    if constexpr (MODE == TK_SEL_KEPT) {
+        const float* row = a.pd + static_cast<size_t>(q) * a.pd_stride;
+#pragma unroll
+        for (int i = 0; i < TK_SEL_V; ++i) {
+            const uint32_t r = 4u * (t + i * TK_SEL_NT);
+            v[i] = make_float4(__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""));
+            if (!all_rows && r < S) {  // the row holds whole vectors
+                v[i] = *reinterpret_cast<const float4*>(row + r);
+                if (r + 1 >= S) v[i].y = __builtin_nanf("");
+                if (r + 2 >= S) v[i].z = __builtin_nanf("");
+                if (r + 3 >= S) v[i].w = __builtin_nanf("");
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < TK_SEL_V; ++i) {
+            const float e[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (tk_finite(e[c])) lo = fminf(lo, e[c]), hi = fmaxf(hi, e[c]);
+        }
+    } else {
+        uint32_t n = t < a.n_cw ? a.cand_n[static_cast<size_t>(t) * a.q_rows + q] : 0u;
+        const bool over = __syncthreads_or(n > a.cap);
+        n = min(n, a.cap);
+        const uint32_t e = block_excl_scan<TK_SEL_NT>(n, L.lds, C);
+        L.off[t] = e;
+        if (t == 0) L.off[TK_SEL_LISTS] = C;
+        __syncthreads();
+        if constexpr (MODE == TK_SEL_CAND) {
+            if (!a.list_off) {
+                if (t == 0) {
+                    a.q_over[q] = over ? 1u : 0u;
+                    if (over) a.qb_over[q / TK_QB] = 1u;
+                }
+                if (over)  // the list path answers: its state (the gate stays its bound)
+                    for (uint32_t c = t; c < a.n_chunks; c += TK_SEL_NT)
+                        a.tau_m[static_cast<size_t>(c) * a.n_q + q] = 0x7F800000u;
+                if (over) return;
+            } else {
+                all_rows = over;
+            }
+        }
+    }
+    auto cand_at = [&](uint32_t i) -> uint2 {  // candidate i of the query's lists
+        uint32_t c = 0;
+#pragma unroll
+        for (uint32_t step = TK_SEL_LISTS / 2; step > 0; step >>= 1)
+            if (L.off[c + step] <= i) c += step;
+        return lists[c * list_step + (i - L.off[c])];
+    };
+    if constexpr (MODE != TK_SEL_KEPT) {
+        for (uint32_t i = t; i < C; i += TK_SEL_NT) {
+            const float e = __uint_as_float(cand_at(i).x);
+            if (tk_finite(e)) lo = fminf(lo, e), hi = fmaxf(hi, e);
+        }
+    }
+    tk_block_range(L, lo, hi);
+    const float scale = hi > lo ? static_cast<float>(TK_SEL_BINS) / (hi - lo) : 0.f;
+    if constexpr (MODE == TK_SEL_KEPT) {
+#pragma unroll
+        for (int i = 0; i < TK_SEL_V; ++i) {
+            const float e[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (tk_finite(e[c])) atomicAdd(&L.hist[tk_bin(e[c], lo, scale)], 1u);
+        }
+    } else {
+        for (uint32_t i = t; i < C; i += TK_SEL_NT) {
+            const float e = __uint_as_float(cand_at(i).x);
+            if (tk_finite(e)) atomicAdd(&L.hist[tk_bin(e, lo, scale)], 1u);
+        }
+    }
+    // Candidate estimates were rounded down by up to twice TK_GATE_ROUND of the gate.
+    const float gate = MODE == TK_SEL_KEPT ? 0.f : __uint_as_float(a.tau[q]);
+    float bound = tk_hist_kth(L, a.k, lo, hi);
+    if (bound < __builtin_inff())
+        bound = fmaxf(bound + 9.1f * TK_EST_ERR * qn + 2.f * TK_GATE_ROUND * gate, 0.f) * (1.f + 8.f * TK_EST_ERR);
+    if (bound_only) {
+        if (t == 0) {
+            a.tau[q] = __float_as_uint(MODE == TK_SEL_KEPT ? bound : fminf(bound, gate));
+            if (MODE == TK_SEL_KEPT && !a.list_off && q % TK_QB == 0) a.qb_over[q / TK_QB] = 0;
+        }
+        return;
+    }
+    if (all_rows) bound = __builtin_inff();
+
+    // Candidates in batches: fp32 direct distances, an order by (distance, id),
+    // and a merge into the running best k.
+    uint32_t nb = 0, cur = 0;
+    auto flush = [&](uint32_t nbatch, bool rows) {  // the batch's ids (or rows of the set) are in key
+        for (uint32_t c0 = 0; c0 < nbatch; c0 += TK_SEL_NT / 8) {  // eight threads (of one wave) per candidate
             const uint32_t c = c0 + t / 8, part = t % 8;
             float e2 = 0.f;
             uint32_t id = 0;
             if (c < nbatch) {
-                const uint32_t r = ci[c];
-                id = a.sel ? a.sel[r] : r;
+                id = static_cast<uint32_t>(L.key[c]);
+                if (rows && a.sel) id = a.sel[id];
                 // the part's 16 dimensions, all loaded before any is used (zeros
                 // past dim, where qv is zero too, add nothing)
                 const float* x = a.base + static_cast<size_t>(id) * a.dim + part * 16;
@@ -1207,10 +1542,10 @@ __global__ __launch_bounds__(TK_SEL_NT) __attribute__((amdgpu_waves_per_eu(8))) 
                     if (a.vec) {  // dim % 4 == 0, 16-byte aligned rows
 #pragma unroll
                         for (uint32_t q4 = 0; q4 < 8; q4 += 4) {
-                            const float4 v = part * 16 + hh + q4 < a.dim
+                            const float4 w = part * 16 + hh + q4 < a.dim
                                                  ? *reinterpret_cast<const float4*>(x + hh + q4)
                                                  : make_float4(0.f, 0.f, 0.f, 0.f);
-                            xv[q4] = v.x, xv[q4 + 1] = v.y, xv[q4 + 2] = v.z, xv[q4 + 3] = v.w;
+                            xv[q4] = w.x, xv[q4 + 1] = w.y, xv[q4 + 2] = w.z, xv[q4 + 3] = w.w;
                         }
                     } else {
 #pragma unroll
@@ -1218,7 +1553,7 @@ __global__ __launch_bounds__(TK_SEL_NT) __attribute__((amdgpu_waves_per_eu(8))) 
                     }
 #pragma unroll
                     for (uint32_t s2 = 0; s2 < 8; ++s2) {
-                        const float e = qv[part * 16 + hh + s2] - xv[s2];
+                        const float e = L.qv[part * 16 + hh + s2] - xv[s2];
                         e2 = fmaf(e, e, e2);
                     }
                 }
@@ -1226,110 +1561,118 @@ __global__ __launch_bounds__(TK_SEL_NT) __attribute__((amdgpu_waves_per_eu(8))) 
             e2 += __shfl_xor(e2, 1, 64);
             e2 += __shfl_xor(e2, 2, 64);
             e2 += __shfl_xor(e2, 4, 64);
-            __syncthreads();  // every thread of the pass has read ci[c]
-            if (c < nbatch && part == 0) {
-                cd[c] = e2;
-                ci[c] = id;
-            }
+            if (c < nbatch && part == 0)  // non-negative: the bits order as values; NaN is no distance
+                L.key[c] = e2 == e2 ? (static_cast<uint64_t>(__float_as_uint(e2)) << 32) | id : TK_NOKEY;
         }
-        uint32_t P = 2;
-        while (P < nbatch) P <<= 1;
-        __syncthreads();
-        for (uint32_t i = nbatch + t; i < P; i += TK_SEL_NT) {
-            cd[i] = __builtin_inff();
-            ci[i] = TK_NOID;
-        }
-        __syncthreads();
-        for (uint32_t size = 2; size <= P; size <<= 1) {
-            for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-                for (uint32_t i = t; i < P / 2; i += TK_SEL_NT) {
-                    const uint32_t lo = 2 * i - (i & (stride - 1));
-                    const uint32_t hi = lo + stride;
-                    const bool up = (lo & size) == 0;
-                    const float dl = cd[lo], dh = cd[hi];
-                    const uint32_t il = ci[lo], ih = ci[hi];
-                    if (tk_less(dh, ih, dl, il) == up) {
-                        cd[lo] = dh;
-                        cd[hi] = dl;
-                        ci[lo] = ih;
-                        ci[hi] = il;
-                    }
-                }
-                __syncthreads();
-            }
-        }
-        // Merge: an entry's rank is its index plus the number of entries of
-        // the other list before it (all (distance, id) pairs are distinct).
+        for (uint32_t i = t; i < TK_KMAX; i += TK_SEL_NT) L.best[cur ^ 1][i] = TK_NOKEY;
         const uint32_t nbt = min(nbatch, a.k);
-        if (t < nb) {
-            const uint32_t r = t + tk_lower_bound(cd, ci, nbt, bd[cur][t], bi[cur][t]);
-            if (r < a.k) {
-                bd[cur ^ 1][r] = bd[cur][t];
-                bi[cur ^ 1][r] = bi[cur][t];
+        if (nb == 0 && nbatch <= TK_SEL_RANK) {
+            // few: each thread counts the keys below its own
+            __syncthreads();
+            const uint64_t mine = t < nbatch ? L.key[t] : TK_NOKEY;
+            uint32_t r = 0;
+            if (t < nbatch)
+                for (uint32_t i = 0; i < nbatch; ++i) r += L.key[i] < mine ? 1u : 0u;
+            if (mine != TK_NOKEY && r < a.k) L.best[cur ^ 1][r] = mine;
+        } else {
+            uint32_t P = 2;
+            while (P < nbatch) P <<= 1;
+            for (uint32_t i = nbatch + t; i < P; i += TK_SEL_NT) L.key[i] = TK_NOKEY;
+            __syncthreads();
+            for (uint32_t size = 2; size <= P; size <<= 1) {
+                for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+                    for (uint32_t i = t; i < P / 2; i += TK_SEL_NT) {
+                        const uint32_t l = 2 * i - (i & (stride - 1));
+                        const uint64_t x = L.key[l], y = L.key[l + stride];
+                        if ((y < x) == ((l & size) == 0)) L.key[l] = y, L.key[l + stride] = x;
+                    }
+                    __syncthreads();
+                }
             }
-        } else if (t - nb < nbt) {
-            const uint32_t e = t - nb;
-            const uint32_t r = e + tk_lower_bound(bd[cur], bi[cur], nb, cd[e], ci[e]);
-            if (r < a.k) {
-                bd[cur ^ 1][r] = cd[e];
-                bi[cur ^ 1][r] = ci[e];
+            // Merge: an entry's rank is its index plus the number of entries of
+            // the other list before it (all keys but TK_NOKEY are distinct).
+            auto below = [](const uint64_t* p, uint32_t n, uint64_t y) {
+                uint32_t l = 0, r = n;
+                while (l < r) {
+                    const uint32_t m = (l + r) >> 1;
+                    if (p[m] < y) l = m + 1;
+                    else r = m;
+                }
+                return l;
+            };
+            if (t < nb) {
+                const uint64_t x = L.best[cur][t];
+                const uint32_t r = t + below(L.key, nbt, x);
+                if (x != TK_NOKEY && r < a.k) L.best[cur ^ 1][r] = x;
+            } else if (t - nb < nbt) {
+                const uint64_t x = L.key[t - nb];
+                const uint32_t r = t - nb + below(L.best[cur], nb, x);
+                if (x != TK_NOKEY && r < a.k) L.best[cur ^ 1][r] = x;
             }
         }
         nb = min(a.k, nb + nbt);
         cur ^= 1;
-        nbatch = 0;
-        if (t == 0) s_nbatch = 0;
+        if (t == 0) L.n = 0;
         __syncthreads();
-        if (nb == a.k) bound = fminf(bound, bd[cur][a.k - 1]);  // the k-th best so far bounds the answer
+        if (nb == a.k) {  // the k-th best so far bounds the answer
+            const uint64_t kth = L.best[cur][a.k - 1];
+            if (kth != TK_NOKEY) bound = fminf(bound, __uint_as_float(static_cast<uint32_t>(kth >> 32)));
+        }
     };
-    // Candidates are few: a thread that finds one takes a batch slot with an
-    // LDS atomic.  Chunks of TK_SEL_RPT consecutive rows per thread (one
-    // 16-byte load), the loads of the next two chunks in flight while one is
-    // tested (clamped to the last whole vector of the row, which the estimate
-    // row holds, and tested against S only where used, so nothing waits for
-    // them early); a batch that could overflow in the next chunk is flushed
-    // first.
-    static_assert(TK_SEL_RPT == 4, "one float4 a thread per chunk");
-    constexpr uint32_t CH = TK_SEL_RPT * TK_SEL_NT;
-    if (t == 0) s_nbatch = 0;
+    // Slots of the batch come from an LDS counter; a batch that the next
+    // TK_SEL_NT values could overflow is flushed first.
+    auto room = [&]() {
+        __syncthreads();  // the slots so far are taken
+        const uint32_t n = L.n;
+        __syncthreads();  // every thread has read the count
+        if (n > TK_SEL_CB - TK_SEL_NT) flush(n, MODE == TK_SEL_KEPT || all_rows);
+    };
     if (all_rows) {
-        for (uint32_t r0 = 0; r0 < S; r0 += CH) {
-            __syncthreads();  // the previous chunk's slots are taken
-            nbatch = s_nbatch;
-            __syncthreads();
-            if (nbatch > TK_SEL_CB - CH) flush();
+        for (uint64_t r0 = 0; r0 < n_rows; r0 += TK_SEL_NT) {
+            room();
+            if (r0 + t < n_rows) L.key[atomicAdd(&L.n, 1u)] = r0 + t;
+        }
+    } else if constexpr (MODE == TK_SEL_KEPT) {
+        uint32_t mine = 0;
 #pragma unroll
-            for (uint32_t i = 0; i < TK_SEL_RPT; ++i) {
-                const uint32_t r = r0 + i * TK_SEL_NT + t;
-                if (r < S) ci[atomicAdd(&s_nbatch, 1u)] = r;
+        for (int i = 0; i < TK_SEL_V; ++i)
+            mine += (v[i].x <= bound ? 1u : 0u) + (v[i].y <= bound ? 1u : 0u) + (v[i].z <= bound ? 1u : 0u) +
+                    (v[i].w <= bound ? 1u : 0u);
+        uint32_t total;
+        uint32_t at = block_excl_scan<TK_SEL_NT>(mine, L.lds, total);
+        if (total <= TK_SEL_CB) {
+#pragma unroll
+            for (int i = 0; i < TK_SEL_V; ++i) {
+                const float e[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (e[c] <= bound) L.key[at++] = 4u * (t + i * TK_SEL_NT) + c;
+            }
+            if (t == 0) L.n = total;
+        } else {
+            const float* row = a.pd + static_cast<size_t>(q) * a.pd_stride;
+            for (uint32_t r0 = 0; r0 < S; r0 += TK_SEL_NT) {
+                room();
+                if (r0 + t < S && row[r0 + t] <= bound) L.key[atomicAdd(&L.n, 1u)] = r0 + t;
+            }
+        }
+    } else {
+        for (uint32_t i0 = 0; i0 < C; i0 += TK_SEL_NT) {
+            room();
+            if (i0 + t < C) {
+                const uint2 e = cand_at(i0 + t);
+                if (__uint_as_float(e.x) <= bound) L.key[atomicAdd(&L.n, 1u)] = e.y;
             }
         }
     }
-    const uint32_t last4 = S > 0 && !all_rows ? (S - 1) & ~3u : 0;
-    auto ld4 = [&](uint32_t r) { return *reinterpret_cast<const float4*>(lrow + min(r, last4)); };
-    float4 l4 = ld4(4 * t), n4 = ld4(CH + 4 * t);
-    for (uint32_t r0 = 0; r0 < (all_rows ? 0u : S); r0 += CH) {
-        const float4 m4 = ld4(r0 + 2 * CH + 4 * t);
-        __syncthreads();  // the previous chunk's slots are taken
-        nbatch = s_nbatch;
-        __syncthreads();  // every thread has read the count before the next slots are taken
-        if (nbatch > TK_SEL_CB - CH) flush();
-        const float lv[4] = {l4.x, l4.y, l4.z, l4.w};
-#pragma unroll
-        for (uint32_t i = 0; i < 4; ++i) {
-            const uint32_t r = r0 + 4 * t + i;
-            if (r < S && lv[i] <= bound) ci[atomicAdd(&s_nbatch, 1u)] = r;
-        }
-        l4 = n4;
-        n4 = m4;
-    }
     __syncthreads();
-    nbatch = s_nbatch;
-    if (nbatch) flush();
+    const uint32_t left = L.n;
+    if (left) flush(left, MODE == TK_SEL_KEPT || all_rows);
     for (uint32_t r = t; r < a.k; r += TK_SEL_NT) {
-        const bool ok = r < nb;
-        out_d[static_cast<size_t>(q) * a.k + r] = ok ? bd[cur][r] : __builtin_inff();
-        out_id[static_cast<size_t>(q) * a.k + r] = ok ? static_cast<int64_t>(bi[cur][r]) : int64_t(-1);
+        const uint64_t x = r < nb ? L.best[cur][r] : TK_NOKEY;
+        const bool ok = x != TK_NOKEY;
+        out_d[static_cast<size_t>(q) * a.k + r] = ok ? __uint_as_float(static_cast<uint32_t>(x >> 32)) : __builtin_inff();
+        out_id[static_cast<size_t>(q) * a.k + r] = ok ? static_cast<int64_t>(static_cast<uint32_t>(x)) : int64_t(-1);
     }
 }
 
@@ -1339,31 +1682,64 @@ __global__ __launch_bounds__(256) void tk_init(TkArgs a)
     tk_init_from(a, static_cast<uint64_t>(blockIdx.x) * 256u + threadIdx.x, static_cast<uint64_t>(gridDim.x) * 256u);
 }
 
-template <int DP>
-int launch_dist(const TkArgs& a, uint32_t grid, uint32_t pairs_grid, float* out_d, int64_t* out_ids, hipStream_t s)
+// One launch of tk_est: n_cw workgroups a query block, rounded up to the XCDs.
+template <int KS, int QW, int QG, bool GATE>
+void launch_est(const TkArgs& a, uint32_t n_qb, uint32_t stage, hipStream_t s)
 {
-    if (a.small_max) {  // estimates of a small set (and its answer), or the seed rows of a larger one and their bound
-        {
-            CR_TIMED("tk_pairs", s);
-            if (a.sel)
-                tk_pairs<DP, true><<<pairs_grid, TK_NT, 0, s>>>(a);
-            else
-                tk_pairs<DP, false><<<pairs_grid, TK_NT, 0, s>>>(a);
-        }
+    const uint32_t grid = (a.n_cw * n_qb + 7u) / 8u * 8u;
+    CR_TIMED(GATE ? "tk_gate" : "tk_pairs", s);
+    if (a.sel)
+        tk_est<KS, QW, QG, true, GATE><<<grid, TK_NT, 0, s>>>(a, n_qb, stage);
+    else
+        tk_est<KS, QW, QG, false, GATE><<<grid, TK_NT, 0, s>>>(a, n_qb, stage);
+}
+
+template <int MODE>
+int launch_select(const TkArgs& a, float* out_d, int64_t* out_ids, hipStream_t s)
+{
+    CR_TIMED("tk_select", s);
+    tk_select<MODE><<<a.n_q, TK_SEL_NT, 0, s>>>(a, out_d, out_ids);
+    CR_LAUNCH_CHECK();
+    return CR_OK;
+}
+
+// The estimate path: the answer of a small set, or the sample's bound, the
+// candidates (in two stages when one bound would let too many through) and
+// the answer from them.
+template <int KS, int QW, int QG>
+int launch_gated(const TkArgs& a, uint32_t n_qb, bool two_stages, float* out_d, int64_t* out_ids, hipStream_t s)
+{
+    launch_est<KS, QW, QG, false>(a, n_qb, 0, s);
+    CR_LAUNCH_CHECK();
+    CR_RET(launch_select<TK_SEL_KEPT>(a, out_d, out_ids, s));
+    if (a.cand_off) return CR_OK;
+    if (two_stages) {
+        launch_est<KS, QW, QG, true>(a, n_qb, 1, s);
         CR_LAUNCH_CHECK();
-        {
-            CR_TIMED("tk_select", s);
-            tk_select<<<a.n_q, TK_SEL_NT, 0, s>>>(a, out_d, out_ids);
-        }
-        CR_LAUNCH_CHECK();
+        CR_RET(launch_select<TK_SEL_BOUND>(a, out_d, out_ids, s));
     }
-    if (!a.list_off) {
-        CR_TIMED("tk_dist", s);
-        if (a.sel)
-            tk_dist<DP, true><<<grid, TK_NT, 0, s>>>(a);
-        else
-            tk_dist<DP, false><<<grid, TK_NT, 0, s>>>(a);
-    }
+    launch_est<KS, QW, QG, true>(a, n_qb, two_stages ? 2 : 0, s);
+    CR_LAUNCH_CHECK();
+    return launch_select<TK_SEL_CAND>(a, out_d, out_ids, s);
+}
+
+template <int QW, int QG>
+int launch_gated_dim(const TkArgs& a, uint32_t n_qb, bool two_stages, float* out_d, int64_t* out_ids, hipStream_t s)
+{
+    if (a.dim <= 32) return launch_gated<2, QW, QG>(a, n_qb, two_stages, out_d, out_ids, s);
+    if (a.dim <= 64) return launch_gated<4, QW, QG>(a, n_qb, two_stages, out_d, out_ids, s);
+    if (a.dim <= 96) return launch_gated<6, QW, QG>(a, n_qb, two_stages, out_d, out_ids, s);
+    return launch_gated<8, QW, QG>(a, n_qb, two_stages, out_d, out_ids, s);
+}
+
+template <int DP>
+int launch_dist(const TkArgs& a, uint32_t grid, hipStream_t s)
+{
+    CR_TIMED("tk_dist", s);
+    if (a.sel)
+        tk_dist<DP, true><<<grid, TK_NT, 0, s>>>(a);
+    else
+        tk_dist<DP, false><<<grid, TK_NT, 0, s>>>(a);
     CR_LAUNCH_CHECK();
     return CR_OK;
 }
@@ -1388,35 +1764,8 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
         return CR_ERR_UNSUPPORTED;
     }
     hipStream_t s = as_stream(stream);
-    const uint32_t n_qb = (n_q + TK_QB - 1) / TK_QB;
-    // Enough (chunk, query block) workgroups to cover every CU once.
     const uint32_t cus = num_cus();
-    uint32_t n_chunks = std::max<uint32_t>(8, (cus + n_qb - 1) / n_qb);
-    n_chunks = (n_chunks + 7) / 8 * 8;
     const uint64_t nb = (n_base + TK_ENUM_IDS - 1) / TK_ENUM_IDS;
-
-    Carver cv;
-    const size_t o_counts = cv.add(filter ? nb * 4 : 0);
-    const size_t o_nsel = cv.add(4);
-    const size_t o_sel = cv.add(filter ? n_base * 4 : 0);
-    const size_t lists = static_cast<size_t>(n_chunks) * n_q * k;
-    const size_t o_ld = cv.add(2 * lists * 4);
-    const size_t o_li = cv.add(2 * lists * 4);
-    const size_t o_ln = cv.add(static_cast<size_t>(n_chunks) * n_q * 4);
-    const size_t o_tau = cv.add(static_cast<size_t>(n_q) * 4);
-    const size_t o_taum = cv.add(static_cast<size_t>(n_chunks) * n_q * 4);
-    // The small-set path keeps every estimate, small_max floats for each query
-    // of every whole query block, within TK_SMALL_BYTES.
-    const uint64_t q_rows = static_cast<uint64_t>(n_qb) * TK_QB;
-    const uint32_t small_max = static_cast<uint32_t>(std::min<uint64_t>(
-        g_topk_small.load(), TK_SMALL_BYTES / (4ull * q_rows) / TK_ROWS * TK_ROWS));
-    const size_t o_pd = cv.add(q_rows * small_max * 4);
-    const size_t o_pq = cv.add(small_max ? static_cast<size_t>(n_q) * 4 : 0);
-    const size_t o_px = cv.add(static_cast<size_t>(small_max) * 4);
-    const size_t o_qlo = cv.add(small_max ? static_cast<size_t>(n_q) * 4 : 0);
-    const size_t o_qhi = cv.add(small_max ? static_cast<size_t>(n_q) * 4 : 0);
-    Scratch sc;
-    CR_RET(sc.alloc(cv.total, s));
 
     TkArgs a{};
     a.base = d_base;
@@ -1425,35 +1774,84 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
     a.n_q = n_q;
     a.dim = dim;
     a.k = k;
-    a.n_chunks = n_chunks;
     a.vec = (dim % 4 == 0) && (reinterpret_cast<uintptr_t>(d_base) % 16 == 0);
     a.qvec = (dim % 4 == 0) && (reinterpret_cast<uintptr_t>(d_queries) % 16 == 0);
+
+    // The most rows that can pass: a filter's recorded cardinality (the
+    // library's uploads and fused multi_and record it, and the reference's
+    // conversions rely on it too, src/to_csr.cu:212-216), plus one per container
+    // for a multi_and's full containers stored as 65535.  An understated one
+    // costs time, never the answer.
+    const uint64_t rows_ub = filter && filter->total_cardinality > 0
+                                 ? std::min<uint64_t>(n_base, filter->total_cardinality + filter->n_containers)
+                                 : n_base;
+
+    // The estimate path: 256 queries a workgroup, or 64 for the few that read
+    // the rows only once anyway.
+    const bool few = n_q <= 64;
+    const uint32_t est_qb = few ? 64 : 256;
+    const uint32_t n_qb = (n_q + est_qb - 1) / est_qb;
+    a.q_rows = n_qb * est_qb;
+    a.n_cw = std::min<uint32_t>(TK_SEL_LISTS, std::max<uint32_t>(1, cus / n_qb));
+    const uint32_t limit = g_topk_small.load();
+    const uint64_t fit = TK_SCRATCH / (4ull * a.q_rows) / TK_ROWS * TK_ROWS;  // estimate rows within the scratch limit
+    a.keep = static_cast<uint32_t>(std::min<uint64_t>(std::min(limit, TK_KEEP), fit));
+    a.sample_lg = 14;
+    static_assert(TK_KEEP == 1u << 14, "the sample is at most the kept rows");
+    while ((1ull << a.sample_lg) > fit && a.sample_lg > 0) --a.sample_lg;
+    a.sample = 1u << a.sample_lg;
+    // limit 0 turns it off; so does a batch of queries too large for a sample
+    // that bounds the k-th distance.
+    a.gate = limit > 0 && a.sample >= std::max<uint32_t>(1024, 8 * k);
+    if (!a.gate) a.keep = 0;
+    a.pd_stride = std::max((a.keep + 63u) / 64u * 64u, a.sample);
+    a.cand_off = a.gate && rows_ub <= a.keep;
+    // Lists that hold every row a workgroup sees need no list path behind them.
+    const uint64_t tile = few ? 128 : 64;
+    const uint64_t list_rows = ((rows_ub + tile - 1) / tile + a.n_cw - 1) / a.n_cw * tile +
+                               (TK_STAGE > 1 ? tile : 0);  // two stages may give a workgroup one tile more
+    const uint64_t lists_fit = TK_SCRATCH / (8ull * a.q_rows * a.n_cw);
+    a.cap = static_cast<uint32_t>(list_rows <= lists_fit ? list_rows : std::min<uint64_t>(TK_CAND_CAP, lists_fit));
+    a.list_off = a.gate && (a.cand_off || a.cap == list_rows);
+
+    // The list path: enough (chunk, query block) workgroups to cover every CU once.
+    const uint32_t list_qb = (n_q + TK_QB - 1) / TK_QB;
+    uint32_t n_chunks = std::max<uint32_t>(8, (cus + list_qb - 1) / list_qb);
+    n_chunks = (n_chunks + 7) / 8 * 8;
+    a.n_chunks = n_chunks;
+    a.m_rank = std::max<uint32_t>(1, (2 * k + n_chunks - 1) / n_chunks);
+
+    Carver cv;
+    const size_t o_counts = cv.add(filter ? nb * 4 : 0);
+    const size_t o_nsel = cv.add(4);
+    const size_t o_sel = cv.add(filter ? n_base * 4 : 0);
+    const size_t o_tau = cv.add(static_cast<size_t>(n_q) * 4);
+    const size_t lists = a.list_off ? 0 : static_cast<size_t>(n_chunks) * n_q * k;
+    const size_t o_ld = cv.add(2 * lists * 4);
+    const size_t o_li = cv.add(2 * lists * 4);
+    const size_t o_ln = cv.add(a.list_off ? 0 : static_cast<size_t>(n_chunks) * n_q * 4);
+    const size_t o_taum = cv.add(a.list_off ? 0 : static_cast<size_t>(n_chunks) * n_q * 4);
+    const size_t o_pd = cv.add(a.gate ? static_cast<size_t>(a.q_rows) * a.pd_stride * 4 : 0);
+    const bool cands = a.gate && !a.cand_off;
+    const size_t o_cand = cv.add(cands ? static_cast<size_t>(a.q_rows) * a.n_cw * a.cap * 8 : 0);
+    const size_t o_candn = cv.add(cands ? static_cast<size_t>(a.q_rows) * a.n_cw * 4 : 0);
+    const size_t o_qover = cv.add(cands ? static_cast<size_t>(n_q) * 4 : 0);
+    const size_t o_qbover = cv.add(cands ? static_cast<size_t>(list_qb) * 4 : 0);
+    Scratch sc;
+    CR_RET(sc.alloc(cv.total, s));
+    a.tau = sc.at<uint32_t>(o_tau);
     a.list_d = sc.at<float>(o_ld);
     a.list_id = sc.at<uint32_t>(o_li);
     a.list_n = sc.at<uint32_t>(o_ln);
     a.plane = lists;
-    a.tau = sc.at<uint32_t>(o_tau);
     a.tau_m = sc.at<uint32_t>(o_taum);
-    a.m_rank = std::max<uint32_t>(1, (2 * k + n_chunks - 1) / n_chunks);
-    a.small_max = small_max;
-    a.pd = small_max ? sc.at<float>(o_pd) : nullptr;
-    a.pq = small_max ? sc.at<float>(o_pq) : nullptr;
-    a.px = small_max ? sc.at<float>(o_px) : nullptr;
-    a.qlo = small_max ? sc.at<uint32_t>(o_qlo) : nullptr;
-    a.qhi = small_max ? sc.at<uint32_t>(o_qhi) : nullptr;
-    // The list path is not launched when the passing count is known to fit the
-    // small-set path: no filter and a small base, or a filter's recorded
-    // cardinality (the library's uploads and fused multi_and record it, and the
-    // reference's conversions rely on it too, src/to_csr.cu:212-216), plus one
-    // per container for a multi_and's full containers stored as 65535.
-    if (small_max) {
-        const uint64_t bound = !filter ? n_base
-                                       : (filter->total_cardinality > 0
-                                              ? std::min<uint64_t>(n_base, filter->total_cardinality + filter->n_containers)
-                                              : UINT64_MAX);
-        a.list_off = bound <= small_max ? 1u : 0u;
-    }
-    if (!filter || nb == 0) {
+    a.pd = sc.at<float>(o_pd);
+    a.cand = sc.at<uint2>(o_cand);
+    a.cand_n = sc.at<uint32_t>(o_candn);
+    a.q_over = sc.at<uint32_t>(o_qover);
+    a.qb_over = sc.at<uint32_t>(o_qbover);
+
+    if (!a.gate && (!filter || nb == 0)) {
         tk_init<<<static_cast<unsigned>((static_cast<uint64_t>(n_chunks) * n_q + 255) / 256), 256, 0, s>>>(a);
         CR_LAUNCH_CHECK();
     }
@@ -1475,23 +1873,29 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
         }
         CR_LAUNCH_CHECK();
     }
-    const uint32_t grid = n_chunks * n_qb;
-    // tk_pairs: one workgroup a CU (two waves a SIMD fill it), each query
-    // block's tiles dealt out among its workgroups
-    const uint32_t pairs_grid = std::max<uint32_t>(1, (cus + n_qb - 1) / n_qb) * n_qb;
-    if (dim <= 32) {
-        CR_RET(launch_dist<32>(a, grid, pairs_grid, d_out_dist, d_out_ids, s));
-    } else if (dim <= 64) {
-        CR_RET(launch_dist<64>(a, grid, pairs_grid, d_out_dist, d_out_ids, s));
-    } else {
-        CR_RET(launch_dist<128>(a, grid, pairs_grid, d_out_dist, d_out_ids, s));
+    if (a.gate) {
+        // One bound from the sample lets about k rows / sample candidates a
+        // query through; past TK_TWO_STAGE of them a second bound, from the
+        // first 16th of the tiles, costs less than it saves.
+        const bool two_stages = static_cast<double>(k) * static_cast<double>(rows_ub) > static_cast<double>(TK_TWO_STAGE) * a.sample;
+        const int rc = few ? launch_gated_dim<1, 2>(a, n_qb, two_stages, d_out_dist, d_out_ids, s)
+                           : launch_gated_dim<2, 4>(a, n_qb, two_stages, d_out_dist, d_out_ids, s);
+        CR_RET(rc);
     }
     if (!a.list_off) {
+        const uint32_t grid = n_chunks * list_qb;
+        if (dim <= 32) {
+            CR_RET(launch_dist<32>(a, grid, s));
+        } else if (dim <= 64) {
+            CR_RET(launch_dist<64>(a, grid, s));
+        } else {
+            CR_RET(launch_dist<128>(a, grid, s));
+        }
         CR_TIMED("tk_merge", s);
         tk_merge<<<(n_q + 3) / 4, TK_MERGE_NT, 0, s>>>(a, a.list_d, a.list_id, a.plane, a.list_n, n_chunks, n_q, k,
                                                         d_out_dist, d_out_ids);
+        CR_LAUNCH_CHECK();
     }
-    CR_LAUNCH_CHECK();
     return CR_OK;
 }
 

@@ -330,8 +330,9 @@ def contains_batch(g: GpuRoaring, d_ids, d_out, mode: int = QUERY_CONTAINS, stre
 
 
 def topk_set_small_limit(rows: int) -> int:
-    """Rows at or below which the top-k keeps every estimate and selects per
-    query (capped at 262144; 0 turns that path off).  Returns the previous limit."""
+    """Rows at or below which the top-k may keep every estimate and select per
+    query (capped at 262144; 0 turns the estimates off: sorted lists answer).
+    Returns the previous limit."""
     return int(load().cr_topk_set_small_limit(rows))
 
 

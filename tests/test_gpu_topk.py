@@ -231,3 +231,93 @@ def test_topk_rejects_unsupported(gpu):
     i = torch.empty((2, 5), dtype=torch.int64, device="cuda")
     with pytest.raises(gpu.CrError):
         gpu.topk_filtered(base, q, 5, None, d, i)
+
+
+# The estimate path past its kept rows (16384): each padded dimension count and
+# its edges, both workgroup shapes (up to 64 queries, and 256 a workgroup with
+# partial groups), one and two candidate stages (k rows > 1024 x 16384), a
+# partial last tile, and exactly one row more than is kept.
+GATED = [
+    # (n_base, n_q, dim, k, filter kind, density, seed)
+    (16385, 1, 32, 1, "none", 1.0, 31),
+    (16385, 257, 31, 5, "none", 1.0, 32),
+    (40001, 65, 64, 3, "none", 1.0, 33),
+    (40063, 64, 33, 7, "none", 1.0, 34),
+    (50000, 100, 96, 10, "ids", 0.9, 35),
+    (33000, 30, 65, 10, "keep", 0.8, 36),
+    (20000, 20, 97, 256, "none", 1.0, 37),
+    (180000, 70, 96, 100, "none", 1.0, 38),  # two stages
+    (300000, 9, 20, 200, "ids", 0.6, 39),  # two stages, a negated filter, few queries
+    (600000, 3, 17, 256, "none", 1.0, 40),
+]
+
+
+@pytest.mark.parametrize("n_base,n_q,dim,k,kind,density,seed", GATED)
+def test_topk_gated(gpu, n_base, n_q, dim, k, kind, density, seed):
+    _say("topk gated", n_base, n_q, dim, k, kind, density, seed)
+    base, queries = _data(n_base, n_q, dim, seed)
+    filt, mask = _filter_from(gpu, kind, n_base, density, seed)
+    got_d, got_i = _run(gpu, base, queries, k, filt)
+    check_topk(base, queries, k, mask, got_d, got_i)
+    if filt is not None:
+        gpu.free(filt)
+
+
+@pytest.mark.parametrize("scale", [1e-8, 1e-3, 1e3, 1e8])
+def test_topk_gated_scales(gpu, scale):
+    """The split's scale follows each vector's norm: rows of very different
+    norms in one set, at magnitudes far outside the range of 16-bit floats."""
+    _say("topk scales", scale)
+    base, queries = _data(30000, 20, 128, 51)
+    base *= np.float32(scale) * np.exp2(np.arange(30000) % 23 - 11).astype(np.float32)[:, None]
+    queries *= np.float32(scale)
+    got_d, got_i = _run(gpu, base, queries, 20, None)
+    check_topk(base, queries, 20, None, got_d, got_i)
+
+
+@pytest.mark.parametrize("n_base", [3000, 30000])
+def test_topk_unusual_rows(gpu, n_base):
+    """Rows and queries that the estimates leave out (zero, or of a norm that
+    overflows or underflows) and rows with infinities or NaN: the finite
+    distances are answered exactly, infinite ones come last, NaN never."""
+    _say("topk unusual", n_base)
+    base, queries = _data(n_base, 8, 64, 53)
+    base[5] = 0
+    base[7] = queries[1]
+    base[11] *= 1e-15
+    base[13, 3] = np.inf
+    base[17, 4] = -np.inf
+    base[19, 5] = np.nan
+    base[23] = 1e25
+    queries[2] = 0
+    queries[3] *= 1e-15
+    got_d, got_i = _run(gpu, base, queries, 10, None)
+    bad = np.isin(np.arange(n_base), [13, 17, 19, 23])
+    mask = (~bad).astype(np.uint8)
+    clean = base.copy()
+    clean[bad] = 0
+    check_topk(clean, queries, 10, mask, got_d, got_i)
+    # fewer finite rows than k: the infinite distances fill up, the NaN row is left out
+    few = np.array([5, 7, 13, 17, 19, 23])
+    sub = np.ascontiguousarray(base[few])
+    got_d, got_i = _run(gpu, sub, queries, 8, None)
+    for q in range(8):
+        assert set(got_i[q, :2].tolist()) == {0, 1} and np.all(np.isfinite(got_d[q, :2]))
+        assert got_i[q, 2:5].tolist() == [2, 3, 5] and np.all(np.isinf(got_d[q, 2:5]))
+        assert np.all(got_i[q, 5:] == -1) and np.all(np.isinf(got_d[q, 5:]))
+
+
+def test_topk_candidates_overflow(gpu):
+    """Every sampled row is far from the queries and every other row near, so the
+    sample bounds nothing and the candidate lists (bounded at this size)
+    overflow: the list path answers."""
+    _say("topk overflow")
+    n, n_q = 200000, 1024
+    base, queries = _data(n, n_q, 32, 55)
+    base *= np.float32(0.1)
+    queries *= np.float32(0.1)
+    sampled = (np.arange(16384, dtype=np.uint64) * np.uint64(n)) >> np.uint64(14)
+    base[sampled] += 50
+    got_d, got_i = _run(gpu, base, queries, 10, None)
+    pick = np.arange(0, n_q, 37)
+    check_topk(base, queries[pick], 10, None, got_d[pick], got_i[pick])
