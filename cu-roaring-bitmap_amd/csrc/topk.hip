@@ -24,6 +24,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <type_traits>
 
 #include "cu_roaring/device/roaring_view.hpp"
 #include "image.hpp"
@@ -896,26 +897,40 @@ __global__ __launch_bounds__(TK_MERGE_NT) void tk_merge(TkArgs a, const float* l
 // the estimate times -sx sq / 2.  The norms come last so that the products are
 // rounded at their own size, as an fp32 MFMA's are before its norms are added.
 //
-// A workgroup's eight waves are QG query groups of 32 QW queries (their halves
-// live in registers) by RG row groups of 32 rows; a tile of 32 RG rows goes
-// through LDS once for all of them, split as it is stored.  Large query counts
-// take 256 queries a workgroup (QW 2, QG 4): the MFMA work per tile covers its
-// conversion; up to 64 queries are bound by reading the rows and take 128-row
-// tiles (QW 1, QG 2).
-// Measured (10M x 128, 1M passing rows, 1024 queries): 706-741 us for the candidate
-// kernel, against 2505 us of fp32 MFMA with sorted lists; the MFMAs alone 480 us.
-// 300K x 100 unfiltered rows, 64 queries: 32 us (3.8 TB/s of rows), against 189 us and
-// 224 us more for merging 256 lists a query.
+// For candidates the accumulator first holds hi.hi alone, whose distance from
+// q.x is bounded (TK_COARSE_ERR): the rank-2 test with that much added excludes
+// most 32 x 32 fragments, and only the others compute the cross products.
+//
+// A workgroup's eight waves are QG query groups of 32 QW queries (their hi
+// halves live in registers) by RG row groups of 32 rows; a tile of 32 RG rows
+// goes through LDS once for all of them.  The next tile's split (its norms,
+// scales and halves, ~150 vector instructions a lane) is cut into pieces that
+// run between the current tile's MFMAs, and rows are loaded two tiles ahead.
+// Large query counts take 256 queries a workgroup (QW 2, QG 4): the tile's
+// split and its reads are then shared by 256; up to 64 queries are bound by
+// reading the rows and take 128-row tiles (QW 1, QG 2).
+// Measured (128 dimensions, 1024 queries): 483 us for a tenth of 10M rows, 1435 us
+// for 4M unfiltered ones, against 2505 us and ~9.5 ms of fp32 MFMA with sorted
+// lists; with all three products for every pair 706 us (the MFMAs alone 480 us:
+// 1.6 PFLOP/s, where the clock gives way to power).  Without the loads, 4M rows
+// take 980 us.  4M rows, 64 queries: 306 us, 6.3 TB/s of rows.
 // The estimate's error against fp64, 32 x 32 blocks of 17 to 128 dimensions
 // (normal, positive, and over 2^20 of magnitudes), rms of |q|^2 + |x|^2:
 // 5.5e-8 to 1.45e-7, with fp32 MFMA 6.4e-8 to 1.73e-7 (lower in each block).
 constexpr uint32_t TK_KEEP = 16384;         // rows whose estimates are all kept, and the sample, at most
 constexpr uint32_t TK_SCRATCH = 1u << 30;   // bytes of estimates, and of candidate lists, at most
 constexpr uint32_t TK_CAND_CAP = 2048;      // candidates a list holds where it cannot hold every row
-constexpr uint32_t TK_TWO_STAGE = 1024;     // expected candidates a query above which a second bound pays
+constexpr double TK_TWO_STAGE = 1024;       // expected candidates of a query, and of all of them, above which a
+constexpr double TK_TWO_STAGE_ALL = 1 << 17;  // second bound pays
+// |q.x - hi.hi| <= (2 x 2^-11 + 2^-22) |q||x|, and 2 |q||x| <= |q|^2 + |x|^2: the
+// test on hi.hi with the norms shrunk by TK_COARSE_ERR more excludes only pairs
+// that the full estimate excludes (2% covers its rounding).
+constexpr float TK_COARSE_ERR = 1.02f * 0x1p-10f;
+constexpr float TK_COARSE = 1.f - TK_COARSE_ERR;
 constexpr float TK_GATE_ROUND = 0x1p-20f;   // rounding of a stored estimate, relative to the gate
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));  // (a float4 struct's load is split where two paths merge)
@@ -926,11 +941,11 @@ struct TkEst {
     static constexpr int T = 32 * RG;         // rows of a tile
     static constexpr int QB = 32 * QW * QG;   // queries of a workgroup
     static constexpr int DP = 16 * KS;        // padded dimensions
-    // Eight threads load a row: thread l takes dimensions 8 l .. + 7 and, past
-    // 64 dimensions, 64 + 8 l .. + 7.  More threads a row would spend more on
-    // its norm and scale than on its elements.
+    // Eight threads load a row, a float4 of each 32 dimensions (whole 128-byte
+    // lines); more threads a row would spend more on its norm and scale than
+    // on its elements.
     static constexpr int TPR = 8;
-    static constexpr int V = DP > 64 ? 16 : 8;  // elements a thread
+    static constexpr int V = DP / 8;          // elements a thread
     static constexpr int RPP = TK_NT / TPR;   // rows per pass
     static constexpr int P = T / RPP;         // passes
     static constexpr int RS = DP + 8;         // row stride in LDS: conflict-free 16-byte reads
@@ -945,10 +960,9 @@ struct alignas(16) TkRow {
 template <int KS, int QW, int QG>
 struct TkEstLds {
     using C = TkEst<KS, QW, QG>;
-    alignas(16) _Float16 hi[2][C::T * C::RS];
-    alignas(16) _Float16 lo[2][C::T * C::RS];
-    TkRow row[2][C::T];
-    alignas(16) float isq[C::QB];
+    alignas(16) _Float16 hi[C::T * C::RS];
+    alignas(16) _Float16 lo[C::T * C::RS];
+    TkRow row[C::T];
 };
 
 // What the candidates need beside it.  A wave appends its candidates to a
@@ -957,7 +971,7 @@ struct TkEstLds {
 // the store too (both count in order).
 template <int QB>
 struct TkGateLds {
-    static constexpr uint32_t WB = QB == 256 ? 512 : 192;  // entries a wave (LDS left by the tiles)
+    static constexpr uint32_t WB = 192;  // entries a wave (LDS left by the tiles)
     float2 gq[QB];  // an estimate is gq.x - acc gq.y / sx
     uint32_t cnt[QB];
     uint2 buf[TK_WAVES][WB];    // (estimate bits, id)
@@ -978,12 +992,18 @@ __device__ __forceinline__ float tk_scale(float ss, float& inv, bool& odd)
     return __uint_as_float(se << 23);
 }
 
+// v_mul_legacy_f32: 0 times anything (infinities and NaN too) is 0.
+extern "C" __device__ float tk_mul_legacy(float, float) __asm("llvm.amdgcn.fmul.legacy");
+
 // hi and lo halves of two scaled values.
 __device__ __forceinline__ void tk_split(float a, float b, f16x2& hi, f16x2& lo)
 {
     const f32x2 v = {a, b};
     hi = __builtin_convertvector(v, f16x2);
-    const f32x2 r = {fmaf(static_cast<float>(hi.x), -1.f, a), fmaf(static_cast<float>(hi.y), -1.f, b)};
+    // a - hi in one instruction each (v_fma_mix_f32 reads a 16-bit half in place)
+    f32x2 r;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r.x) : "v"(hi), "v"(a));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r.y) : "v"(hi), "v"(b));
     lo = __builtin_convertvector(r, f16x2);
 }
 
@@ -995,40 +1015,45 @@ struct TkSpan {
     uint32_t lg;     // log2 of the sample's size, 0 for every row
 };
 
-template <class C, bool SEL>
+// Ids of a tile's rows [r0, r0 + T) of the launch's sp.n (past the last: the last's).
+template <class C, bool SEL, bool SAMPLE>
 __device__ __forceinline__ void tk_est_ids(const TkArgs& a, const TkSpan& sp, uint64_t r0, uint32_t (&raw)[C::P])
 {
+    const uint32_t at = static_cast<uint32_t>(std::min<uint64_t>(r0, sp.n - 1));
+    const uint32_t left = static_cast<uint32_t>(sp.n - 1) - at;
 #pragma unroll
     for (int p = 0; p < C::P; ++p) {
-        uint64_t r = std::min<uint64_t>(r0 + p * C::RPP + threadIdx.x / C::TPR, sp.n - 1);
-        if (sp.lg) r = (r * sp.rows) >> sp.lg;
-        raw[p] = SEL ? a.sel[r] : static_cast<uint32_t>(r);
+        uint32_t r = at + min(p * C::RPP + threadIdx.x / C::TPR, left);
+        if (SAMPLE && sp.lg) r = static_cast<uint32_t>((static_cast<uint64_t>(r) * sp.rows) >> sp.lg);
+        raw[p] = SEL ? a.sel[r] : r;
     }
 }
 
-template <class C>
-__device__ __forceinline__ void tk_est_valid(uint64_t r0, uint64_t n, uint32_t (&id)[C::P])
-{
-#pragma unroll
-    for (int p = 0; p < C::P; ++p)
-        if (r0 + p * C::RPP + threadIdx.x / C::TPR >= n) id[p] = TK_NOID;
-}
-
-// A thread's elements of its rows (dimensions past dim repeat the last; they are
-// zeroed where they are used, so that nothing waits for a load where it is issued).
+// Dimension of element e of a thread's row.
 template <class C>
 __device__ __forceinline__ uint32_t tk_est_col(int e)
 {
-    return (threadIdx.x % C::TPR) * 8u + (e < 8 ? 0u : 64u) + (e & 7u);
+    return 32u * (e / 4) + (threadIdx.x % C::TPR) * 4u + (e & 3u);
 }
 
-template <class C>
+// Dimension at position 8 i + e of a split row in LDS, and of the queries'
+// operand: the eight values that a thread stores at once are its float4s of two
+// 32-dimension groups; a last odd group keeps its order.
+template <int DP>
+__device__ __forceinline__ uint32_t tk_est_dim(uint32_t i, uint32_t e)
+{
+    return i < DP / 64 * 8u ? (i / 8) * 64u + (i % 8) * 4u + 32u * (e / 4) + (e & 3u) : 8u * i + e;
+}
+
+// A thread's elements of its rows.  Dimensions past dim repeat valid ones: the
+// norm leaves them out, and the queries hold zeros there.
+template <class C, bool VEC>
 __device__ __forceinline__ void tk_est_rows(const TkArgs& a, const uint32_t (&id)[C::P], float (&pre)[C::P][C::V])
 {
 #pragma unroll
     for (int p = 0; p < C::P; ++p) {
-        const float* src = a.base + static_cast<size_t>(id[p] != TK_NOID ? id[p] : 0u) * a.dim;
-        if (a.vec) {
+        const float* src = a.base + static_cast<size_t>(id[p]) * a.dim;
+        if constexpr (VEC) {
 #pragma unroll
             for (int e = 0; e < C::V; e += 4) {
                 const f32x4 v = *reinterpret_cast<const f32x4*>(src + min(tk_est_col<C>(e), a.dim - 4u));
@@ -1041,62 +1066,70 @@ __device__ __forceinline__ void tk_est_rows(const TkArgs& a, const uint32_t (&id
     }
 }
 
-template <class C, class Lds>
-__device__ __forceinline__ void tk_est_store(const TkArgs& a, Lds& L, int buf, const float (&pre)[C::P][C::V],
-                                             const uint32_t (&id)[C::P])
-{
-    const uint32_t l = threadIdx.x % C::TPR;
+// A tile's rows from registers into an LDS buffer, split, in PIECES steps of a
+// few vector instructions that the tile loop puts between MFMAs: per pass
+// V / 4 for the norm's partial sums, one for the sum over the row's threads,
+// one for the scale, V / 2 that split two elements each, one for the record.
+template <class C, bool VEC>
+struct TkSplit {
+    static constexpr int PER = C::V / 4 + 2 + C::V / 2 + 1;
+    static constexpr int PIECES = C::P * PER;
+    float ss, unit, inv, sx;
+    bool odd;
+    f16x8 hv, lv;
+
+    template <class Buf>
+    __device__ __forceinline__ void piece(int i, Buf& B, const float (&pre)[C::P][C::V], const uint32_t (&id)[C::P],
+                                          uint32_t valid, uint32_t dim)
+    {
+        const uint32_t l = threadIdx.x % C::TPR;
+        const int p = i / PER, k = i % PER;
+        const uint32_t row = p * C::RPP + threadIdx.x / C::TPR;
+        if (k < C::V / 4) {
+            if (k == 0) ss = 0.f;
+            float x[4];
 #pragma unroll
-    for (int p = 0; p < C::P; ++p) {
-        const int row = p * C::RPP + static_cast<int>(threadIdx.x / C::TPR);
-        float v[C::V];
-        float ss = 0.f;
-#pragma unroll
-        for (int e = 0; e < C::V; ++e) {
-            v[e] = tk_est_col<C>(e) < a.dim ? pre[p][e] : 0.f;
-            ss = fmaf(v[e], v[e], ss);
-        }
-        ss = tk_group_sum<8>(ss);
-        float inv;
-        bool odd;
-        const float sx = tk_scale(ss, inv, odd);
-        if (__ballot(odd)) {  // rows that are not estimated multiply as zeros ...
-#pragma unroll
-            for (int e = 0; e < C::V; ++e) v[e] = odd ? 0.f : v[e];
-        }
-        _Float16* H = &L.hi[buf][row * C::RS + 8 * l];
-        _Float16* W = &L.lo[buf][row * C::RS + 8 * l];
-#pragma unroll
-        for (int c = 0; c < C::V; c += 8) {
-            f16x8 hv, lv;
-#pragma unroll
-            for (int e = 0; e < 8; e += 2) {
-                f16x2 hi, lo;
-                tk_split(v[c + e] * sx, v[c + e + 1] * sx, hi, lo);
-                hv[e] = hi.x, hv[e + 1] = hi.y, lv[e] = lo.x, lv[e + 1] = lo.y;
+            for (int e = 0; e < 4; ++e) x[e] = VEC || tk_est_col<C>(4 * k + e) < dim ? pre[p][4 * k + e] : 0.f;
+            const float s4 = fmaf(x[0], x[0], x[1] * x[1]) + fmaf(x[2], x[2], x[3] * x[3]);
+            ss += !VEC || tk_est_col<C>(4 * k) < dim ? s4 : 0.f;
+        } else if (k == C::V / 4) {
+            ss = tk_group_sum<8>(ss);
+        } else if (k == C::V / 4 + 1) {
+            unit = tk_scale(ss, inv, odd);
+            sx = odd ? 0.f : unit;  // rows that are not estimated multiply as zeros ...
+        } else if (k < PER - 1) {
+            const int e = 2 * (k - C::V / 4 - 2);
+            f16x2 hi, lo;
+            tk_split(tk_mul_legacy(pre[p][e], sx), tk_mul_legacy(pre[p][e + 1], sx), hi, lo);
+            hv[e & 7] = hi.x, hv[(e & 7) + 1] = hi.y, lv[e & 7] = lo.x, lv[(e & 7) + 1] = lo.y;
+            if ((e & 7) == 6) {
+                const uint32_t at = row * C::RS + 8u * l + 8u * (e & ~7);
+                *reinterpret_cast<f16x8*>(&B.hi[at]) = hv;
+                *reinterpret_cast<f16x8*>(&B.lo[at]) = lv;
+            } else if (e == C::V - 2) {  // an odd group
+                const uint32_t at = row * C::RS + 4u * l + 8u * (e & ~7);
+                *reinterpret_cast<f16x4*>(&B.hi[at]) = __builtin_shufflevector(hv, hv, 0, 1, 2, 3);
+                *reinterpret_cast<f16x4*>(&B.lo[at]) = __builtin_shufflevector(lv, lv, 0, 1, 2, 3);
             }
-            if (8 * l + 8 * c < C::DP) {
-                *reinterpret_cast<f16x8*>(H + 8 * c) = hv;
-                *reinterpret_cast<f16x8*>(W + 8 * c) = lv;
-            }
-        }
-        if (l == 0) {  // ... and their factor makes them pass every gate, or (past the last row) none
-            TkRow r;
-            r.u = id[p] == TK_NOID ? -__builtin_inff() : odd ? __builtin_inff() : -0.5f * (1.f - TK_EST_ERR) * ss * sx;
-            r.z = sx;
-            r.isx = inv;
-            r.id = id[p];
-            L.row[buf][row] = r;
+        } else {
+            // ... and their factor makes them pass every gate, or (past the last
+            // row) none.  Thread l writes word l % 4 of the row's record.
+            const float u = row >= valid ? -__builtin_inff()
+                                         : odd ? __builtin_inff() : -0.5f * (1.f - TK_EST_ERR) * ss * sx;
+            uint32_t w0 = __float_as_uint(u), w1 = __float_as_uint(unit), w2 = __float_as_uint(inv), w3 = id[p];
+            asm("" : "+v"(w0), "+v"(w1), "+v"(w2), "+v"(w3));  // selects, not branches, which would end the block
+            const uint32_t lo = (l & 1u) ? w1 : w0, hi = (l & 1u) ? w3 : w2;
+            reinterpret_cast<uint32_t*>(&B.row[row])[l & 3u] = (l & 2u) ? hi : lo;
         }
     }
-}
+};
 
 // GATE false: estimates of a small set or of the sample, into pd.  GATE true:
 // candidates of a larger set; `stage` 0 takes every tile, 1 every 16th, 2 the
 // others (the counts then continue).
 constexpr uint32_t TK_STAGE = 16;
 
-template <int KS, int QW, int QG, bool SEL, bool GATE>
+template <int KS, int QW, int QG, bool SEL, bool VEC, bool GATE>
 __global__ __launch_bounds__(TK_NT) void tk_est(TkArgs a, uint32_t n_qb, uint32_t stage)
 {
     using C = TkEst<KS, QW, QG>;
@@ -1117,12 +1150,18 @@ __global__ __launch_bounds__(TK_NT) void tk_est(TkArgs a, uint32_t n_qb, uint32_
     const uint64_t first = (all + TK_STAGE - 1) / TK_STAGE;  // tiles of stage 1
     const uint64_t part = stage == 0 ? all : stage == 1 ? first : all - first;
     const uint32_t n_tiles = chunk < part ? static_cast<uint32_t>((part - chunk + a.n_cw - 1) / a.n_cw) : 0u;
-    auto tile_r0 = [&](uint32_t i) -> uint64_t {
-        const uint64_t g = chunk + static_cast<uint64_t>(i) * a.n_cw;
-        const uint64_t t = stage == 0 ? g : stage == 1 ? g * TK_STAGE : g + g / (TK_STAGE - 1) + 1;
-        return t * C::T;
+    const uint32_t mul = stage == 1 ? TK_STAGE : 1u;
+    auto tile_r0 = [&](uint32_t i) -> uint64_t {  // first row of the workgroup's tile i
+        const uint32_t g = chunk + i * a.n_cw;
+        return static_cast<uint64_t>(g * mul + (stage == 2 ? g / (TK_STAGE - 1) + 1u : 0u)) * C::T;
     };
-    __shared__ TkEstLds<KS, QW, QG> L;
+    // Two tiles, as objects of their own: writes to one may pass reads of the other.
+    __shared__ TkEstLds<KS, QW, QG> T0, T1;
+    __shared__ alignas(16) float s_isq[C::QB];
+    // Candidates rarely need the queries' lo halves: they stay in LDS where
+    // registers are short.
+    constexpr bool QL_LDS = GATE && QW == 2;
+    __shared__ alignas(16) _Float16 s_ql[QL_LDS ? C::QB * C::RS : 8];
     using Gate = TkGateLds<GATE ? C::QB : 1>;
     __shared__ Gate G;
     const uint32_t lane = __lane_id();
@@ -1133,18 +1172,23 @@ __global__ __launch_bounds__(TK_NT) void tk_est(TkArgs a, uint32_t n_qb, uint32_
     const uint32_t q0 = qb * C::QB + lq0;
     const bool busy = q0 < a.n_q;  // wave-uniform
 
-    float pre[C::P][C::V];
-    uint32_t id[C::P], nid[C::P];
-    if (n_tiles > 0) {
-        tk_est_ids<C, SEL>(a, sp, tile_r0(0), id);
-        tk_est_ids<C, SEL>(a, sp, tile_r0(1), nid);
-        tk_est_valid<C>(tile_r0(0), sp.n, id);
-        tk_est_rows<C>(a, id, pre);
-    }
+    // Tile t's rows are in set t & 1 of pre, with their ids.
+    float pre[2][C::P][C::V];
+    uint32_t id[2][C::P], nid[C::P];
+    tk_est_ids<C, SEL, !GATE>(a, sp, tile_r0(0), id[0]);
+    tk_est_ids<C, SEL, !GATE>(a, sp, tile_r0(1), id[1]);
+    tk_est_rows<C, VEC>(a, id[0], pre[0]);
+    tk_est_ids<C, SEL, !GATE>(a, sp, tile_r0(2), nid);
+    tk_est_rows<C, VEC>(a, id[1], pre[1]);
+    // Rows of tile t (0 past the last tile).
+    auto tile_rows = [&](uint32_t t) -> uint32_t {
+        const uint64_t r0 = tile_r0(t);
+        return t < n_tiles && r0 < sp.n ? static_cast<uint32_t>(std::min<uint64_t>(sp.n - r0, C::T)) : 0u;
+    };
 
-    // A operand: the wave's queries, split, dimensions 16 s + 8 h .. + 7 a lane.
-    f16x8 qh[QW][KS], ql[QW][KS];
-    float vw[QW];  // the rank-2 product's query factors: sq (lanes 0-31), (gate - |q|^2) sq / 2 (lanes 32-63)
+    // A operand: the wave's queries, split, positions 16 s + 8 h .. + 7 a lane.
+    f16x8 qh[QW][KS], ql[QL_LDS ? 1 : QW][QL_LDS ? 1 : KS];
+    float vw[QW], vc[QW];  // the rank-2 product's query factors: sq (lanes 0-31), (gate - |q|^2) sq / 2 (lanes 32-63)
 #pragma unroll
     for (int f = 0; f < QW; ++f) {
         const uint32_t q = q0 + 32u * f + j;
@@ -1154,17 +1198,17 @@ __global__ __launch_bounds__(TK_NT) void tk_est(TkArgs a, uint32_t n_qb, uint32_
         if (a.qvec) {
 #pragma unroll
             for (int e = 0; e < 8 * KS; e += 4) {
-                const f32x4 v = *reinterpret_cast<const f32x4*>(src + min(16u * (e / 8) + 8u * h + e % 8, a.dim - 4u));
+                const f32x4 v = *reinterpret_cast<const f32x4*>(src + min(tk_est_dim<C::DP>(2u * (e / 8) + h, e % 8), a.dim - 4u));
                 x[e] = v.x, x[e + 1] = v.y, x[e + 2] = v.z, x[e + 3] = v.w;
             }
         } else {
 #pragma unroll
-            for (int e = 0; e < 8 * KS; ++e) x[e] = src[min(16u * (e / 8) + 8u * h + e % 8, a.dim - 1u)];
+            for (int e = 0; e < 8 * KS; ++e) x[e] = src[min(tk_est_dim<C::DP>(2u * (e / 8) + h, e % 8), a.dim - 1u)];
         }
         float ss = 0.f;
 #pragma unroll
         for (int e = 0; e < 8 * KS; ++e) {
-            x[e] = ok && 16u * (e / 8) + 8u * h + e % 8 < a.dim ? x[e] : 0.f;
+            x[e] = ok && tk_est_dim<C::DP>(2u * (e / 8) + h, e % 8) < a.dim ? x[e] : 0.f;
             ss += x[e] * x[e];
         }
         ss += __shfl_xor(ss, 32, 64);
@@ -1172,20 +1216,28 @@ __global__ __launch_bounds__(TK_NT) void tk_est(TkArgs a, uint32_t n_qb, uint32_
         bool odd;
         const float sq = tk_scale(ss, inv, odd);
 #pragma unroll
-        for (int s = 0; s < KS; ++s)
+        for (int s = 0; s < KS; ++s) {
+            f16x8 l8;
 #pragma unroll
             for (int e = 0; e < 8; e += 2) {
                 f16x2 hi, lo;
                 tk_split(odd ? 0.f : x[8 * s + e] * sq, odd ? 0.f : x[8 * s + e + 1] * sq, hi, lo);
                 qh[f][s][e] = hi.x, qh[f][s][e + 1] = hi.y;
-                ql[f][s][e] = lo.x, ql[f][s][e + 1] = lo.y;
+                l8[e] = lo.x, l8[e + 1] = lo.y;
             }
+            if constexpr (QL_LDS) {
+                if (rg == 0) *reinterpret_cast<f16x8*>(&s_ql[(lq0 + 32u * f + j) * C::RS + 16u * s + 8u * h]) = l8;
+            } else {
+                ql[f][s] = l8;
+            }
+        }
         const float gate = GATE && ok ? __uint_as_float(a.tau[q]) : 0.f;
         const bool pass = odd || !(gate < __builtin_inff());  // every row is a candidate
         const float qgn = (1.f - TK_EST_ERR) * ss;
         vw[f] = h == 0 ? (ok ? sq : 0.f) : !ok ? -__builtin_inff() : pass ? __builtin_inff() : 0.5f * (gate - qgn) * sq;
+        vc[f] = h == 0 || !ok || pass ? vw[f] : 0.5f * (gate - qgn * TK_COARSE) * sq;
         if (rg == 0 && h == 0) {
-            L.isq[lq0 + 32u * f + j] = inv;
+            s_isq[lq0 + 32u * f + j] = inv;
             if (GATE) {
                 G.gq[lq0 + 32u * f + j] = make_float2(pass ? -__builtin_inff() : gate - TK_GATE_ROUND * gate, 2.f * inv);
                 G.cnt[lq0 + 32u * f + j] =
@@ -1193,19 +1245,12 @@ __global__ __launch_bounds__(TK_NT) void tk_est(TkArgs a, uint32_t n_qb, uint32_
             }
         }
     }
-    // A tile into LDS, from registers that were loaded a
-    // tile ago; then the rows of the tile after it (their ids known since the
-    // last tile) and the ids of the one after that.  Past the last tile they
-    // repeat valid rows that nothing reads.
-    auto next = [&](uint32_t t, int buf) {
-        if (t < n_tiles) tk_est_store<C>(a, L, buf, pre, id);
+    TkSplit<C, VEC> split;
+    {
+        const uint32_t valid = tile_rows(0);
 #pragma unroll
-        for (int p = 0; p < C::P; ++p) id[p] = nid[p];
-        tk_est_valid<C>(tile_r0(t + 1), t + 1 < n_tiles ? sp.n : 0, id);
-        tk_est_rows<C>(a, id, pre);
-        tk_est_ids<C, SEL>(a, sp, tile_r0(t + 2), nid);
-    };
-    if (n_tiles > 0) next(0, 0);
+        for (int i = 0; i < TkSplit<C, VEC>::PIECES; ++i) split.piece(i, T0, pre[0], id[0], valid, a.dim);
+    }
     __syncthreads();
 
     // The workgroup's lists (TK_SCRATCH bounds them: 32-bit offsets).
@@ -1221,51 +1266,92 @@ __global__ __launch_bounds__(TK_NT) void tk_est(TkArgs a, uint32_t n_qb, uint32_
         wave_lds_fence();
         held = 0;
     };
-    // Waves 0-3 (one a SIMD) multiply first and convert the next tile then,
-    // waves 4-7 the other way round: a SIMD's matrix unit works for one of its
-    // two waves while its vector unit converts for the other.
-    const bool late = __builtin_amdgcn_readfirstlane(wave) >= 4;
-    for (uint32_t t = 0; t < n_tiles; ++t) {
-        const int b = static_cast<int>(t & 1u);
-        if (late) next(t + 1, b ^ 1);
-        if (busy) {
+    // Tile t (in LDS buffer b = t & 1): tile t + 3's ids and tile t + 2's rows
+    // are issued first; tile t + 1, loaded during tile t - 1, is split into the
+    // other buffer between tile t's MFMAs.  Past the last tile the loads repeat
+    // valid rows that nothing reads.
+    auto tile = [&](uint32_t t, auto bc) {
+        constexpr int b = decltype(bc)::value;
+#pragma unroll
+        for (int p = 0; p < C::P; ++p) id[b][p] = nid[p];
+        tk_est_ids<C, SEL, !GATE>(a, sp, tile_r0(t + 3), nid);  // (first: the next tile's wait for them leaves the rows)
+        tk_est_rows<C, VEC>(a, id[b], pre[b]);
+        const uint32_t next = tile_rows(t + 1);
+        auto& B = b == 0 ? T0 : T1;
+        auto& N = b == 0 ? T1 : T0;
+        if (!busy) {
+#pragma unroll
+            for (int i = 0; i < TkSplit<C, VEC>::PIECES; ++i) split.piece(i, N, pre[b ^ 1], id[b ^ 1], next, a.dim);
+        } else {
             f32x16 acc[QW];
-            const TkRow* R = &L.row[b][rg * 32u + j];
+            const TkRow* R = &B.row[rg * 32u + j];
             const float uz = h == 0 ? R->u : R->z;
 #pragma unroll
             for (int f = 0; f < QW; ++f) acc[f] = f32x16{};
-            const _Float16* H = &L.hi[b][(rg * 32u + j) * C::RS + 8u * h];
-            const _Float16* W = &L.lo[b][(rg * 32u + j) * C::RS + 8u * h];
-            // hi.hi last for few dimensions, the cross products with it for
-            // many, which saves keeping or reading the row's halves twice.
+            const _Float16* H = &B.hi[(rg * 32u + j) * C::RS + 8u * h];
+            const _Float16* W = &B.lo[(rg * 32u + j) * C::RS + 8u * h];
+            // The products, each QW MFMAs and a share of the next tile's split:
+            // candidates first need hi.hi only; estimates need all three, hi.hi
+            // last for few dimensions (its larger sums are then rounded fewer
+            // times), the three of a step together for many (which reads the
+            // row's halves once).
             constexpr bool CROSS_FIRST = KS <= 4;
-            f16x8 xh[KS];
+            constexpr int PRODUCTS = GATE ? KS : 3 * KS;
+            f16x8 xh[!GATE && CROSS_FIRST ? KS : 1], xl;
+            int piece = 0;
 #pragma unroll
-            for (int s = 0; s < KS; ++s) {
-                xh[s] = *reinterpret_cast<const f16x8*>(H + 16 * s);
-                const f16x8 xl = *reinterpret_cast<const f16x8*>(W + 16 * s);
-                if constexpr (!CROSS_FIRST) {
-#pragma unroll
-                    for (int f = 0; f < QW; ++f) acc[f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(qh[f][s], xh[s], acc[f], 0, 0, 0);
+            for (int i = 0; i < PRODUCTS; ++i) {
+                const bool last = !GATE && CROSS_FIRST && i >= 2 * KS;
+                const int s = GATE ? i : CROSS_FIRST ? (last ? i - 2 * KS : i / 2) : i / 3;
+                const int what = GATE || last ? 0 : CROSS_FIRST ? 1 + i % 2 : i % 3;  // hi.hi, lo.hi, hi.lo
+                f16x8& x = xh[!GATE && CROSS_FIRST ? s : 0];
+                if (GATE || (!last && (CROSS_FIRST ? i % 2 : i % 3) == 0)) {
+                    x = *reinterpret_cast<const f16x8*>(H + 16 * s);
+                    if (!GATE) xl = *reinterpret_cast<const f16x8*>(W + 16 * s);
                 }
 #pragma unroll
-                for (int f = 0; f < QW; ++f) acc[f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ql[f][s], xh[s], acc[f], 0, 0, 0);
+                for (int f = 0; f < QW; ++f)
+                    acc[f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(what == 1 ? ql[QL_LDS ? 0 : f][QL_LDS ? 0 : s] : qh[f][s],
+                                                                     what == 2 ? xl : x, acc[f], 0, 0, 0);
+                const int end = (i + 1) * TkSplit<C, VEC>::PIECES / PRODUCTS;
 #pragma unroll
-                for (int f = 0; f < QW; ++f) acc[f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(qh[f][s], xl, acc[f], 0, 0, 0);
+                for (int k = piece; k < end; ++k) split.piece(k, N, pre[b ^ 1], id[b ^ 1], next, a.dim);
+                piece = end;
+                if (QW == 2) __builtin_amdgcn_sched_barrier(0);  // (up to 64 queries wait for rows, not for this order)
             }
-            if constexpr (CROSS_FIRST) {
+            if constexpr (!GATE) {
 #pragma unroll
-                for (int s = 0; s < KS; ++s)
-#pragma unroll
-                    for (int f = 0; f < QW; ++f) acc[f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(qh[f][s], xh[s], acc[f], 0, 0, 0);
+                for (int f = 0; f < QW; ++f) acc[f] = __builtin_amdgcn_mfma_f32_32x32x2f32(vw[f], uz, acc[f], 0, 0, 0);
             }
-#pragma unroll
-            for (int f = 0; f < QW; ++f) acc[f] = __builtin_amdgcn_mfma_f32_32x32x2f32(vw[f], uz, acc[f], 0, 0, 0);
             // Register r of fragment f: query 32 f + 8 (r / 4) + 4 h + r % 4,
             // row j of the row group.
             if constexpr (GATE) {
+                // hi.hi is within TK_COARSE_ERR of q.x: most fragments hold no pair
+                // that could pass, whatever the cross products are.
+                const float uc = h == 0 ? R->u * TK_COARSE : R->z;
+                f32x16 c[QW];
+#pragma unroll
+                for (int f = 0; f < QW; ++f) c[f] = __builtin_amdgcn_mfma_f32_32x32x2f32(vc[f], uc, acc[f], 0, 0, 0);
 #pragma unroll
                 for (int f = 0; f < QW; ++f) {
+                    uint32_t mc = ~0u;  // below 2^31: a sign bit is clear (a value >= 0, or a NaN, which fails below)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) mc = min(mc, __float_as_uint(c[f][r]));
+                    if (!__ballot(mc < 0x80000000u)) continue;
+                    f32x16 cross = {};
+#pragma unroll
+                    for (int s = 0; s < KS; ++s) {
+                        const f16x8 x = *reinterpret_cast<const f16x8*>(H + 16 * s);
+                        const f16x8 y = *reinterpret_cast<const f16x8*>(W + 16 * s);
+                        f16x8 l8;
+                        if constexpr (QL_LDS) l8 = *reinterpret_cast<const f16x8*>(&s_ql[(lq0 + 32u * f + j) * C::RS + 16u * s + 8u * h]);
+                        else l8 = ql[f][s];
+                        cross = __builtin_amdgcn_mfma_f32_32x32x16_f16(l8, x, cross, 0, 0, 0);
+                        cross = __builtin_amdgcn_mfma_f32_32x32x16_f16(qh[f][s], y, cross, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[f][r] += cross[r];
+                    acc[f] = __builtin_amdgcn_mfma_f32_32x32x2f32(vw[f], uz, acc[f], 0, 0, 0);
                     float m[4];
 #pragma unroll
                     for (int g = 0; g < 4; ++g)
@@ -1304,7 +1390,7 @@ __global__ __launch_bounds__(TK_NT) void tk_est(TkArgs a, uint32_t n_qb, uint32_
 #pragma unroll
                         for (int r4 = 0; r4 < 4; ++r4) {
                             const uint32_t lq = lq0 + 32u * f + 8u * r4 + 4u * h;
-                            const float4 iq = *reinterpret_cast<const float4*>(&L.isq[lq]);
+                            const float4 iq = *reinterpret_cast<const float4*>(&s_isq[lq]);
                             float* dst = a.pd + static_cast<size_t>(qb * C::QB + lq) * a.pd_stride + r0 + j;
                             dst[0] = acc[f][4 * r4 + 0] * nisx2 * iq.x;
                             dst[a.pd_stride] = acc[f][4 * r4 + 1] * nisx2 * iq.y;
@@ -1314,8 +1400,11 @@ __global__ __launch_bounds__(TK_NT) void tk_est(TkArgs a, uint32_t n_qb, uint32_
                 }
             }
         }
-        if (!late) next(t + 1, b ^ 1);
         __syncthreads();
+    };
+    for (uint32_t t = 0; t < n_tiles; t += 2) {
+        tile(t, std::integral_constant<int, 0>{});
+        if (t + 1 < n_tiles) tile(t + 1, std::integral_constant<int, 1>{});
     }
     if constexpr (GATE) {
         drain();
@@ -1688,10 +1777,14 @@ void launch_est(const TkArgs& a, uint32_t n_qb, uint32_t stage, hipStream_t s)
 {
     const uint32_t grid = (a.n_cw * n_qb + 7u) / 8u * 8u;
     CR_TIMED(GATE ? "tk_gate" : "tk_pairs", s);
-    if (a.sel)
-        tk_est<KS, QW, QG, true, GATE><<<grid, TK_NT, 0, s>>>(a, n_qb, stage);
+    if (a.sel && a.vec)
+        tk_est<KS, QW, QG, true, true, GATE><<<grid, TK_NT, 0, s>>>(a, n_qb, stage);
+    else if (a.sel)
+        tk_est<KS, QW, QG, true, false, GATE><<<grid, TK_NT, 0, s>>>(a, n_qb, stage);
+    else if (a.vec)
+        tk_est<KS, QW, QG, false, true, GATE><<<grid, TK_NT, 0, s>>>(a, n_qb, stage);
     else
-        tk_est<KS, QW, QG, false, GATE><<<grid, TK_NT, 0, s>>>(a, n_qb, stage);
+        tk_est<KS, QW, QG, false, false, GATE><<<grid, TK_NT, 0, s>>>(a, n_qb, stage);
 }
 
 template <int MODE>
@@ -1875,9 +1968,11 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
     }
     if (a.gate) {
         // One bound from the sample lets about k rows / sample candidates a
-        // query through; past TK_TWO_STAGE of them a second bound, from the
-        // first 16th of the tiles, costs less than it saves.
-        const bool two_stages = static_cast<double>(k) * static_cast<double>(rows_ub) > static_cast<double>(TK_TWO_STAGE) * a.sample;
+        // query through.  A second bound, from the first 16th of the tiles,
+        // costs two launches; it saves most of the lists, and of the cross
+        // products (a fragment computes them for any candidate it may hold).
+        const double cands = static_cast<double>(k) * static_cast<double>(rows_ub) / a.sample;
+        const bool two_stages = cands > TK_TWO_STAGE || cands * n_q > TK_TWO_STAGE_ALL;
         const int rc = few ? launch_gated_dim<1, 2>(a, n_qb, two_stages, d_out_dist, d_out_ids, s)
                            : launch_gated_dim<2, 4>(a, n_qb, two_stages, d_out_dist, d_out_ids, s);
         CR_RET(rc);
