@@ -901,19 +901,21 @@ __global__ __launch_bounds__(TK_MERGE_NT) void tk_merge(TkArgs a, const float* l
 // q.x is bounded (TK_COARSE_ERR): the rank-2 test with that much added excludes
 // most 32 x 32 fragments, and only the others compute the cross products.
 //
-// A workgroup's eight waves are QG query groups of 32 QW queries (their hi
-// halves live in registers) by RG row groups of 32 rows; a tile of 32 RG rows
-// goes through LDS once for all of them.  The next tile's split (its norms,
-// scales and halves, ~150 vector instructions a lane) is cut into pieces that
-// run between the current tile's MFMAs, and rows are loaded two tiles ahead.
-// Large query counts take 256 queries a workgroup (QW 2, QG 4): the tile's
-// split and its reads are then shared by 256; up to 64 queries are bound by
-// reading the rows and take 128-row tiles (QW 1, QG 2).
+// A workgroup's waves are QG query groups of 32 QW queries (their hi halves live
+// in registers) by two row groups of 32 rows; a tile of 64 rows goes through
+// LDS once for all of them.  The next tile's split (its norms, scales and
+// halves, ~150 vector instructions a lane) is cut into pieces that run between
+// the current tile's MFMAs, and rows are loaded two tiles ahead.  Large query
+// counts take 256 queries a workgroup (QW 2, QG 4, eight waves, one a CU): the
+// tile's split and its reads are then shared by 256.  Up to 64 queries are bound
+// by reading the rows (QW 1, QG 2, four waves): two workgroups a CU, which do
+// not wait for each other's loads.
 // Measured (128 dimensions, 1024 queries): 483 us for a tenth of 10M rows, 1435 us
 // for 4M unfiltered ones, against 2505 us and ~9.5 ms of fp32 MFMA with sorted
 // lists; with all three products for every pair 706 us (the MFMAs alone 480 us:
 // 1.6 PFLOP/s, where the clock gives way to power).  Without the loads, 4M rows
-// take 980 us.  4M rows, 64 queries: 306 us, 6.3 TB/s of rows.
+// take 980 us.  64 queries: 4M rows 315 us (6.1 TB/s of rows; 306 us with one
+// 128-row workgroup a CU), 300K x 100 33 us (36 us).
 // The estimate's error against fp64, 32 x 32 blocks of 17 to 128 dimensions
 // (normal, positive, and over 2^20 of magnitudes), rms of |q|^2 + |x|^2:
 // 5.5e-8 to 1.45e-7, with fp32 MFMA 6.4e-8 to 1.73e-7 (lower in each block).
@@ -937,7 +939,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));  // (a float4 struct's 
 
 template <int KS, int QW, int QG>
 struct TkEst {
-    static constexpr int RG = TK_WAVES / QG;
+    static constexpr int RG = 2;
+    static constexpr int WAVES = RG * QG;
+    static constexpr int NT = 64 * WAVES;
     static constexpr int T = 32 * RG;         // rows of a tile
     static constexpr int QB = 32 * QW * QG;   // queries of a workgroup
     static constexpr int DP = 16 * KS;        // padded dimensions
@@ -946,7 +950,7 @@ struct TkEst {
     // on its elements.
     static constexpr int TPR = 8;
     static constexpr int V = DP / 8;          // elements a thread
-    static constexpr int RPP = TK_NT / TPR;   // rows per pass
+    static constexpr int RPP = NT / TPR;      // rows per pass
     static constexpr int P = T / RPP;         // passes
     static constexpr int RS = DP + 8;         // row stride in LDS: conflict-free 16-byte reads
 };
@@ -969,13 +973,13 @@ struct TkEstLds {
 // buffer and writes them to their lists when it is nearly full: a store to
 // memory in the tile loop would make the next wait for a tile's rows wait for
 // the store too (both count in order).
-template <int QB>
+template <int QB, int WAVES>
 struct TkGateLds {
     static constexpr uint32_t WB = 192;  // entries a wave (LDS left by the tiles)
     float2 gq[QB];  // an estimate is gq.x - acc gq.y / sx
     uint32_t cnt[QB];
-    uint2 buf[TK_WAVES][WB];    // (estimate bits, id)
-    uint16_t lq[TK_WAVES][WB];  // query within the workgroup
+    uint2 buf[WAVES][WB];     // (estimate bits, id)
+    uint16_t lq[WAVES][WB];    // query within the workgroup
 };
 
 // Scale for a squared norm: the power of two that brings the norm into
@@ -1130,7 +1134,7 @@ struct TkSplit {
 constexpr uint32_t TK_STAGE = 16;
 
 template <int KS, int QW, int QG, bool SEL, bool VEC, bool GATE>
-__global__ __launch_bounds__(TK_NT) void tk_est(TkArgs a, uint32_t n_qb, uint32_t stage)
+__global__ __launch_bounds__((TkEst<KS, QW, QG>::NT)) __attribute__((amdgpu_waves_per_eu(2))) void tk_est(TkArgs a, uint32_t n_qb, uint32_t stage)
 {
     using C = TkEst<KS, QW, QG>;
     const uint64_t rows = tk_rows(a);
@@ -1162,7 +1166,7 @@ __global__ __launch_bounds__(TK_NT) void tk_est(TkArgs a, uint32_t n_qb, uint32_
     // registers are short.
     constexpr bool QL_LDS = GATE && QW == 2;
     __shared__ alignas(16) _Float16 s_ql[QL_LDS ? C::QB * C::RS : 8];
-    using Gate = TkGateLds<GATE ? C::QB : 1>;
+    using Gate = TkGateLds<GATE ? C::QB : 1, GATE ? C::WAVES : 1>;
     __shared__ Gate G;
     const uint32_t lane = __lane_id();
     const uint32_t wave = threadIdx.x >> 6;
@@ -1409,7 +1413,7 @@ __global__ __launch_bounds__(TK_NT) void tk_est(TkArgs a, uint32_t n_qb, uint32_
     if constexpr (GATE) {
         drain();
         __syncthreads();
-        for (uint32_t i = threadIdx.x; i < C::QB; i += TK_NT)
+        for (uint32_t i = threadIdx.x; i < C::QB; i += C::NT)
             a.cand_n[static_cast<size_t>(chunk) * a.q_rows + qb * C::QB + i] = G.cnt[i];
     }
 }
@@ -1776,15 +1780,16 @@ template <int KS, int QW, int QG, bool GATE>
 void launch_est(const TkArgs& a, uint32_t n_qb, uint32_t stage, hipStream_t s)
 {
     const uint32_t grid = (a.n_cw * n_qb + 7u) / 8u * 8u;
+    constexpr int NT = TkEst<KS, QW, QG>::NT;
     CR_TIMED(GATE ? "tk_gate" : "tk_pairs", s);
     if (a.sel && a.vec)
-        tk_est<KS, QW, QG, true, true, GATE><<<grid, TK_NT, 0, s>>>(a, n_qb, stage);
+        tk_est<KS, QW, QG, true, true, GATE><<<grid, NT, 0, s>>>(a, n_qb, stage);
     else if (a.sel)
-        tk_est<KS, QW, QG, true, false, GATE><<<grid, TK_NT, 0, s>>>(a, n_qb, stage);
+        tk_est<KS, QW, QG, true, false, GATE><<<grid, NT, 0, s>>>(a, n_qb, stage);
     else if (a.vec)
-        tk_est<KS, QW, QG, false, true, GATE><<<grid, TK_NT, 0, s>>>(a, n_qb, stage);
+        tk_est<KS, QW, QG, false, true, GATE><<<grid, NT, 0, s>>>(a, n_qb, stage);
     else
-        tk_est<KS, QW, QG, false, false, GATE><<<grid, TK_NT, 0, s>>>(a, n_qb, stage);
+        tk_est<KS, QW, QG, false, false, GATE><<<grid, NT, 0, s>>>(a, n_qb, stage);
 }
 
 template <int MODE>
@@ -1885,7 +1890,7 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
     const uint32_t est_qb = few ? 64 : 256;
     const uint32_t n_qb = (n_q + est_qb - 1) / est_qb;
     a.q_rows = n_qb * est_qb;
-    a.n_cw = std::min<uint32_t>(TK_SEL_LISTS, std::max<uint32_t>(1, cus / n_qb));
+    a.n_cw = std::min<uint32_t>(TK_SEL_LISTS, std::max<uint32_t>(1, (few ? 2 : 1) * cus / n_qb));
     const uint32_t limit = g_topk_small.load();
     const uint64_t fit = TK_SCRATCH / (4ull * a.q_rows) / TK_ROWS * TK_ROWS;  // estimate rows within the scratch limit
     a.keep = static_cast<uint32_t>(std::min<uint64_t>(std::min(limit, TK_KEEP), fit));
@@ -1900,9 +1905,8 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
     a.pd_stride = std::max((a.keep + 63u) / 64u * 64u, a.sample);
     a.cand_off = a.gate && rows_ub <= a.keep;
     // Lists that hold every row a workgroup sees need no list path behind them.
-    const uint64_t tile = few ? 128 : 64;
-    const uint64_t list_rows = ((rows_ub + tile - 1) / tile + a.n_cw - 1) / a.n_cw * tile +
-                               (TK_STAGE > 1 ? tile : 0);  // two stages may give a workgroup one tile more
+    const uint64_t list_rows = ((rows_ub + TK_ROWS - 1) / TK_ROWS + a.n_cw - 1) / a.n_cw * TK_ROWS +
+                               TK_ROWS;  // two stages may give a workgroup one tile more
     const uint64_t lists_fit = TK_SCRATCH / (8ull * a.q_rows * a.n_cw);
     a.cap = static_cast<uint32_t>(list_rows <= lists_fit ? list_rows : std::min<uint64_t>(TK_CAND_CAP, lists_fit));
     a.list_off = a.gate && (a.cand_off || a.cap == list_rows);
