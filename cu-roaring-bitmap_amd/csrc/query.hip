@@ -6,7 +6,7 @@
 // loads of different queries overlap (random queries are latency-bound gathers
 // from the 256 MB Infinity Cache / HBM).  Modes 0 and 1 on an all-bitmap view
 // take the view's two-load fast path written without branches; on other
-// layouts mode 0 calls GpuRoaringView::contains and mode 1 runs a lockstep
+// layouts mode 0 searches arrays by 128-byte windows and mode 1 runs a lockstep
 // search of each lane's queries; modes 2 and 3, on every layout, call
 // GpuRoaringView::contains and wavefront_contains unchanged.
 #include <algorithm>
@@ -85,8 +85,8 @@ __global__ __launch_bounds__(Q_NT) void contains_allbitmap(GpuRoaringView v, con
 // Measured at 2^30 on 16384 array containers: clustered queries 198 Gq/s
 // (0.1%) and 161 (1%) against 102 and 77 for wavefront_contains one query at a
 // time; on uniform queries, which are bound by the L2's request rate rather
-// than by latency, lockstep searching loses (7.6 against 11.8 Gq/s at 1%), so
-// mode 0 keeps the header function there.  QI = 4 measured above 2, 8 and 16.
+// than by latency, lockstep searching loses (mode 0 is below).  QI = 4 measured
+// above 2, 8 and 16.
 constexpr int QI = 4;
 
 __global__ __launch_bounds__(Q_NT) void contains_interleaved(GpuRoaringView v, const uint32_t* __restrict__ ids,
@@ -190,6 +190,86 @@ __global__ __launch_bounds__(Q_NT) void contains_interleaved(GpuRoaringView v, c
             const uint64_t i = blk + static_cast<uint64_t>(q) * Q_NT + threadIdx.x;
             if (i < n) __builtin_nontemporal_store(r[q] ^ neg, out + i);
         }
+    }
+}
+
+// Whether a sorted array of more than AW values holds `low`: the array is read
+// in windows of AW values (128 bytes, a cache line except at the array's ends),
+// the first where `low` would lie among evenly spread values.  A window whose
+// first and last values enclose `low` holds it or nothing does; otherwise the
+// next one is the neighbour on its side, and after three a binary search of
+// what is left decides.
+constexpr uint32_t AW = 64;
+
+__device__ __forceinline__ bool array_has(const uint16_t* arr, uint32_t card, uint32_t low)
+{
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(4)));
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    const uint32_t line = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(arr) >> 1) & (AW - 1u);  // arr's place in its line
+    const u16x2 want = {static_cast<uint16_t>(low), static_cast<uint16_t>(low)};
+    uint32_t lo = 0, hi = card;  // `low` can only lie in [lo, hi)
+    uint32_t at = (low * card) >> 16;
+    for (int tries = 0; tries < 3; ++tries) {
+        // the line of value `at`, moved inside the array, at a 4-byte address
+        int32_t s = static_cast<int32_t>((line + at) & ~(AW - 1u)) - static_cast<int32_t>(line);
+        s = max(0, min(s, static_cast<int32_t>(card - AW)));
+        if ((line + static_cast<uint32_t>(s)) & 1u) s += s > 0 ? -1 : 1;  // (card > AW: one up stays inside)
+        const u32x4* p = reinterpret_cast<const u32x4*>(arr + s);
+        u32x4 w[AW / 8];
+#pragma unroll
+        for (uint32_t i = 0; i < AW / 8; ++i) w[i] = p[i];
+        u16x2 m = {0xFFFF, 0xFFFF};  // a zero half: a value equals `low`
+#pragma unroll
+        for (uint32_t i = 0; i < AW / 8; ++i)
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                m = __builtin_elementwise_min(m, static_cast<u16x2>(__builtin_bit_cast(u16x2, static_cast<uint32_t>(w[i][c])) ^ want));
+        if (low < (w[0].x & 0xFFFFu)) {
+            hi = min(hi, static_cast<uint32_t>(s));
+            at = hi > 0 ? hi - 1u : 0u;
+        } else if (low > (w[AW / 8 - 1].w >> 16)) {
+            lo = max(lo, static_cast<uint32_t>(s) + AW);
+            at = lo;
+        } else {
+            return m.x == 0 || m.y == 0;
+        }
+        if (lo >= hi) return false;
+    }
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        const uint32_t x = arr[mid];
+        if (x == low) return true;
+        if (x < low) lo = mid + 1u;
+        else hi = mid;
+    }
+    return false;
+}
+
+// Mode 0 on a view that is not all-bitmap: contains()'s rules, one query a
+// thread, arrays by windows.  A random query's binary search reads four or five
+// lines of a 655-value array, one after another; a window is one line, and at
+// uniform values the first one decides most queries.  One query a thread: a
+// thread's queries run one after another, so eight of them left a small batch
+// on few waves.  Measured at 2^30 against the header function, eight queries a
+// thread: 1% arrays 1M uniform queries 81 -> 42 us, 10M 936 -> 359 us, clustered
+// 108 -> 79 us; 0.1% arrays 10M uniform 383 -> 319 us; 5000 queries 42 -> 8 us.
+__global__ __launch_bounds__(Q_NT) void contains_windows(GpuRoaringView v, const uint32_t* __restrict__ ids, uint64_t n,
+                                                         uint32_t* __restrict__ out)
+{
+    using cu_roaring::ContainerTypeD;
+    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * Q_NT;
+    for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * Q_NT + threadIdx.x; i < n; i += stride) {
+        const uint32_t id = __builtin_nontemporal_load(ids + i);
+        const int idx = v.lookup_key(id >> 16);
+        bool r = false;
+        if (idx >= 0) {
+            const uint32_t type = static_cast<uint32_t>(v.types[idx]), off = v.offsets[idx], card = v.cardinalities[idx], low = id & 0xFFFFu;
+            if (type == static_cast<uint32_t>(ContainerTypeD::ARRAY) && card > AW)
+                r = array_has(v.array_data + (off >> 1), card, low);
+            else
+                r = v.container_contains(type, off, card, low);
+        }
+        __builtin_nontemporal_store((r ? 1u : 0u) ^ (v.negated ? 1u : 0u), out + i);
     }
 }
 
@@ -482,6 +562,10 @@ extern "C" int cr_contains_batch(const cr_gpu_roaring_view* view, const uint32_t
             contains_interleaved<<<gi, Q_NT, 0, s>>>(v, d_ids, n, d_out);
         } else if (mode == CR_QUERY_WAVEFRONT_API) {
             contains_general<CR_QUERY_WAVEFRONT><<<grid, Q_NT, 0, s>>>(v, d_ids, n, d_out);
+        } else if (mode == CR_QUERY_CONTAINS) {
+            const unsigned gw = static_cast<unsigned>(
+                std::max<uint64_t>(1, std::min<uint64_t>((n + Q_NT - 1) / Q_NT, static_cast<uint64_t>(cus) * 64u)));
+            contains_windows<<<gw, Q_NT, 0, s>>>(v, d_ids, n, d_out);
         } else {
             contains_general<CR_QUERY_CONTAINS><<<grid, Q_NT, 0, s>>>(v, d_ids, n, d_out);
         }

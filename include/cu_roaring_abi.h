@@ -51,9 +51,9 @@ extern "C" {
 /* Modes 0 and 1 answer as GpuRoaringView::contains does, in batched kernels:
  * on an all-bitmap view a copy of its two-load fast path (mode 1 reads a
  * key_index entry once when the whole wave shares a key, as
- * wavefront_contains does); on other layouts mode 0 calls the header function
- * per query and mode 1 runs its lookup rules with each lane's queries searched
- * in lockstep, for wave-coherent (clustered) batches. */
+ * wavefront_contains does); on other layouts mode 0 runs its lookup rules per
+ * query, with arrays searched a cache line at a time, and mode 1 with each
+ * lane's queries searched in lockstep, for wave-coherent (clustered) batches. */
 #define CR_QUERY_CONTAINS 0   /* GpuRoaringView::contains per lane */
 #define CR_QUERY_WAVEFRONT 1  /* wavefront_contains (== warp_contains) */
 /* Modes 2 and 3 always run the header functions wavefront_contains() and

@@ -802,3 +802,46 @@ def test_tile_sort_paths_random_sweep(gpu, i):
     torch.cuda.synchronize()
     assert np.array_equal(out.cpu().numpy().view(np.uint32), orc.contains_many(want, q)), (i, kind)
     gpu.free(g)
+
+
+def _window_arrays():
+    """Sorted u16 arrays around the 64-value windows' sizes, at even and odd
+    places of the pool, spread evenly and piled up at either end or around one
+    value, with 0 and 65535 in and out."""
+    rng = np.random.default_rng(91)
+    out = []
+    for n in (1, 63, 64, 65, 66, 127, 128, 129, 130, 191, 193, 1000, 4095, 4096):
+        for kind in ("spread", "low", "high", "steps"):
+            if kind == "spread":
+                v = rng.choice(65536, n, replace=False)
+            elif kind == "low":
+                v = np.concatenate([np.arange(n - 1), [65535]])
+            elif kind == "high":
+                v = np.concatenate([[0], 65536 - np.arange(1, n)])
+            else:
+                v = np.concatenate([30000 + 2 * np.arange(n // 2), 40000 + np.arange(n - n // 2)])
+            out.append(np.unique(v).astype(np.uint16))
+    return out
+
+
+def test_contains_array_windows(gpu):
+    """Mode 0 on compressed layouts searches arrays by 128-byte windows: every
+    value of every key, against the arrays themselves."""
+    torch = _torch()
+    arrays = _window_arrays()
+    g = gpu.upload_containers([(k, orc.TC_ARRAY, a.size, a) for k, a in enumerate(arrays)], 0, False, 0,
+                              orc.PROMOTE_KEEP_DEFAULT)
+    assert g.n_array_containers == len(arrays)
+    for k0 in range(0, len(arrays), 8):
+        q = np.arange(k0 << 16, min(len(arrays), k0 + 8) << 16, dtype=np.uint32)
+        dq = torch.from_numpy(q.view(np.int32)).cuda()
+        out = torch.empty_like(dq)
+        gpu.contains_batch(g, dq, out, gpu.QUERY_CONTAINS)
+        torch.cuda.synchronize()
+        got = out.cpu().numpy().reshape(-1, 65536)
+        for i in range(got.shape[0]):
+            want = np.zeros(65536, np.int32)
+            want[arrays[k0 + i]] = 1
+            bad = np.nonzero(got[i] != want)[0]
+            assert bad.size == 0, f"array of {arrays[k0 + i].size} at key {k0 + i}: value {bad[0]} answered {got[i][bad[0]]}"
+    gpu.free(g)
