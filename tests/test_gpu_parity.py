@@ -376,6 +376,36 @@ def test_upload_from_bitset_parity(gpu, universe, density, seed):
     gpu.free(g)
 
 
+@pytest.mark.parametrize("invert", [False, True])
+@pytest.mark.parametrize("n_chunks", [1, 2047, 2048, 2049, 4097, 6145])
+def test_upload_from_bitset_chunks_per_workgroup(gpu, n_chunks, invert):
+    """One, two, three and four chunks a workgroup (2048 workgroups), whole and
+    with a short last workgroup and chunk, half of the chunks empty in blocks
+    and one by one; an unaligned device pointer too."""
+    _say("upload_from_bitset chunks", n_chunks, invert)
+    U = 65536 * n_chunks - 1000
+    rng = np.random.default_rng(n_chunks)
+    words = np.zeros(((U + 31) // 32 + 2047) // 2048 * 2048, np.uint32).reshape(-1, 2048)
+    c = np.arange(words.shape[0])
+    kept = ((c // 37) % 2 == 0) & (rng.random(c.size) < 0.8) | (c == 0)
+    words[kept, rng.integers(0, 2048, int(kept.sum()))] = rng.integers(1, 1 << 32, int(kept.sum()), dtype=np.uint64).astype(np.uint32)
+    words[c % 101 == 3] = 0xFFFFFFFF  # full chunks
+    words = np.ascontiguousarray(words.reshape(-1)[: (U + 31) // 32])
+    words[-1] &= np.uint32((1 << (U % 32)) - 1)
+    if invert:
+        words = ~words
+        words[-1] &= np.uint32((1 << (U % 32)) - 1)
+    want = orc.upload_from_bitset(words, U)
+    g = gpu.upload_from_device_bitset(_dev_u32(words), U)
+    assert bool(g.negated) == invert
+    assert_same(gpu.download(g), want, strict=True, what="bitset chunks")
+    gpu.free(g)
+    d = _dev_u32(np.concatenate([np.zeros(1, np.uint32), words]))[1:]
+    g = gpu.upload_from_device_bitset(d, U)
+    assert_same(gpu.download(g), want, strict=True, what="bitset chunks, unaligned")
+    gpu.free(g)
+
+
 def test_upload_from_bitset_extra_words_and_tail(gpu):
     # n_words beyond ceil(U/32): inverted words past the tail stay all-ones (reference quirk)
     _say("upload_from_bitset extra words")
