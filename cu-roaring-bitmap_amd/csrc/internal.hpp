@@ -66,6 +66,20 @@ struct HostSlotGuard {
     const volatile T* host() const { return static_cast<const volatile T*>(slot.host); }
 };
 
+// A 12 KiB page of pinned host memory for a small call's inputs and results,
+// from a pool that is kept until the process ends.  Acquire before the launches
+// that use it and let the guard go after the stream's sync.
+constexpr size_t HOST_PAGE_BYTES = 12288;
+struct HostPageGuard {
+    void* host = nullptr;
+    void* dev = nullptr;
+    HostPageGuard() = default;
+    HostPageGuard(const HostPageGuard&) = delete;
+    HostPageGuard& operator=(const HostPageGuard&) = delete;
+    ~HostPageGuard();
+    int acquire();
+};
+
 // Copies `bytes` (<= HOST_SLOT_BYTES through a pinned slot) from device
 // memory once the stream reaches this point, then synchronises the stream.
 int read_back(void* host, const void* dev, size_t bytes, hipStream_t s);

@@ -79,6 +79,40 @@ void host_slot_release(HostSlot* slot)
     slot->dev = nullptr;
 }
 
+// Pages grow by blocks of 16 to the most that were ever in use at once.
+static std::mutex g_page_mu;
+static std::vector<void*> g_page_free;
+
+int HostPageGuard::acquire()
+{
+    {
+        std::lock_guard<std::mutex> lk(g_page_mu);
+        if (g_page_free.empty()) {
+            constexpr int N = 16;
+            void* blk = nullptr;
+            if (hipHostMalloc(&blk, N * HOST_PAGE_BYTES, hipHostMallocDefault) != hipSuccess || !blk) {
+                set_error("hipHostMalloc of %d pages failed", N);
+                return CR_ERR_ALLOC;
+            }
+            for (int i = N; i-- > 0;) g_page_free.push_back(static_cast<char*>(blk) + i * HOST_PAGE_BYTES);
+        }
+        host = g_page_free.back();
+        g_page_free.pop_back();
+    }
+    if (hipHostGetDevicePointer(&dev, host, 0) != hipSuccess || !dev) {
+        set_error("hipHostGetDevicePointer failed for a page");
+        return CR_ERR_HIP;  // (the guard returns the page)
+    }
+    return CR_OK;
+}
+
+HostPageGuard::~HostPageGuard()
+{
+    if (!host) return;
+    std::lock_guard<std::mutex> lk(g_page_mu);
+    g_page_free.push_back(host);
+}
+
 int read_back(void* host, const void* dev, size_t bytes, hipStream_t s)
 {
     if (bytes > HOST_SLOT_BYTES) {

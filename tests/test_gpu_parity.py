@@ -133,6 +133,36 @@ def test_upload_from_ids_input_orders(gpu, order):
     gpu.free(g)
 
 
+def _few_ids(kind, rng):
+    if kind == "one":
+        return np.array([0xFFFFFFFE]), 0xFFFFFFFF
+    if kind == "keys":  # 1024 ids of 1024 keys, the first and the last among them
+        keys = np.concatenate([[0, 65535], rng.choice(np.arange(1, 65535), 1022, replace=False)])
+        return (keys << 16) | rng.integers(0, 65535, 1024), 0xFFFFFFFF
+    if kind == "same":
+        return np.full(1024, (63 << 16) | 65535), 1 << 24
+    if kind == "dense":  # one container, every id twice
+        return np.tile(np.arange(65024, 65536), 2), 1 << 20
+    if kind == "half":  # the last universe that takes no complement, given the ids' count
+        return rng.permutation(2 * 700)[:700], 2 * 700
+    assert kind == "past_half"
+    return rng.permutation(2 * 700 - 1)[:700], 2 * 700 - 1
+
+
+@pytest.mark.parametrize("kind", ["one", "keys", "same", "dense", "half", "past_half"])
+def test_upload_from_few_host_ids(gpu, kind):
+    """Up to 1024 host ids, every container a bitmap: host grouping and one kernel;
+    the same ids from device memory take the general path."""
+    _say("upload_from_ids few", kind)
+    ids, universe = _few_ids(kind, np.random.default_rng(77))
+    ids = ids.astype(np.uint32)
+    for thr in (orc.PROMOTE_ALL, orc.PROMOTE_AUTO):
+        want = orc.upload_from_ids(ids, universe, thr, auto_l2(gpu))
+        for g in (gpu.upload_from_ids(ids, universe, thr), gpu.upload_from_device_ids(_dev_u32(ids), universe, thr)):
+            assert_same(gpu.download(g), want, strict=True, what=kind)
+            gpu.free(g)
+
+
 def test_upload_from_ids_rejects_out_of_universe_keys(gpu):
     _say("upload_from_ids invalid")
     ids = np.arange(2000, dtype=np.uint32) + (5 << 16)
