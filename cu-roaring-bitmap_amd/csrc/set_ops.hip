@@ -1764,6 +1764,11 @@ struct FusedArgs {
 //                  of all earlier words, one thread per key writes its rank.
 constexpr uint32_t KEY_RANGES = 64;
 
+// Finished workgroups and their cardinality, see mand_and.
+constexpr uint32_t DONE_CELLS = 128;
+constexpr uint32_t DONE_STRIDE = 16;  // u64s: a cell per cache line
+constexpr uint64_t DONE_ONE = 1ull << 40;
+
 __global__ __launch_bounds__(256) void mand_presence(FusedArgs args, uint32_t* gpres)
 {
     __shared__ uint32_t words[32];
@@ -1794,13 +1799,23 @@ __device__ __forceinline__ uint32_t common_word(const FusedArgs& args, const uin
         return lo >= mkp1 ? 0u : (lo + 32u <= mkp1 ? ~0u : ((1u << (mkp1 - lo)) - 1u));
     }
     uint32_t acc = ~0u;
-    for (uint32_t k = 0; k < args.count; ++k)
-        if (!((args.neg_mask >> k) & 1u)) acc &= gpres[k * 2048u + j];
+    for (uint32_t k0 = 0; k0 < args.count; k0 += 8u) {  // eight inputs' words in flight
+        uint32_t x[8];
+#pragma unroll
+        for (uint32_t i = 0; i < 8u; ++i) {
+            const uint32_t k = k0 + i;
+            x[i] = ~0u;
+            if (k < args.count && !((args.neg_mask >> k) & 1u)) x[i] = gpres[k * 2048u + j];
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < 8u; ++i) acc &= x[i];
+    }
     return acc;
 }
 
-__global__ __launch_bounds__(1024) void mand_common(FusedArgs args, const uint32_t* gpres, uint32_t mkp1,
-                                                    uint16_t* common, uint32_t* n_common)
+__global__ __launch_bounds__(1024) void mand_common(FusedArgs args, const uint32_t* gpres, uint32_t mkp1, uint32_t cap,
+                                                    uint16_t* common, uint32_t* n_common, uint64_t* done,
+                                                    uint16_t* key_index, uint32_t kidx_len)
 {
     __shared__ uint32_t lds[16];
     const uint32_t w = blockIdx.x, t = threadIdx.x;
@@ -1814,7 +1829,11 @@ __global__ __launch_bounds__(1024) void mand_common(FusedArgs args, const uint32
     uint32_t here;
     const uint32_t rank = before + block_excl_scan<1024>(present ? 1u : 0u, lds, here);
     if (present) common[rank] = static_cast<uint16_t>(key);
+    // The index is sized from the universe; a key beyond it (a bitset upload
+    // whose words outrun U) has no slot -- the reference writes out of bounds.
+    if (key < kidx_len) key_index[key] = static_cast<uint16_t>(present && rank < cap ? rank : 0xFFFFu);
     if (t == 0 && w == KEY_RANGES - 1) *n_common = before + here;
+    if (w == 0 && t <= DONE_CELLS) done[t * DONE_STRIDE] = 0;
 }
 
 __device__ __forceinline__ int32_t fused_lookup(const FusedIn& in, uint32_t key)
@@ -1838,108 +1857,101 @@ __device__ __forceinline__ int32_t fused_lookup(const FusedIn& in, uint32_t key)
     return -1;
 }
 
-__global__ __launch_bounds__(EXEC_NT) void mand_and(FusedArgs args, const uint16_t* common, const uint32_t* n_common_p,
+// Bound by HBM: every input's containers are read once, the result written once.
+// One workgroup per common key, NT threads of 512 / NT 16-byte columns; a thread
+// issues the loads of eight inputs back to back and then folds them.  Lane k of
+// each wave resolves input k's container.  Over 2^30 (16384 keys), us of the
+// kernel for 2, 3, 4, 5, 6, 8 inputs: 67, 85, 108, 132, 158, 210 with 256 threads,
+// 76, 91, 109, 129, 150, 204 with 512 (fewer loads a wave, more waves: ahead
+// where there are many inputs to read for one result), so the line is at 5.
+// With a wave per key, two inputs in flight, it was 97 at 3 and 210 at 8.
+// The last workgroup to finish hands the host the counts.  A cell carries the
+// cardinality of its workgroups (at most 2^32) and, from bit 40, how many have
+// finished, so that one atomic serves both and orders them; the last of each of
+// DONE_CELLS cells adds its cell to the top one.  (All workgroups on one cell
+// would bound the kernel: 16384 atomics on one address take 215 us.)
+constexpr uint32_t MAND_DEPTH = 8;
+
+template <bool VEC, uint32_t NT>
+__global__ __launch_bounds__(NT) void mand_and(FusedArgs args, const uint16_t* common, const uint32_t* n_common_p,
                                                     uint32_t cap, uint64_t* out_bmp, uint16_t* keys, uint8_t* types,
-                                                    uint32_t* offsets, uint16_t* cards, uint16_t* key_index,
-                                                    uint32_t kidx_len, uint32_t* total)
+                                                    uint32_t* offsets, uint16_t* cards, uint64_t* done, uint32_t* host)
 {
-    // One wavefront per common key: lane k resolves input k's container, the wave
-    // then streams every input's 8 KiB (8 x 16-byte loads per lane per input)
-    // into a register accumulator.  The total cardinality is summed per wave and
-    // added once per workgroup.
-    __shared__ uint32_t wave_total[EXEC_NT / 64];
-    const uint32_t n_common = min(*n_common_p, cap);  // cap: the containers the output was allocated for
-    const uint32_t lane = __lane_id();
-    const uint32_t n_waves = gridDim.x * (EXEC_NT / 64);
-    uint32_t my_total = 0;
-    for (uint32_t c = (blockIdx.x * EXEC_NT + threadIdx.x) >> 6; c < n_common; c += n_waves) {
+    constexpr uint32_t COLS = 512 / NT;
+    __shared__ uint32_t red[NT / 64];
+    const uint32_t n_common = *n_common_p, c = blockIdx.x, t = threadIdx.x, lane = __lane_id();
+    uint32_t pc = 0;
+    if (c < n_common) {  // (the grid is cap workgroups: the containers the output was allocated for)
         const uint32_t key = common[c];
         // The container is addressed by its index (bitmap_data + idx * 1024,
         // src/set_ops.cu:1390), not by its offset; an absent key reads as the
         // all-zeros sentinel, which a negated input turns into all-ones.
         const int32_t my_idx = lane < args.count ? fused_lookup(args.in[lane], key) : -1;
-        uint4 acc[8];
+        uint4 acc[COLS];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[j] = make_uint4(~0u, ~0u, ~0u, ~0u);
-        // Input k + 1's eight 16-byte loads are issued before input k is ANDed
-        // in, so a wave keeps two inputs' reads in flight.
-        auto src_of = [&](uint32_t k, int32_t& idx) -> const uint64_t* {
-            idx = __shfl(my_idx, static_cast<int>(k), 64);
-            return idx < 0 ? nullptr : args.in[k].bmp + static_cast<uint64_t>(idx) * 1024u;
-        };
-        auto load8 = [&](const uint64_t* p, uint4 (&x)[8]) {
-            if (!p) return;
-            if ((reinterpret_cast<uintptr_t>(p) & 15u) == 0) {
-                const uint4* p4 = reinterpret_cast<const uint4*>(p);
+        for (uint32_t j = 0; j < COLS; ++j) acc[j] = make_uint4(~0u, ~0u, ~0u, ~0u);
+        for (uint32_t k0 = 0; k0 < args.count; k0 += MAND_DEPTH) {
+            uint4 x[MAND_DEPTH][COLS];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) x[j] = ld_stream(p4 + lane + 64 * j);
-            } else {
-                const uint32_t* p32 = reinterpret_cast<const uint32_t*>(p);
+            for (uint32_t i = 0; i < MAND_DEPTH; ++i) {
+                const uint32_t k = k0 + i;
+                const int32_t idx = k < args.count ? __builtin_amdgcn_readlane(my_idx, k) : -1;
+                // (an input past the last reads as all ones)
+                const uint32_t absent = k < args.count ? 0u : ~0u;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const uint32_t b = 4 * (lane + 64 * j);
-                    x[j] = make_uint4(p32[b], p32[b + 1], p32[b + 2], p32[b + 3]);
+                for (uint32_t j = 0; j < COLS; ++j) x[i][j] = make_uint4(absent, absent, absent, absent);
+                if (idx >= 0) {
+                    const uint64_t* p = args.in[k].bmp + static_cast<uint64_t>(idx) * 1024u;
+#pragma unroll
+                    for (uint32_t j = 0; j < COLS; ++j) {
+                        const uint32_t at = t + NT * j;
+                        if (VEC) {
+                            x[i][j] = ld_stream(reinterpret_cast<const uint4*>(p) + at);
+                        } else {
+                            const uint64_t lo = p[2 * at], hi = p[2 * at + 1];
+                            x[i][j] = make_uint4(static_cast<uint32_t>(lo), static_cast<uint32_t>(lo >> 32),
+                                                 static_cast<uint32_t>(hi), static_cast<uint32_t>(hi >> 32));
+                        }
+                    }
                 }
             }
-        };
-        uint4 cur[8], nxt[8];
-        int32_t idx_cur = -1, idx_nxt = -1;
-        const uint64_t* p_cur = args.count ? src_of(0, idx_cur) : nullptr;
-        load8(p_cur, cur);
-        for (uint32_t k = 0; k < args.count; ++k) {
-            const uint64_t* p_nxt = k + 1 < args.count ? src_of(k + 1, idx_nxt) : nullptr;
-            load8(p_nxt, nxt);
-            const bool neg = (args.neg_mask >> k) & 1u;
-            if (idx_cur < 0) {
-                if (!neg) {
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) acc[j] = make_uint4(0, 0, 0, 0);
-                }
-            } else {
-                const uint32_t m = neg ? ~0u : 0u;
+            for (uint32_t i = 0; i < MAND_DEPTH; ++i) {
+                const uint32_t k = k0 + i, m = k < args.count && ((args.neg_mask >> k) & 1u) ? ~0u : 0u;
 #pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    acc[j] = make_uint4(acc[j].x & (cur[j].x ^ m), acc[j].y & (cur[j].y ^ m), acc[j].z & (cur[j].z ^ m),
-                                        acc[j].w & (cur[j].w ^ m));
+                for (uint32_t j = 0; j < COLS; ++j)
+                    acc[j] = make_uint4(acc[j].x & (x[i][j].x ^ m), acc[j].y & (x[i][j].y ^ m),
+                                        acc[j].z & (x[i][j].z ^ m), acc[j].w & (x[i][j].w ^ m));
             }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) cur[j] = nxt[j];
-            idx_cur = idx_nxt;
         }
         uint4* dst = reinterpret_cast<uint4*>(out_bmp + static_cast<uint64_t>(c) * 1024u);
-        uint32_t pc = 0;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            st_stream(dst + lane + 64 * j, acc[j]);
+        for (uint32_t j = 0; j < COLS; ++j) {
+            st_stream(dst + t + NT * j, acc[j]);
             pc += __popc(acc[j].x) + __popc(acc[j].y) + __popc(acc[j].z) + __popc(acc[j].w);
         }
-        pc = wave_sum(pc);
-        my_total += pc;
-        if (lane == 0) {
+        pc = block_sum<NT>(pc, red);
+        if (t == 0) {
             cards[c] = static_cast<uint16_t>(pc > 65535u ? 65535u : pc);  // clamp (src/set_ops.cu:1468)
             keys[c] = static_cast<uint16_t>(key);
             types[c] = CR_BITMAP;
             offsets[c] = c * 8192u;
-            // The index is sized from the universe; a key beyond it (a bitset upload
-            // whose words outrun U) has no slot -- the reference writes out of bounds.
-            if (key < kidx_len) key_index[key] = static_cast<uint16_t>(c);
         }
     }
-    if (lane == 0) wave_total[threadIdx.x >> 6] = my_total;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t s = 0;
-        for (int i = 0; i < EXEC_NT / 64; ++i) s += wave_total[i];
-        if (s) atomicAdd(total, s);  // u32 like the reference's counter (src/set_ops.cu:1652-1654)
+    if (t == 0) {
+        auto* cells = reinterpret_cast<unsigned long long*>(done);
+        const uint32_t cell = c % DONE_CELLS, members = (gridDim.x - cell + DONE_CELLS - 1) / DONE_CELLS;
+        uint64_t sum = atomicAdd(cells + (1 + cell) * DONE_STRIDE, DONE_ONE | pc) + (DONE_ONE | pc);
+        if (sum / DONE_ONE == members) {
+            const uint64_t part = DONE_ONE | (sum % DONE_ONE);
+            sum = atomicAdd(cells, part) + part;
+            if (sum / DONE_ONE == min(gridDim.x, DONE_CELLS)) {
+                volatile uint32_t* h = host;
+                h[0] = n_common;
+                h[1] = static_cast<uint32_t>(sum);  // u32 like the reference's counter (src/set_ops.cu:1652-1654)
+            }
+        }
     }
-}
-
-// n_common and the total cardinality, for the host's one read after the sync.
-__global__ void mand_finish(const uint32_t* cnt, uint32_t* host)
-{
-    volatile uint32_t* h = host;
-    h[0] = cnt[0];
-    h[1] = cnt[1];
 }
 
 static int fused_multi_and(const cr_gpu_roaring* in, uint32_t count, hipStream_t s, cr_gpu_roaring* out)
@@ -1947,11 +1959,13 @@ static int fused_multi_and(const cr_gpu_roaring* in, uint32_t count, hipStream_t
     FusedArgs args{};
     args.count = count;
     uint32_t universe = in[0].universe_size;
+    bool vec = true;  // 16-byte loads of every input
     for (uint32_t i = 0; i < count; ++i) {
         if (in[i].negated) args.neg_mask |= 1u << i;
         universe = std::max(universe, in[i].universe_size);
         args.in[i].keys = in[i].keys;
         args.in[i].bmp = in[i].bitmap_data;
+        vec = vec && (reinterpret_cast<uintptr_t>(in[i].bitmap_data) & 15u) == 0;
         args.in[i].kidx = in[i].key_index;
         args.in[i].n = in[i].n_containers;
         args.in[i].kidx_len = in[i].key_index ? in[i].max_key + 1u : 0u;
@@ -1961,23 +1975,6 @@ static int fused_multi_and(const cr_gpu_roaring* in, uint32_t count, hipStream_t
     reset(out);
     out->universe_size = universe;
 
-    Carver c;
-    const size_t o_common = c.add(2 * 65536);
-    const size_t o_cnt = c.add(2 * sizeof(uint32_t));
-    const size_t o_pres = c.add(sizeof(uint32_t) * 2048u * count);
-    Scratch sc;
-    CR_RET(sc.alloc(c.total, s));
-    uint16_t* common = sc.at<uint16_t>(o_common);
-    uint32_t* cnt = sc.at<uint32_t>(o_cnt);  // [0] n_common, [1] total cardinality
-    uint32_t* gpres = sc.at<uint32_t>(o_pres);
-    {
-        CR_TIMED("mand_keys", s);
-        mand_presence<<<dim3(KEY_RANGES, count), 256, 0, s>>>(args, gpres);
-        mand_common<<<KEY_RANGES, 1024, 0, s>>>(args, gpres, mkp1, common, cnt);
-    }
-    CR_LAUNCH_CHECK();
-    CR_RET(fill_u32(cnt + 1, 0u, 1, s));
-
     // One synchronisation: the output is allocated for the most common keys
     // there can be -- the fewest containers of a non-negated input (the common
     // keys are a subset of each one's keys), or every key of the universe when
@@ -1986,26 +1983,41 @@ static int fused_multi_and(const cr_gpu_roaring* in, uint32_t count, hipStream_t
     for (uint32_t i = 0; i < count; ++i)
         if (!in[i].negated) cap = std::min(cap, in[i].n_containers);
     if (cap == 0xFFFFFFFFu) cap = mkp1;
+    if (cap == 0) return sync_stream(s);  // src/set_ops.cu:1579-1583
     const uint32_t max_key = mkp1 == 0 ? 0u : mkp1 - 1u;
     const uint64_t kidx_len = static_cast<uint64_t>(max_key) + 1u;
+
+    Carver c;
+    const size_t o_common = c.add(2 * 65536);
+    const size_t o_done = c.add(sizeof(uint64_t) * DONE_STRIDE * (1 + DONE_CELLS));
+    const size_t o_cnt = c.add(sizeof(uint32_t));
+    const size_t o_pres = c.add(sizeof(uint32_t) * 2048u * count);
+    Scratch sc;
+    CR_RET(sc.alloc(c.total, s));
+    uint16_t* common = sc.at<uint16_t>(o_common);
+    uint64_t* done = sc.at<uint64_t>(o_done);
+    uint32_t* n_common_p = sc.at<uint32_t>(o_cnt);
+    uint32_t* gpres = sc.at<uint32_t>(o_pres);
     HostSlotGuard hs;
     CR_RET(hs.acquire());
-    if (cap > 0) {
-        const OutLayout L = plan_out(cap, kidx_len, static_cast<uint64_t>(cap) * 1024u, 0, 0);
-        CR_RET(alloc_out(out, L, cap, kidx_len, static_cast<uint64_t>(cap) * 1024u, 0, 0, s));
-        out->max_key = max_key;
-        CR_RET(fill_u16(out->key_index, 0xFFFFu, kidx_len, s));
-        CR_TIMED("mand_and", s);
-        // One common key per wave (a grid capped at 8 workgroups per CU, two
-        // keys a wave, measured 0.69 of peak against 0.71 at k = 3); waves past
-        // the common keys exit.
-        const unsigned gm = std::max(1u, (cap + 3) / 4);
-        mand_and<<<gm, EXEC_NT, 0, s>>>(args, common, cnt, cap, out->bitmap_data, out->keys, out->types,
-                                        out->offsets, out->cardinalities, out->key_index,
-                                        static_cast<uint32_t>(kidx_len), cnt + 1);
+    const OutLayout L = plan_out(cap, kidx_len, static_cast<uint64_t>(cap) * 1024u, 0, 0);
+    CR_RET(alloc_out(out, L, cap, kidx_len, static_cast<uint64_t>(cap) * 1024u, 0, 0, s));
+    out->max_key = max_key;
+    {
+        CR_TIMED("mand_keys", s);
+        mand_presence<<<dim3(KEY_RANGES, count), 256, 0, s>>>(args, gpres);
+        mand_common<<<KEY_RANGES, 1024, 0, s>>>(args, gpres, mkp1, cap, common, n_common_p, done, out->key_index,
+                                                static_cast<uint32_t>(kidx_len));
     }
     CR_LAUNCH_CHECK();
-    mand_finish<<<1, 1, 0, s>>>(cnt, hs.dev<uint32_t>());
+    {
+        CR_TIMED("mand_and", s);
+        const unsigned nt = count >= 5 ? 512 : 256;
+        auto* kernel = nt == 512 ? (vec ? mand_and<true, 512> : mand_and<false, 512>)
+                                 : (vec ? mand_and<true, 256> : mand_and<false, 256>);
+        kernel<<<cap, nt, 0, s>>>(args, common, n_common_p, cap, out->bitmap_data, out->keys, out->types,
+                                       out->offsets, out->cardinalities, done, hs.dev<uint32_t>());
+    }
     CR_LAUNCH_CHECK();
     CR_RET(sync_stream(s));
     const volatile uint32_t* h = hs.host<uint32_t>();

@@ -905,3 +905,46 @@ def test_contains_array_windows(gpu):
             bad = np.nonzero(got[i] != want)[0]
             assert bad.size == 0, f"array of {arrays[k0 + i].size} at key {k0 + i}: value {bad[0]} answered {got[i][bad[0]]}"
     gpu.free(g)
+
+
+@pytest.mark.parametrize("count", [2, 4, 5, 8, 9, 17])
+@pytest.mark.parametrize("misaligned", [False, True])
+def test_multi_and_inputs_per_pass(gpu, count, misaligned):
+    """The fused AND folds eight inputs a pass, in workgroups of 256 threads up to
+    four inputs and 512 above; a bitmap pool off 16 bytes takes 8-byte loads.  The
+    keys (200, more than the cells of finished workgroups) are missing here and
+    there, and one input is negated."""
+    _say("multi_and inputs", count, misaligned)
+    rng = np.random.default_rng(100 * count + misaligned)
+    universe = 200 * 65536
+    base = rng.random(universe) < 0.2
+    want, gs = np.ones(universe, dtype=bool), []
+    for i in range(count):
+        bits = rng.random(universe) < 0.0002 if i == 1 else base | (rng.random(universe) < 0.2)
+        if i % 3 == 0:
+            bits.reshape(200, 65536)[3 + i::23] = False
+        want &= ~bits if i == 1 else bits
+        gs.append(gpu.upload_from_ids(np.flatnonzero(bits).astype(np.uint32), universe, orc.PROMOTE_ALL))
+        assert gs[i].n_bitmap_containers == gs[i].n_containers and not gs[i].negated
+    gs[1].negated = True
+    own = gs[0].bitmap_data
+    if misaligned:
+        words = _torch().from_numpy(gpu.download(gs[0]).bitmap_data.view(np.int64))
+        moved = _torch().zeros(len(words) + 1, dtype=words.dtype, device="cuda")
+        moved[1:] = words.cuda()
+        _torch().cuda.synchronize()
+        gs[0].bitmap_data = moved.data_ptr() + 8
+    out = gpu.multi_and(gs)
+    got = gpu.download(out)
+    keys, cards = got.keys.astype(np.int64), want.reshape(200, 65536).sum(1)
+    assert got.total_cardinality == cards.sum()
+    assert len(keys) == 200 - sum(len(range(3 + i, 200, 23)) for i in range(0, min(count, 20), 3))
+    assert np.array_equal(got.cards, cards[keys])
+    bits = np.unpackbits(got.bitmap_data.view(np.uint8), bitorder="little").reshape(-1, 65536)
+    assert np.array_equal(bits, want.reshape(200, 65536)[keys])
+    index = np.full(200, 0xFFFF)
+    index[keys] = np.arange(len(keys))
+    assert np.array_equal(got.key_index, index)
+    gs[0].bitmap_data = own
+    for g in [*gs, out]:
+        gpu.free(g)
