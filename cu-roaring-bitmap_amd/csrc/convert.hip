@@ -109,7 +109,12 @@ __global__ __launch_bounds__(NT) void cv_decompress(cr_gpu_roaring r, uint32_t* 
 // Writes stay below `cap` ids.
 // Ids stored in container c (a wave computes it; every lane returns the sum):
 // a bitmap's popcount (8 loads of 16 B per lane in flight), an array's
-// cardinality, a run container's sum of (length + 1).
+// cardinality, a run container's sum of (length + 1).  AGAIN: the next kernel
+// reads the bitmaps again and they fit in the Infinity Cache, so that ordinary
+// loads leave them there (the line is at its 256 MB: 2^30 ids' 134 MB, 10% set,
+// 232 us with nontemporal loads here and 215 with ordinary ones; 250 MB, 2% set,
+// 172 and 160; 537 MB, 1% set, 320 and 330).
+template <bool AGAIN>
 __device__ inline uint32_t container_count(const cr_gpu_roaring& r, uint32_t c, uint32_t lane)
 {
     const uint8_t type = r.types[c];
@@ -122,7 +127,7 @@ __device__ inline uint32_t container_count(const cr_gpu_roaring& r, uint32_t c, 
             const uint4* bm = reinterpret_cast<const uint4*>(p);
             uint4 v[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = ld_stream(bm + j * 64 + lane);
+            for (int j = 0; j < 8; ++j) v[j] = AGAIN ? bm[j * 64 + lane] : ld_stream(bm + j * 64 + lane);
 #pragma unroll
             for (int j = 0; j < 8; ++j) n += __popc(v[j].x) + __popc(v[j].y) + __popc(v[j].z) + __popc(v[j].w);
         } else {
@@ -137,12 +142,13 @@ __device__ inline uint32_t container_count(const cr_gpu_roaring& r, uint32_t c, 
     return wave_sum(n);
 }
 
+template <bool AGAIN>
 __global__ __launch_bounds__(CV_NT) void cv_enum_count(cr_gpu_roaring r, uint64_t* counts)
 {
     const uint32_t c = (blockIdx.x * CV_NT + threadIdx.x) >> 6;
     const uint32_t lane = __lane_id();
     if (c >= r.n_containers) return;
-    const uint32_t n = container_count(r, c, lane);
+    const uint32_t n = container_count<AGAIN>(r, c, lane);
     if (lane == 0) counts[c] = n;
 }
 
@@ -160,7 +166,7 @@ __global__ __launch_bounds__(CS_NT) void cv_card_sum(cr_gpu_roaring r, unsigned 
     const uint32_t lane = __lane_id();
     const uint32_t nw = gridDim.x * (CS_NT / 64);
     unsigned long long n = 0;
-    for (uint32_t c = blockIdx.x * (CS_NT / 64) + wave; c < r.n_containers; c += nw) n += container_count(r, c, lane);
+    for (uint32_t c = blockIdx.x * (CS_NT / 64) + wave; c < r.n_containers; c += nw) n += container_count<false>(r, c, lane);
     if (lane == 0) part[wave] = n;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -257,6 +263,26 @@ __device__ __forceinline__ unsigned long long block_excl_scan_u64(unsigned long 
     return base + incl - v;
 }
 
+// ids base | stage[0, n) to out[start, ...), below cap: 16 bytes a thread between
+// an odd first and last id (2% of 2^30: the kernel 80 us with 8-byte stores, 70
+// with these).
+__device__ __forceinline__ void write_ids(const uint16_t* stage, uint32_t n, int64_t base, uint64_t start, uint64_t cap,
+                                          int64_t* out)
+{
+    if (start >= cap) return;
+    n = static_cast<uint32_t>(min(static_cast<uint64_t>(n), cap - start));
+    int64_t* dst = out + start;
+    const uint32_t t = threadIdx.x, head = (reinterpret_cast<uintptr_t>(dst) >> 3) & 1u;
+    for (uint32_t i = head + 2u * t; i + 1u < n; i += 2u * CV_NT) {
+        const uint64_t a = static_cast<uint64_t>(base | stage[i]), b = static_cast<uint64_t>(base | stage[i + 1u]);
+        st_stream(reinterpret_cast<uint4*>(dst + i),
+                  make_uint4(static_cast<uint32_t>(a), static_cast<uint32_t>(a >> 32), static_cast<uint32_t>(b),
+                             static_cast<uint32_t>(b >> 32)));
+    }
+    if (t == 0 && head && n) st_stream(dst, base | stage[0]);
+    if (t == 64 && n > head && ((n - head) & 1u)) st_stream(dst + n - 1u, base | stage[n - 1u]);
+}
+
 template <bool LEAN>
 __global__ __launch_bounds__(CV_NT) void cv_enum_write(cr_gpu_roaring r, const uint64_t* starts, uint64_t cap,
                                                        int64_t* __restrict__ out)
@@ -327,8 +353,7 @@ __global__ __launch_bounds__(CV_NT) void cv_enum_write(cr_gpu_roaring r, const u
                 stage[pos++] = static_cast<uint16_t>(32u * (wi + 1u) + __builtin_ctz(x));
         }
         __syncthreads();
-        for (uint32_t i = t; i < all; i += CV_NT)
-            if (start + i < cap) st_stream(out + start + i, base | stage[i]);
+        write_ids(stage, all, base, start, cap, out);
         return;
     }
     uint64_t written = start;
@@ -340,8 +365,7 @@ __global__ __launch_bounds__(CV_NT) void cv_enum_write(cr_gpu_roaring r, const u
         for (uint32_t x = v[ch].y; x; x &= x - 1)
             stage[pos++] = static_cast<uint16_t>(32u * (wi + 1u) + __builtin_ctz(x));
         __syncthreads();
-        for (uint32_t i = t; i < tot[ch]; i += CV_NT)
-            if (written + i < cap) st_stream(out + written + i, base | stage[i]);
+        write_ids(stage, tot[ch], base, written, cap, out);
         written += tot[ch];
         __syncthreads();
     }
@@ -524,6 +548,12 @@ int promote_impl(const cr_gpu_roaring* bm, hipStream_t s, cr_gpu_roaring* out)
     return CR_OK;
 }
 
+void launch_enum_count(const cr_gpu_roaring* bm, uint64_t* counts, hipStream_t s)
+{
+    auto* kernel = bm->n_bitmap_containers <= (256u << 20) / 8192u ? cv_enum_count<true> : cv_enum_count<false>;
+    kernel<<<(bm->n_containers + 3) / 4, CV_NT, 0, s>>>(*bm, counts);
+}
+
 // The three launches of enumerate_ids over given counts/starts buffers
 // (n_containers u64 each), untimed (enumerate_impl below times each launch).
 // cv_enum_count writes every count and the scan every start, so neither
@@ -532,7 +562,7 @@ int enumerate_launch(const cr_gpu_roaring* bm, int64_t* d_out, uint64_t cap, uin
                      hipStream_t s)
 {
     const uint32_t n = bm->n_containers;
-    cv_enum_count<<<(n + 3) / 4, CV_NT, 0, s>>>(*bm, counts);
+    launch_enum_count(bm, counts, s);
     CR_RET(scan_exclusive_u64(counts, n, starts, s));
     if (bm->n_bitmap_containers == 0 && bm->n_run_containers == 0)
         cv_enum_write_arrays<<<(n + 3) / 4, CV_NT, 0, s>>>(*bm, starts, cap, d_out);
@@ -558,7 +588,7 @@ int enumerate_impl(const cr_gpu_roaring* bm, int64_t* d_out, uint64_t cap, hipSt
     uint64_t* starts = sc.at<uint64_t>(n * 8ull);
     {
         CR_TIMED("cv_enum_count", s);
-        cv_enum_count<<<(n + 3) / 4, CV_NT, 0, s>>>(*bm, counts);
+        launch_enum_count(bm, counts, s);
     }
     {
         CR_TIMED("cv_enum_scan", s);

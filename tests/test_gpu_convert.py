@@ -116,6 +116,42 @@ def test_enumerate_capacity_bound(gpu, kind):
     gpu.free(g)
 
 
+@pytest.mark.parametrize("offset", [0, 1])
+def test_enumerate_pairs(gpu, offset):
+    """Ids go out two at a time from a 16-byte boundary: containers of odd and even
+    counts (one id, and more than the 16384 that are staged whole), a buffer on and
+    off that boundary, capacities that end anywhere in a pair."""
+    _say("enumerate pairs", offset)
+    torch = _torch()
+    rng = np.random.default_rng(5)
+    counts = [1, 2, 3, 16383, 16384, 16385, 40001, 1, 65535]
+    ids = np.concatenate([(k << 16) + np.sort(rng.choice(65536, n, replace=False)) for k, n in enumerate(counts)])
+    g = gpu.upload_from_ids(ids.astype(np.uint32), 64 << 16, orc.PROMOTE_ALL)
+    assert g.n_bitmap_containers == len(counts) and not g.negated
+    for cap in (ids.size, ids.size - 1, 0, 1, 2, 5, 6, 7, 16000, 16001):
+        buf = torch.full((ids.size + 8,), SENT64, dtype=torch.int64, device="cuda")
+        gpu.enumerate_ids(g, buf[offset:], cap)
+        gpu.synchronize()
+        got = buf.cpu().numpy()
+        assert np.array_equal(got[offset:offset + cap], ids[:cap]), cap
+        assert np.all(got[:offset] == SENT64) and np.all(got[offset + cap:] == SENT64), cap
+    gpu.free(g)
+
+
+@pytest.mark.parametrize("n", [32768, 32769])
+def test_enumerate_past_the_cache(gpu, n):
+    """256 MB of bitmaps are counted with ordinary loads, more with streaming ones."""
+    _say("enumerate cache line", n)
+    ids = ((np.arange(n, dtype=np.uint64) << 16) + (np.arange(n, dtype=np.uint64) * 40503) % 65536).astype(np.uint32)
+    g = gpu.upload_from_ids(ids, 0xFFFFFFFF, orc.PROMOTE_ALL)
+    assert g.n_bitmap_containers == n
+    buf = _torch().full((n + 2,), SENT64, dtype=_torch().int64, device="cuda")
+    gpu.enumerate_ids(g, buf)
+    gpu.synchronize()
+    assert np.array_equal(buf.cpu().numpy(), np.concatenate([ids.astype(np.int64), [SENT64, SENT64]]))
+    gpu.free(g)
+
+
 @pytest.mark.parametrize("kind", ["ids_keep", "runs_mixed", "negated_runs", "setop_result", "empty"])
 def test_enumerate_alloc(gpu, kind):
     _say("enumerate_alloc", kind)
