@@ -1,4 +1,4 @@
-// Fused filtered brute-force top-k on fp32 MFMA (no reference implementation;
+// Fused filtered brute-force top-k on the matrix cores (no reference implementation;
 // the reference motivates the path only in prose, README.md:265).
 //
 // For each query q: the k smallest squared L2 distances ||q - x_i||^2 over the

@@ -140,10 +140,9 @@ SMALL_LIMITS = {"lists": 0, "small_16384": 16384, "small_default": 1 << 18}
 
 @pytest.fixture(params=list(SMALL_LIMITS))
 def path(request, gpu):
-    """Runs a test with the small-set path off (every case on the per-chunk
-    candidate lists), with a limit of 16384 passing rows (both sides of it in
-    the cases below), and with the default limit (every case here keeps every
-    estimate and selects per query)."""
+    """Runs a test with the limit at 0 (every case on the per-chunk sorted lists),
+    at 16384 passing rows (both sides of it in the cases below), and with the
+    default limit (estimates kept, or candidates under a bound)."""
     prev = gpu.topk_set_small_limit(SMALL_LIMITS[request.param])
     yield request.param
     gpu.topk_set_small_limit(prev)
