@@ -919,7 +919,8 @@ __global__ __launch_bounds__(TK_MERGE_NT) void tk_merge(TkArgs a, const float* l
 // The estimate's error against fp64, 32 x 32 blocks of 17 to 128 dimensions
 // (normal, positive, and over 2^20 of magnitudes), rms of |q|^2 + |x|^2:
 // 5.5e-8 to 1.45e-7, with fp32 MFMA 6.4e-8 to 1.73e-7 (lower in each block).
-constexpr uint32_t TK_KEEP = 16384;         // rows whose estimates are all kept, and the sample, at most
+constexpr uint32_t TK_KEEP = 16384;         // rows whose estimates are all kept, and the sample, at most ...
+constexpr uint32_t TK_KEEP_MAX = 40960;     // ... rows kept where that is all of a call's rows
 constexpr uint32_t TK_SCRATCH = 1u << 30;   // bytes of estimates, and of candidate lists, at most
 constexpr uint32_t TK_CAND_CAP = 2048;      // candidates a list holds where it cannot hold every row
 constexpr double TK_TWO_STAGE = 1024;       // expected candidates of a query, and of all of them, above which a
@@ -1435,7 +1436,8 @@ constexpr int TK_SEL_W = TK_SEL_NT / 64;
 constexpr uint32_t TK_SEL_BINS = 1024;
 constexpr uint32_t TK_SEL_CB = 2048;   // candidates per batch
 constexpr uint32_t TK_SEL_RANK = 512;  // ... ranked by counting (one a thread) up to here, sorted above
-constexpr int TK_SEL_V = TK_KEEP / (4 * TK_SEL_NT);  // 16-byte loads a thread that hold every kept estimate
+// 16-byte loads a thread that hold every kept estimate
+constexpr int TK_SEL_V = TK_KEEP / (4 * TK_SEL_NT), TK_SEL_V_MAX = TK_KEEP_MAX / (4 * TK_SEL_NT);
 constexpr uint32_t TK_SEL_LISTS = 512;  // candidate lists a query has at most
 constexpr uint64_t TK_NOKEY = ~0ull;    // no candidate: after every (distance, id) key
 // Limit of the small-set path's rows (cr_topk_set_small_limit).
@@ -1494,7 +1496,7 @@ __device__ __forceinline__ float tk_hist_kth(TkSelLds& L, uint32_t k, float lo, 
     return fminf(hi, edge + 0x1p-20f * (fabsf(lo) + fabsf(hi)));
 }
 
-template <int MODE>
+template <int MODE, int V>
 __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, int64_t* out_id)
 {
     __shared__ TkSelLds L;
@@ -1524,7 +1526,7 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
     // The estimates: a small set's or the sample's in registers, the
     // candidate lists' through the running counts.
     const uint32_t S = MODE == TK_SEL_KEPT ? static_cast<uint32_t>(small ? n_rows : std::min<uint64_t>(n_rows, a.sample)) : 0u;
-    float4 v[MODE == TK_SEL_KEPT ? TK_SEL_V : 1];
+    float4 v[V];
     uint32_t C = 0;  // candidates in the lists
     const uint2* lists = a.cand + static_cast<size_t>(q) * a.cap;
     const size_t list_step = static_cast<size_t>(a.q_rows) * a.cap;
@@ -1532,7 +1534,7 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
     if constexpr (MODE == TK_SEL_KEPT) {
         const float* row = a.pd + static_cast<size_t>(q) * a.pd_stride;
 #pragma unroll
-        for (int i = 0; i < TK_SEL_V; ++i) {
+        for (int i = 0; i < V; ++i) {
             const uint32_t r = 4u * (t + i * TK_SEL_NT);
             v[i] = make_float4(__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""));
             if (!all_rows && r < S) {  // the row holds whole vectors
@@ -1543,7 +1545,7 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
             }
         }
 #pragma unroll
-        for (int i = 0; i < TK_SEL_V; ++i) {
+        for (int i = 0; i < V; ++i) {
             const float e[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
 #pragma unroll
             for (int c = 0; c < 4; ++c)
@@ -1589,7 +1591,7 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
     const float scale = hi > lo ? static_cast<float>(TK_SEL_BINS) / (hi - lo) : 0.f;
     if constexpr (MODE == TK_SEL_KEPT) {
 #pragma unroll
-        for (int i = 0; i < TK_SEL_V; ++i) {
+        for (int i = 0; i < V; ++i) {
             const float e[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
 #pragma unroll
             for (int c = 0; c < 4; ++c)
@@ -1728,14 +1730,14 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
     } else if constexpr (MODE == TK_SEL_KEPT) {
         uint32_t mine = 0;
 #pragma unroll
-        for (int i = 0; i < TK_SEL_V; ++i)
+        for (int i = 0; i < V; ++i)
             mine += (v[i].x <= bound ? 1u : 0u) + (v[i].y <= bound ? 1u : 0u) + (v[i].z <= bound ? 1u : 0u) +
                     (v[i].w <= bound ? 1u : 0u);
         uint32_t total;
         uint32_t at = block_excl_scan<TK_SEL_NT>(mine, L.lds, total);
         if (total <= TK_SEL_CB) {
 #pragma unroll
-            for (int i = 0; i < TK_SEL_V; ++i) {
+            for (int i = 0; i < V; ++i) {
                 const float e[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
 #pragma unroll
                 for (int c = 0; c < 4; ++c)
@@ -1792,11 +1794,11 @@ void launch_est(const TkArgs& a, uint32_t n_qb, uint32_t stage, hipStream_t s)
         tk_est<KS, QW, QG, false, false, GATE><<<grid, NT, 0, s>>>(a, n_qb, stage);
 }
 
-template <int MODE>
+template <int MODE, int V = 1>
 int launch_select(const TkArgs& a, float* out_d, int64_t* out_ids, hipStream_t s)
 {
     CR_TIMED("tk_select", s);
-    tk_select<MODE><<<a.n_q, TK_SEL_NT, 0, s>>>(a, out_d, out_ids);
+    tk_select<MODE, V><<<a.n_q, TK_SEL_NT, 0, s>>>(a, out_d, out_ids);
     CR_LAUNCH_CHECK();
     return CR_OK;
 }
@@ -1809,7 +1811,9 @@ int launch_gated(const TkArgs& a, uint32_t n_qb, bool two_stages, float* out_d, 
 {
     launch_est<KS, QW, QG, false>(a, n_qb, 0, s);
     CR_LAUNCH_CHECK();
-    CR_RET(launch_select<TK_SEL_KEPT>(a, out_d, out_ids, s));
+    const int kept = a.keep > TK_KEEP ? launch_select<TK_SEL_KEPT, TK_SEL_V_MAX>(a, out_d, out_ids, s)
+                                      : launch_select<TK_SEL_KEPT, TK_SEL_V>(a, out_d, out_ids, s);
+    CR_RET(kept);
     if (a.cand_off) return CR_OK;
     if (two_stages) {
         launch_est<KS, QW, QG, true>(a, n_qb, 1, s);
@@ -1893,7 +1897,12 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
     a.n_cw = std::min<uint32_t>(TK_SEL_LISTS, std::max<uint32_t>(1, (few ? 2 : 1) * cus / n_qb));
     const uint32_t limit = g_topk_small.load();
     const uint64_t fit = TK_SCRATCH / (4ull * a.q_rows) / TK_ROWS * TK_ROWS;  // estimate rows within the scratch limit
-    a.keep = static_cast<uint32_t>(std::min<uint64_t>(std::min(limit, TK_KEEP), fit));
+    // For few queries and up to TK_KEEP_MAX rows, two launches over every estimate
+    // are less than the sample, its bound, the candidates and the choice: 24000
+    // rows, 6 and 40 queries 26.7 and 31.9 us against 38.1 and 45.4; 40000 rows 32.2
+    // and 39.0 against 40.8 and 49.9.  With 300 queries it is 49.8 against 45.5.
+    const uint32_t most = few && rows_ub > TK_KEEP && rows_ub <= TK_KEEP_MAX ? TK_KEEP_MAX : TK_KEEP;
+    a.keep = static_cast<uint32_t>(std::min<uint64_t>(std::min(limit, most), fit));
     a.sample_lg = 14;
     static_assert(TK_KEEP == 1u << 14, "the sample is at most the kept rows");
     while ((1ull << a.sample_lg) > fit && a.sample_lg > 0) --a.sample_lg;

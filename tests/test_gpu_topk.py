@@ -195,6 +195,25 @@ def test_topk_multi_and_filter(gpu, path):
         gpu.free(g)
 
 
+@pytest.mark.parametrize("rows", [16384, 16385, 24003, 40960, 40961])
+@pytest.mark.parametrize("filtered", [False, True])
+def test_topk_kept_estimates(gpu, rows, filtered):
+    """Every estimate is kept up to 16384 rows, and for at most 64 queries up to
+    40960; otherwise the sample and candidate lists answer."""
+    _say("topk kept estimates", rows, filtered)
+    n_base = rows + 9000 if filtered else rows
+    mask = np.ones(n_base, np.uint8)
+    if filtered:
+        mask[np.random.default_rng(rows).choice(n_base, 9000, replace=False)] = 0
+    base, queries = _data(n_base, 70, 48, rows)
+    g = gpu.upload_from_ids(np.flatnonzero(mask).astype(np.uint32), n_base) if filtered else None
+    for n_q, k in ((5, 3), (70, 100)):
+        got_d, got_i = _run(gpu, base, queries[:n_q], k, g)
+        check_topk(base, queries[:n_q], k, mask, got_d, got_i)
+    if filtered:
+        gpu.free(g)
+
+
 def test_topk_understated_cardinality(gpu):
     """The host leaves the list path out when a filter's recorded cardinality
     fits the small-set limit.  A caller-built struct whose total_cardinality
