@@ -103,6 +103,7 @@ struct TkArgs {
     uint32_t* list_id;  // the same two planes
     size_t plane;       // elements per plane
     uint32_t* list_n;   // [n_chunks][n_q]: list length | (plane holding the list << 31)
+    uint32_t* tau_first;  // [n_q] the sample's bound, at which the first candidates are rounded (tau may fall since)
     uint32_t* tau;      // [n_q] bits of the smallest k-th distance any chunk has reached
     uint32_t* tau_m;    // [n_chunks][n_q] bits of each chunk's m_rank-th distance (+inf: fewer entries)
     uint32_t m_rank;    // ceil(2k / n_chunks)
@@ -1603,14 +1604,16 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
             if (tk_finite(e)) atomicAdd(&L.hist[tk_bin(e, lo, scale)], 1u);
         }
     }
-    // Candidate estimates were rounded down by up to twice TK_GATE_ROUND of the gate.
-    const float gate = MODE == TK_SEL_KEPT ? 0.f : __uint_as_float(a.tau[q]);
+    // Candidate estimates were rounded down by up to twice TK_GATE_ROUND of the
+    // gate that they passed, the first candidates' being the largest.
+    const float gate = MODE == TK_SEL_KEPT ? 0.f : __uint_as_float(a.tau_first[q]);
     float bound = tk_hist_kth(L, a.k, lo, hi);
     if (bound < __builtin_inff())
         bound = fmaxf(bound + 9.1f * TK_EST_ERR * qn + 2.f * TK_GATE_ROUND * gate, 0.f) * (1.f + 8.f * TK_EST_ERR);
     if (bound_only) {
         if (t == 0) {
             a.tau[q] = __float_as_uint(MODE == TK_SEL_KEPT ? bound : fminf(bound, gate));
+            if (MODE == TK_SEL_KEPT) a.tau_first[q] = __float_as_uint(bound);
             if (MODE == TK_SEL_KEPT && !a.list_off && q % TK_QB == 0) a.qb_over[q / TK_QB] = 0;
         }
         return;
@@ -1940,6 +1943,7 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
     const size_t o_pd = cv.add(a.gate ? static_cast<size_t>(a.q_rows) * a.pd_stride * 4 : 0);
     const bool cands = a.gate && !a.cand_off;
     const size_t o_cand = cv.add(cands ? static_cast<size_t>(a.q_rows) * a.n_cw * a.cap * 8 : 0);
+    const size_t o_tau_first = cv.add(cands ? static_cast<size_t>(n_q) * 4 : 0);
     const size_t o_candn = cv.add(cands ? static_cast<size_t>(a.q_rows) * a.n_cw * 4 : 0);
     const size_t o_qover = cv.add(cands ? static_cast<size_t>(n_q) * 4 : 0);
     const size_t o_qbover = cv.add(cands ? static_cast<size_t>(list_qb) * 4 : 0);
@@ -1953,6 +1957,7 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
     a.tau_m = sc.at<uint32_t>(o_taum);
     a.pd = sc.at<float>(o_pd);
     a.cand = sc.at<uint2>(o_cand);
+    a.tau_first = sc.at<uint32_t>(o_tau_first);
     a.cand_n = sc.at<uint32_t>(o_candn);
     a.q_over = sc.at<uint32_t>(o_qover);
     a.qb_over = sc.at<uint32_t>(o_qbover);

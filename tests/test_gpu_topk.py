@@ -339,3 +339,27 @@ def test_topk_candidates_overflow(gpu):
     got_d, got_i = _run(gpu, base, queries, 10, None)
     pick = np.arange(0, n_q, 37)
     check_topk(base, queries[pick], 10, None, got_d[pick], got_i[pick])
+
+
+@pytest.mark.parametrize("n_q", [1, 70])
+def test_topk_second_bound_rounding(gpu, n_q):
+    """The sampled rows bound the k-th distance by 1, the first tiles by less than
+    1e-6 of that: the candidates of the first tiles are rounded at the size of
+    the first bound, and nearer rows of the other tiles must still be answered."""
+    _say("topk second bound", n_q)
+    n, k = 100000, 256  # k n / 16384 > 1024: two stages
+    row = np.arange(n)
+    sampled = np.zeros(n, bool)
+    sampled[(np.arange(16384, dtype=np.uint64) * np.uint64(n)) >> np.uint64(14)] = True
+    first = row // 64 % 16 == 0  # the tiles that give the second bound
+    d = np.full(n, 2.0)
+    d[sampled & ~first] = 1.0
+    d[np.flatnonzero(first & ~sampled)[:300]] = 8e-7
+    nearest = np.flatnonzero(~first & ~sampled)[:50]
+    d[nearest] = 5e-7
+    base = np.zeros((n, 32), np.float32)
+    base[:, 0] = np.sqrt(d)
+    queries = np.zeros((n_q, 32), np.float32)
+    got_d, got_i = _run(gpu, base, queries, k, None)
+    check_topk(base, queries, k, None, got_d, got_i)
+    assert np.array_equal(np.sort(got_i[:, :50], axis=1), np.broadcast_to(nearest, (n_q, 50)))
