@@ -251,9 +251,19 @@ def test_topk_rejects_unsupported(gpu):
         gpu.topk_filtered(base, q, 5, None, d, i)
 
 
-# The estimate path past its kept rows (16384): each padded dimension count and
-# its edges, both workgroup shapes (up to 64 queries, and 256 a workgroup with
-# partial groups), one and two candidate stages (k rows > 1024 x 16384), a
+@pytest.fixture
+def keep16384(gpu):
+    """At most 16384 rows keep their estimates, whatever the number of queries:
+    larger sets go through the sample and the candidate kernel."""
+    prev = gpu.topk_set_small_limit(16384)
+    yield
+    gpu.topk_set_small_limit(prev)
+
+
+# The estimate path past its kept rows (16384 here): each padded dimension count
+# and its edges, both workgroup shapes (up to 64 queries, and 256 a workgroup
+# with partial groups), one and two candidate stages (k rows > 1024 x 16384, or
+# times the queries > 2^17 x 16384) of either shape, with a filter and without, a
 # partial last tile, and exactly one row more than is kept.
 GATED = [
     # (n_base, n_q, dim, k, filter kind, density, seed)
@@ -267,11 +277,13 @@ GATED = [
     (180000, 70, 96, 100, "none", 1.0, 38),  # two stages
     (300000, 9, 20, 200, "ids", 0.6, 39),  # two stages, a negated filter, few queries
     (600000, 3, 17, 256, "none", 1.0, 40),
+    (200000, 300, 64, 60, "ids", 0.5, 41),  # two stages, a filter, two blocks of 256 queries
+    (220000, 130, 128, 150, "keep", 0.4, 42),  # the same with key-searched ids, a partial query group
 ]
 
 
 @pytest.mark.parametrize("n_base,n_q,dim,k,kind,density,seed", GATED)
-def test_topk_gated(gpu, n_base, n_q, dim, k, kind, density, seed):
+def test_topk_gated(gpu, keep16384, n_base, n_q, dim, k, kind, density, seed):
     _say("topk gated", n_base, n_q, dim, k, kind, density, seed)
     base, queries = _data(n_base, n_q, dim, seed)
     filt, mask = _filter_from(gpu, kind, n_base, density, seed)
@@ -281,25 +293,27 @@ def test_topk_gated(gpu, n_base, n_q, dim, k, kind, density, seed):
         gpu.free(filt)
 
 
+@pytest.mark.parametrize("n_q", [20, 90])
 @pytest.mark.parametrize("scale", [1e-8, 1e-3, 1e3, 1e8])
-def test_topk_gated_scales(gpu, scale):
+def test_topk_gated_scales(gpu, keep16384, scale, n_q):
     """The split's scale follows each vector's norm: rows of very different
     norms in one set, at magnitudes far outside the range of 16-bit floats."""
-    _say("topk scales", scale)
-    base, queries = _data(30000, 20, 128, 51)
+    _say("topk scales", scale, n_q)
+    base, queries = _data(30000, n_q, 128, 51)
     base *= np.float32(scale) * np.exp2(np.arange(30000) % 23 - 11).astype(np.float32)[:, None]
     queries *= np.float32(scale)
     got_d, got_i = _run(gpu, base, queries, 20, None)
     check_topk(base, queries, 20, None, got_d, got_i)
 
 
+@pytest.mark.parametrize("n_q", [8, 80])
 @pytest.mark.parametrize("n_base", [3000, 30000])
-def test_topk_unusual_rows(gpu, n_base):
+def test_topk_unusual_rows(gpu, keep16384, n_base, n_q):
     """Rows and queries that the estimates leave out (zero, or of a norm that
     overflows or underflows) and rows with infinities or NaN: the finite
     distances are answered exactly, infinite ones come last, NaN never."""
-    _say("topk unusual", n_base)
-    base, queries = _data(n_base, 8, 64, 53)
+    _say("topk unusual", n_base, n_q)
+    base, queries = _data(n_base, n_q, 64, 53)
     base[5] = 0
     base[7] = queries[1]
     base[11] *= 1e-15
@@ -319,7 +333,7 @@ def test_topk_unusual_rows(gpu, n_base):
     few = np.array([5, 7, 13, 17, 19, 23])
     sub = np.ascontiguousarray(base[few])
     got_d, got_i = _run(gpu, sub, queries, 8, None)
-    for q in range(8):
+    for q in range(n_q):
         assert set(got_i[q, :2].tolist()) == {0, 1} and np.all(np.isfinite(got_d[q, :2]))
         assert got_i[q, 2:5].tolist() == [2, 3, 5] and np.all(np.isinf(got_d[q, 2:5]))
         assert np.all(got_i[q, 5:] == -1) and np.all(np.isinf(got_d[q, 5:]))
@@ -338,6 +352,23 @@ def test_topk_candidates_overflow(gpu):
     base[sampled] += 50
     got_d, got_i = _run(gpu, base, queries, 10, None)
     pick = np.arange(0, n_q, 37)
+    check_topk(base, queries[pick], 10, None, got_d[pick], got_i[pick])
+
+
+def test_topk_some_queries_overflow(gpu):
+    """One block of 256 queries where every third one's candidate lists overflow:
+    those are near the rows that the sample leaves out, the others near the
+    sampled ones.  The list path answers the former and leaves the latter."""
+    _say("topk some overflow")
+    n, n_q = 200000, 1024
+    base, queries = _data(n, n_q, 32, 56)
+    base *= np.float32(0.1)
+    queries *= np.float32(0.1)
+    sampled = (np.arange(16384, dtype=np.uint64) * np.uint64(n)) >> np.uint64(14)
+    base[sampled] += 50
+    queries[np.arange(n_q) % 3 != 0] += 50
+    got_d, got_i = _run(gpu, base, queries, 10, None)
+    pick = np.arange(0, n_q, 35)
     check_topk(base, queries[pick], 10, None, got_d[pick], got_i[pick])
 
 
