@@ -572,7 +572,10 @@ __global__ __launch_bounds__(TK_NT) void tk_dist(TkArgs a)
 
     const uint32_t q0 = qb * TK_QB + wave * TK_QW;
     const uint32_t nq_wave = q0 < a.n_q ? std::min<uint32_t>(TK_QW, a.n_q - q0) : 0u;
-    const bool qok = j < nq_wave;
+    // After candidates the list path answers the queries whose lists overflowed;
+    // the block's others have no state here and take no part.
+    const bool qok = j < nq_wave && (!a.gate || a.q_over[q0 + j]);
+    const bool busy = __ballot(qok) != 0;  // wave-uniform
     const size_t list_row = (static_cast<size_t>(chunk) * a.n_q + q0) * a.k;
     uint32_t* tau_q0 = a.tau + q0;
     uint32_t* tau_m_q0 = a.tau_m + static_cast<size_t>(chunk) * a.n_q + q0;
@@ -631,7 +634,7 @@ __global__ __launch_bounds__(TK_NT) void tk_dist(TkArgs a)
         }
         const float tsh_new = qok ? tk_atomic_load(tau_q0 + j) : __builtin_inff();
 
-        if (nq_wave > 0) {
+        if (busy) {
             f32x16 acc0 = {}, acc1 = {};
             const float* A0 = &L.tile[b][j * (DP + 4) + h * (DP / 2)];
             const float* A1 = A0 + 32 * (DP + 4);
@@ -793,7 +796,7 @@ __global__ __launch_bounds__(TK_NT) void tk_dist(TkArgs a)
             tidv = W.tid[j];
             if (qok) tsh = fminf(tsh, tk_atomic_load(tau_q0 + j));
         }
-        if (nq_wave > 0 && (t & 7u) == 7u)
+        if (busy && (t & 7u) == 7u)
             tsh = fminf(tsh, tk_spread_bound(a.tau_m, a.n_chunks, a.n_q, q0 + j, qok, h, a.k, a.m_rank));
     }
     if (nq_wave > 0) {
