@@ -339,6 +339,21 @@ def test_topk_unusual_rows(gpu, keep16384, n_base, n_q):
         assert np.all(got_i[q, 5:] == -1) and np.all(np.isinf(got_d[q, 5:]))
 
 
+@pytest.mark.parametrize("n_q", [9, 75])
+@pytest.mark.parametrize("n_base,k", [(9000, 10), (30000, 10), (120000, 200)])
+@pytest.mark.parametrize("far", [1e3, 1e6])
+def test_topk_far_rows(gpu, keep16384, n_base, k, far, n_q):
+    """A few rows at 10^6 and 10^12 times the others' distance, sampled ones among
+    them: the histogram of the estimates holds nearly every row in its first bin
+    and is taken again over that."""
+    _say("topk far rows", n_base, k, far, n_q)
+    base, queries = _data(n_base, n_q, 64, 57)
+    base[::97] *= np.float32(far)
+    got_d, got_i = _run(gpu, base, queries, k, None)
+    pick = np.arange(0, n_q, 5)
+    check_topk(base, queries[pick], k, None, got_d[pick], got_i[pick])
+
+
 def test_topk_candidates_overflow(gpu):
     """Every sampled row is far from the queries and every other row near, so the
     sample bounds nothing and the candidate lists (bounded at this size)
