@@ -1483,7 +1483,8 @@ __device__ __forceinline__ uint32_t tk_bin(float v, float lo, float scale)
 }
 
 // The bin of the k-th smallest of the binned values (TK_NOID with fewer), and
-// how many values the bins up to it hold.
+// how many values the bins up to it hold.  Every bin's count becomes that of the
+// bins up to it.
 __device__ __forceinline__ uint32_t tk_hist_kth(TkSelLds& L, uint32_t k, uint32_t& upto)
 {
     const uint32_t t = threadIdx.x;
@@ -1498,6 +1499,7 @@ __device__ __forceinline__ uint32_t tk_hist_kth(TkSelLds& L, uint32_t k, uint32_
         L.bin = 2 * t + (first ? 0u : 1u);
         L.upto = e + h0 + (first ? 0u : h1);
     }
+    L.hist[2 * t] = e + h0, L.hist[2 * t + 1] = e + h0 + h1;
     __syncthreads();
     upto = L.upto;
     return L.bin;
@@ -1540,13 +1542,13 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
 
     // The estimates: a small set's or the sample's in registers, the
     // candidate lists' through the running counts.
-    const uint32_t S = MODE == TK_SEL_KEPT ? static_cast<uint32_t>(small ? n_rows : std::min<uint64_t>(n_rows, a.sample)) : 0u;
+    const uint32_t S = MODE == TK_SEL_KEPT ? static_cast<uint32_t>(small || n_rows < a.sample ? n_rows : a.sample) : 0u;
     float4 v[V];
     uint32_t C = 0;  // candidates in the lists
     const uint2* lists = a.cand + static_cast<size_t>(q) * a.cap;
     const size_t list_step = static_cast<size_t>(a.q_rows) * a.cap;
     float lo = __builtin_inff(), hi = -__builtin_inff();
-    if constexpr (MODE == TK_SEL_KEPT) {
+    auto load = [&]() {
         const float* row = a.pd + static_cast<size_t>(q) * a.pd_stride;
 #pragma unroll
         for (int i = 0; i < V; ++i) {
@@ -1559,6 +1561,9 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
                 if (r + 3 >= S) v[i].w = __builtin_nanf("");
             }
         }
+    };
+    if constexpr (MODE == TK_SEL_KEPT) {
+        load();
 #pragma unroll
         for (int i = 0; i < V; ++i) {
             const float e[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
@@ -1603,7 +1608,7 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
         }
     }
     tk_block_range(L, lo, hi);
-    const float scale = hi > lo ? static_cast<float>(TK_SEL_BINS) / (hi - lo) : 0.f;
+    float scale = hi > lo ? static_cast<float>(TK_SEL_BINS) / (hi - lo) : 0.f;
     if constexpr (MODE == TK_SEL_KEPT) {
 #pragma unroll
         for (int i = 0; i < V; ++i) {
@@ -1628,16 +1633,18 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
     // cost calls that never come here 1.5 us).  One row in 2000 at 1000 times the
     // others' size, 300K rows, 64 queries: 1362 us without, 102 with.
     const uint32_t few = max(4 * a.k + 256u, bound_only ? 0u : TK_SEL_RANK);
+    bool again = false;
     for (int round = 0; round < TK_SEL_ROUNDS && upto > few && edge < hi; ++round) {
         lo = fmaxf(lo, lo + static_cast<float>(bin) * ((hi - lo) * (1.f / TK_SEL_BINS)) - 0x1p-20f * (fabsf(lo) + fabsf(hi)));
         hi = edge;
         for (uint32_t i = t; i < TK_SEL_BINS; i += TK_SEL_NT) L.hist[i] = 0;
         __syncthreads();
-        const float s1 = hi > lo ? static_cast<float>(TK_SEL_BINS) / (hi - lo) : 0.f;
+        scale = hi > lo ? static_cast<float>(TK_SEL_BINS) / (hi - lo) : 0.f;
+        again = true;
 #pragma unroll 4
         for (uint32_t i = t; i < (MODE == TK_SEL_KEPT ? S : C); i += TK_SEL_NT) {
             const float e = MODE == TK_SEL_KEPT ? a.pd[static_cast<size_t>(q) * a.pd_stride + i] : __uint_as_float(cand_at(i).x);
-            if (tk_finite(e) && e <= hi) atomicAdd(&L.hist[tk_bin(e, lo, s1)], 1u);
+            if (tk_finite(e) && e <= hi) atomicAdd(&L.hist[tk_bin(e, lo, scale)], 1u);
         }
         bin = tk_hist_kth(L, a.k, upto);
         edge = tk_edge(bin, lo, hi);
@@ -1648,12 +1655,24 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
     float bound = edge;
     if (bound < __builtin_inff())
         bound = fmaxf(bound + 9.1f * TK_EST_ERR * qn + 2.f * TK_GATE_ROUND * gate, 0.f) * (1.f + 8.f * TK_EST_ERR);
-    if (bound_only) {
+    // The margin is of the size of the norms: on vectors far from the origin it
+    // lets many through.  The rows with the k-th smallest estimates are the
+    // nearest all the same (an estimate's error is far below its bound), so
+    // their distances are taken first, and their k-th bounds the answer.  128
+    // dimensions, every coordinate moved by 20 and by 40 (|q|^2 at 317 and 1182
+    // times d_k): 10000 rows, 1024 queries 116 -> 81 us and 281 -> 110, 2M rows
+    // 3590 -> 1790 and 15.4 -> 3.6 ms.
+    const bool near_first = !all_rows && bound < __builtin_inff() &&
+                            ((again && bound > hi) || L.hist[tk_bin(bound, lo, scale)] > (bound_only ? 2 * a.k + 32u : few));
+    auto write_bound = [&]() {
         if (t == 0) {
             a.tau[q] = __float_as_uint(MODE == TK_SEL_KEPT ? bound : fminf(bound, gate));
             if (MODE == TK_SEL_KEPT) a.tau_first[q] = __float_as_uint(bound);
             if (MODE == TK_SEL_KEPT && !a.list_off && q % TK_QB == 0) a.qb_over[q / TK_QB] = 0;
         }
+    };
+    if (bound_only && !near_first) {
+        write_bound();
         return;
     }
     if (all_rows) bound = __builtin_inff();
@@ -1763,6 +1782,47 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
         __syncthreads();  // every thread has read the count
         if (n > TK_SEL_CB - TK_SEL_NT) flush(n, MODE == TK_SEL_KEPT || all_rows);
     };
+    if (near_first) {
+        // The rows up to the edge, TK_SEL_CB of them where ties make them more,
+        // which bound the k-th distance as well.  They are taken again below.
+        if constexpr (MODE == TK_SEL_KEPT) {
+            uint32_t mine = 0;
+#pragma unroll
+            for (int i = 0; i < V; ++i)
+                mine += (v[i].x <= edge ? 1u : 0u) + (v[i].y <= edge ? 1u : 0u) + (v[i].z <= edge ? 1u : 0u) +
+                        (v[i].w <= edge ? 1u : 0u);
+            uint32_t total;
+            uint32_t at = block_excl_scan<TK_SEL_NT>(mine, L.lds, total);
+#pragma unroll
+            for (int i = 0; i < V; ++i) {
+                const float e[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    if (!(e[c] <= edge)) continue;
+                    const uint32_t r = 4u * (t + i * TK_SEL_NT) + c;
+                    // (a sampled row's place in the set)
+                    if (at < TK_SEL_CB) L.key[at] = bound_only && S < n_rows ? (r * n_rows) >> a.sample_lg : r;
+                    ++at;
+                }
+            }
+            if (t == 0) L.n = total;
+        } else {
+            for (uint32_t i = t; i < C; i += TK_SEL_NT) {
+                const uint2 e = cand_at(i);
+                if (!(__uint_as_float(e.x) <= edge)) continue;
+                const uint32_t at = atomicAdd(&L.n, 1u);
+                if (at < TK_SEL_CB) L.key[at] = e.y;
+            }
+        }
+        __syncthreads();
+        flush(min(L.n, TK_SEL_CB), MODE == TK_SEL_KEPT);
+        if (bound_only) {
+            write_bound();
+            return;
+        }
+        nb = 0;
+        if constexpr (MODE == TK_SEL_KEPT) load();  // (not held in registers all the while)
+    }
     if (all_rows) {
         for (uint64_t r0 = 0; r0 < n_rows; r0 += TK_SEL_NT) {
             room();

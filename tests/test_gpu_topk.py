@@ -354,6 +354,37 @@ def test_topk_far_rows(gpu, keep16384, n_base, k, far, n_q):
     check_topk(base, queries[pick], k, None, got_d[pick], got_i[pick])
 
 
+# (n_base, n_q, dim, k, filter kind, density): kept estimates, candidates in one
+# stage and in two, with row loads of one float and of four, whole and partial
+# blocks of either workgroup shape
+OFF_CENTRE = [
+    (9000, 5, 128, 10, "none", 1.0),
+    (9000, 70, 33, 30, "ids", 0.6),
+    (30000, 60, 100, 10, "none", 1.0),
+    (40000, 300, 64, 10, "keep", 0.7),
+    (200000, 1, 96, 100, "none", 1.0),
+    (200000, 70, 31, 100, "ids", 0.8),
+]
+
+
+@pytest.mark.parametrize("n_base,n_q,dim,k,kind,density", OFF_CENTRE)
+@pytest.mark.parametrize("shift", [20.0, 300.0])
+def test_topk_off_centre(gpu, keep16384, shift, n_base, n_q, dim, k, kind, density):
+    """Vectors far from the origin, where the estimates' margin is large beside the
+    distances (300: beyond every distance in the set)."""
+    _say("topk off centre", shift, n_base, n_q, dim, k, kind, density)
+    base, queries = _data(n_base, n_q, dim, 58)
+    move = np.float32(shift) * np.where(np.arange(dim) % 3 == 0, -1, 1).astype(np.float32)
+    base += move
+    queries += move
+    filt, mask = _filter_from(gpu, kind, n_base, density, 58)
+    got_d, got_i = _run(gpu, base, queries, k, filt)
+    pick = np.arange(0, n_q, 7)
+    check_topk(base, queries[pick], k, mask, got_d[pick], got_i[pick])
+    if filt is not None:
+        gpu.free(filt)
+
+
 def test_topk_candidates_overflow(gpu):
     """Every sampled row is far from the queries and every other row near, so the
     sample bounds nothing and the candidate lists (bounded at this size)
