@@ -119,6 +119,11 @@ struct TkArgs {
     uint32_t n_cw;       // candidate lists a query has: one per workgroup of its query block
     uint32_t cap;        // entries of a list
     uint32_t q_rows;     // queries of whole query blocks
+    // A query block's centre (tk_centre), where rows and queries are taken about it.
+    uint32_t est_qb;     // queries of an estimate workgroup's block
+    float* qc;           // [n_q][dim] the queries about their blocks' centres
+    float* centre;       // [blocks][128]
+    uint32_t* moved;     // [blocks] the centre is not the origin
     uint2* cand;         // [n_cw][q_rows][cap] (estimate bits, id)
     uint32_t* cand_n;    // [n_cw][q_rows] candidates found, beyond cap too
     uint32_t* q_over;    // [n_q] the query's lists overflowed: tk_dist and tk_merge answer it
@@ -1167,6 +1172,14 @@ __global__ __launch_bounds__((TkEst<KS, QW, QG>::NT)) __attribute__((amdgpu_wave
     // Two tiles, as objects of their own: writes to one may pass reads of the other.
     __shared__ TkEstLds<KS, QW, QG> T0, T1;
     __shared__ alignas(16) float s_isq[C::QB];
+    // Candidates are found about the query block's centre.
+    __shared__ alignas(16) float s_centre[GATE ? C::DP : 4];
+    bool moved = false;  // wave-uniform
+    float c_t = 0.f;
+    if constexpr (GATE) {
+        moved = a.moved[qb] != 0;
+        c_t = a.centre[qb * 128u + min(threadIdx.x, C::DP - 1u)];  // (written to LDS once the rows are on their way)
+    }
     // Candidates rarely need the queries' lo halves: they stay in LDS where
     // registers are short.
     constexpr bool QL_LDS = GATE && QW == 2;
@@ -1254,6 +1267,21 @@ __global__ __launch_bounds__((TkEst<KS, QW, QG>::NT)) __attribute__((amdgpu_wave
             }
         }
     }
+    auto move = [&](float (&x)[C::P][C::V], const float* c) {  // one uniform branch a tile
+        if (!moved) return;
+#pragma unroll
+        for (int e = 0; e < C::V; e += 4) {
+            const f32x4 m = *reinterpret_cast<const f32x4*>(c + tk_est_col<C>(e));
+#pragma unroll
+            for (int p = 0; p < C::P; ++p)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x[p][e + i] -= m[i];
+        }
+    };
+    if constexpr (GATE) {
+        if (threadIdx.x < C::DP) s_centre[threadIdx.x] = c_t;
+        move(pre[0], a.centre + qb * 128u);
+    }
     TkSplit<C, VEC> split;
     {
         const uint32_t valid = tile_rows(0);
@@ -1286,6 +1314,7 @@ __global__ __launch_bounds__((TkEst<KS, QW, QG>::NT)) __attribute__((amdgpu_wave
         tk_est_ids<C, SEL, !GATE>(a, sp, tile_r0(t + 3), nid);  // (first: the next tile's wait for them leaves the rows)
         tk_est_rows<C, VEC>(a, id[b], pre[b]);
         const uint32_t next = tile_rows(t + 1);
+        if constexpr (GATE) move(pre[b ^ 1], s_centre);
         auto& B = b == 0 ? T0 : T1;
         auto& N = b == 0 ? T1 : T0;
         if (!busy) {
@@ -1449,6 +1478,69 @@ constexpr uint64_t TK_NOKEY = ~0ull;    // no candidate: after every (distance, 
 constexpr uint32_t TK_SMALL = 1u << 18;
 std::atomic<uint32_t> g_topk_small{TK_SMALL};
 
+// Candidates are found about a common point of a query block, which leaves
+// distances as they are and brings the norms, and with them the estimates'
+// margins, from the distance to the origin down to the spread of the vectors.  The
+// point is, dimension by dimension, the median of nine of the block's queries (a
+// few far ones do not move it), or the origin where that is nearer than a quarter
+// of the width of the middle ones of the nine.  A difference of two floats is
+// rounded at its own size, 2.4e-7 of |q|^2 + |x|^2 in a distance: TK_EST_ERR
+// holds.  The sample's selection computes it; it costs calls that need none 1 us
+// there and in the candidate kernels' start.  128 dimensions, every coordinate
+// moved by 100, 2M rows: 64 queries 58.4 ms without, 256 us with, 1024 queries 31.6
+// ms and 1125 us.  (Kept and sampled estimates stay about the origin: it would
+// be 1 to 2 us of calls of 20, and few of those rows get their distance taken.)
+struct TkCentre {
+    float v[9];
+    float med;
+
+    // Nine queries' dimension t (t < 128; past dim the one that stands in for it).
+    __device__ __forceinline__ void load(const TkArgs& a, uint32_t q)
+    {
+        const uint32_t t = threadIdx.x, q0 = q / a.est_qb * a.est_qb, n = min(a.est_qb, a.n_q - q0);
+        const uint32_t d = t < a.dim ? t : a.vec ? a.dim - 4u + (t & 3u) : a.dim - 1u;
+        if (t < 128) {
+#pragma unroll
+            for (uint32_t i = 0; i < 9; ++i) v[i] = a.queries[static_cast<size_t>(q0 + i * n / 9u) * a.dim + d];
+        }
+    }
+
+    // The median, and in red[0, 4) and red[4, 8) the parts of the squared sums of it and of the width.
+    __device__ __forceinline__ void median(const TkArgs& a, float* red)
+    {
+        const uint32_t t = threadIdx.x;
+        if (t >= 128) return;
+        float lo[3], mid[3], hi[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            float x[3];
+#pragma unroll
+            for (int j = 0; j < 3; ++j) x[j] = fabsf(v[3 * i + j]) <= 0x1p30f ? v[3 * i + j] : 0.f;
+            lo[i] = fminf(fminf(x[0], x[1]), x[2]);
+            hi[i] = fmaxf(fmaxf(x[0], x[1]), x[2]);
+            mid[i] = __builtin_amdgcn_fmed3f(x[0], x[1], x[2]);
+        }
+        med = __builtin_amdgcn_fmed3f(fmaxf(fmaxf(lo[0], lo[1]), lo[2]), __builtin_amdgcn_fmed3f(mid[0], mid[1], mid[2]),
+                                      fminf(fminf(hi[0], hi[1]), hi[2]));
+        const float w = __builtin_amdgcn_fmed3f(hi[0], hi[1], hi[2]) - __builtin_amdgcn_fmed3f(lo[0], lo[1], lo[2]);
+        const float c2 = tk_group_sum<32>(t < a.dim ? med * med : 0.f), w2 = tk_group_sum<32>(t < a.dim ? w * w : 0.f);
+        if ((t & 31u) == 31u) red[t >> 5] = c2, red[4 + (t >> 5)] = w2;
+    }
+
+    // After a barrier: query q about the centre, and the block's by its first query.
+    __device__ __forceinline__ void write(const TkArgs& a, uint32_t q, const float* red, const float* qv)
+    {
+        const uint32_t t = threadIdx.x;
+        if (t >= 128) return;
+        const bool moved = red[0] + red[1] + red[2] + red[3] > 0.0625f * (red[4] + red[5] + red[6] + red[7]);
+        const float c = moved ? med : 0.f;
+        if (t < a.dim) a.qc[static_cast<size_t>(q) * a.dim + t] = qv[t] - c;
+        if (q % a.est_qb) return;
+        a.centre[q / a.est_qb * 128u + t] = c;
+        if (t == 0) a.moved[q / a.est_qb] = moved ? 1u : 0u;
+    }
+};
+
 struct TkSelLds {
     uint64_t key[TK_SEL_CB];      // a batch: ids (or rows), then distance bits << 32 | id
     uint64_t best[2][TK_KMAX];    // the running best k, ascending (two planes)
@@ -1457,6 +1549,7 @@ struct TkSelLds {
     float qv[128];
     uint32_t lds[TK_SEL_W];
     float redf[2][TK_SEL_W];
+    float redc[8];
     uint32_t bin, upto, n;
 };
 
@@ -1532,9 +1625,14 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
     for (uint32_t i = t; i < TK_SEL_BINS; i += TK_SEL_NT) L.hist[i] = 0;
     if (t == 0) L.n = 0;
     __syncthreads();
-    float qn = 0.f;  // |q|^2, each wave by itself
+    float qn = 0.f;  // |q|^2 as the estimates have it, each wave by itself
     {
-        const float x = L.qv[t & 63u], y = L.qv[64u + (t & 63u)];
+        float x = L.qv[t & 63u], y = L.qv[64u + (t & 63u)];
+        if constexpr (MODE != TK_SEL_KEPT) {
+            const float* c = a.qc + static_cast<size_t>(q) * a.dim;
+            x = (t & 63u) < a.dim ? c[t & 63u] : 0.f;
+            y = 64u + (t & 63u) < a.dim ? c[64u + (t & 63u)] : 0.f;
+        }
         qn = x * x + y * y;
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) qn += __shfl_xor(qn, o, 64);
@@ -1562,8 +1660,11 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
             }
         }
     };
+    TkCentre centre;
     if constexpr (MODE == TK_SEL_KEPT) {
+        if (bound_only) centre.load(a, q);
         load();
+        if (bound_only) centre.median(a, L.redc);
 #pragma unroll
         for (int i = 0; i < V; ++i) {
             const float e[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
@@ -1608,6 +1709,7 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
         }
     }
     tk_block_range(L, lo, hi);
+    if (MODE == TK_SEL_KEPT && bound_only) centre.write(a, q, L.redc, L.qv);
     float scale = hi > lo ? static_cast<float>(TK_SEL_BINS) / (hi - lo) : 0.f;
     if constexpr (MODE == TK_SEL_KEPT) {
 #pragma unroll
@@ -1662,7 +1764,7 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
     // dimensions, every coordinate moved by 20 and by 40 (|q|^2 at 317 and 1182
     // times d_k): 10000 rows, 1024 queries 116 -> 81 us and 281 -> 110, 2M rows
     // 3590 -> 1790 and 15.4 -> 3.6 ms.
-    const bool near_first = !all_rows && bound < __builtin_inff() &&
+    const bool near_first = MODE != TK_SEL_BOUND && !all_rows && bound < __builtin_inff() &&
                             ((again && bound > hi) || L.hist[tk_bin(bound, lo, scale)] > (bound_only ? 2 * a.k + 32u : few));
     auto write_bound = [&]() {
         if (t == 0) {
@@ -1782,7 +1884,7 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
         __syncthreads();  // every thread has read the count
         if (n > TK_SEL_CB - TK_SEL_NT) flush(n, MODE == TK_SEL_KEPT || all_rows);
     };
-    if (near_first) {
+    if (__builtin_expect(near_first, 0)) {
         // The rows up to the edge, TK_SEL_CB of them where ties make them more,
         // which bound the k-th distance as well.  They are taken again below.
         if constexpr (MODE == TK_SEL_KEPT) {
@@ -1916,12 +2018,15 @@ int launch_gated(const TkArgs& a, uint32_t n_qb, bool two_stages, float* out_d, 
                                       : launch_select<TK_SEL_KEPT, TK_SEL_V>(a, out_d, out_ids, s);
     CR_RET(kept);
     if (a.cand_off) return CR_OK;
+    TkArgs g = a;  // the candidates' queries are the moved ones
+    g.queries = a.qc;
+    g.qvec = a.dim % 4 == 0;
     if (two_stages) {
-        launch_est<KS, QW, QG, true>(a, n_qb, 1, s);
+        launch_est<KS, QW, QG, true>(g, n_qb, 1, s);
         CR_LAUNCH_CHECK();
         CR_RET(launch_select<TK_SEL_BOUND>(a, out_d, out_ids, s));
     }
-    launch_est<KS, QW, QG, true>(a, n_qb, two_stages ? 2 : 0, s);
+    launch_est<KS, QW, QG, true>(g, n_qb, two_stages ? 2 : 0, s);
     CR_LAUNCH_CHECK();
     return launch_select<TK_SEL_CAND>(a, out_d, out_ids, s);
 }
@@ -1995,6 +2100,7 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
     const uint32_t est_qb = few ? 64 : 256;
     const uint32_t n_qb = (n_q + est_qb - 1) / est_qb;
     a.q_rows = n_qb * est_qb;
+    a.est_qb = est_qb;
     a.n_cw = std::min<uint32_t>(TK_SEL_LISTS, std::max<uint32_t>(1, (few ? 2 : 1) * cus / n_qb));
     const uint32_t limit = g_topk_small.load();
     const uint64_t fit = TK_SCRATCH / (4ull * a.q_rows) / TK_ROWS * TK_ROWS;  // estimate rows within the scratch limit
@@ -2041,6 +2147,9 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
     const size_t o_pd = cv.add(a.gate ? static_cast<size_t>(a.q_rows) * a.pd_stride * 4 : 0);
     const bool cands = a.gate && !a.cand_off;
     const size_t o_cand = cv.add(cands ? static_cast<size_t>(a.q_rows) * a.n_cw * a.cap * 8 : 0);
+    const size_t o_qc = cv.add(cands ? static_cast<size_t>(n_q) * dim * 4 : 0);
+    const size_t o_centre = cv.add(cands ? static_cast<size_t>(n_qb) * 128 * 4 : 0);
+    const size_t o_moved = cv.add(cands ? static_cast<size_t>(n_qb) * 4 : 0);
     const size_t o_tau_first = cv.add(cands ? static_cast<size_t>(n_q) * 4 : 0);
     const size_t o_candn = cv.add(cands ? static_cast<size_t>(a.q_rows) * a.n_cw * 4 : 0);
     const size_t o_qover = cv.add(cands ? static_cast<size_t>(n_q) * 4 : 0);
@@ -2055,6 +2164,9 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
     a.tau_m = sc.at<uint32_t>(o_taum);
     a.pd = sc.at<float>(o_pd);
     a.cand = sc.at<uint2>(o_cand);
+    a.qc = sc.at<float>(o_qc);
+    a.centre = sc.at<float>(o_centre);
+    a.moved = sc.at<uint32_t>(o_moved);
     a.tau_first = sc.at<uint32_t>(o_tau_first);
     a.cand_n = sc.at<uint32_t>(o_candn);
     a.q_over = sc.at<uint32_t>(o_qover);
