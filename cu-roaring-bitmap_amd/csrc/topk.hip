@@ -929,7 +929,7 @@ __global__ __launch_bounds__(TK_MERGE_NT) void tk_merge(TkArgs a, const float* l
 // (normal, positive, and over 2^20 of magnitudes), rms of |q|^2 + |x|^2:
 // 5.5e-8 to 1.45e-7, with fp32 MFMA 6.4e-8 to 1.73e-7 (lower in each block).
 constexpr uint32_t TK_KEEP = 16384;         // rows whose estimates are all kept, and the sample, at most ...
-constexpr uint32_t TK_KEEP_MAX = 40960;     // ... rows kept where that is all of a call's rows
+constexpr uint32_t TK_KEEP_MAX[] = {24576, 40960, 65536};  // ... rows kept where that is all of a call's rows
 constexpr uint32_t TK_SCRATCH = 1u << 30;   // bytes of estimates, and of candidate lists, at most
 constexpr uint32_t TK_CAND_CAP = 2048;      // candidates a list holds where it cannot hold every row
 constexpr double TK_TWO_STAGE = 1024;       // expected candidates of a query, and of all of them, above which a
@@ -1469,8 +1469,8 @@ constexpr int TK_SEL_W = TK_SEL_NT / 64;
 constexpr uint32_t TK_SEL_BINS = 1024;
 constexpr uint32_t TK_SEL_CB = 2048;   // candidates per batch
 constexpr uint32_t TK_SEL_RANK = 512;  // ... ranked by counting (one a thread) up to here, sorted above
-// 16-byte loads a thread that hold every kept estimate
-constexpr int TK_SEL_V = TK_KEEP / (4 * TK_SEL_NT), TK_SEL_V_MAX = TK_KEEP_MAX / (4 * TK_SEL_NT);
+// 16-byte loads a thread that hold `rows` kept estimates
+constexpr int tk_sel_v(uint32_t rows) { return static_cast<int>(rows / (4 * TK_SEL_NT)); }
 constexpr uint32_t TK_SEL_LISTS = 512;  // candidate lists a query has at most
 constexpr int TK_SEL_ROUNDS = 4;        // histograms beyond the first
 constexpr uint64_t TK_NOKEY = ~0ull;    // no candidate: after every (distance, id) key
@@ -2014,9 +2014,11 @@ int launch_gated(const TkArgs& a, uint32_t n_qb, bool two_stages, float* out_d, 
 {
     launch_est<KS, QW, QG, false>(a, n_qb, 0, s);
     CR_LAUNCH_CHECK();
-    const int kept = a.keep > TK_KEEP ? launch_select<TK_SEL_KEPT, TK_SEL_V_MAX>(a, out_d, out_ids, s)
-                                      : launch_select<TK_SEL_KEPT, TK_SEL_V>(a, out_d, out_ids, s);
-    CR_RET(kept);
+    auto* select = a.keep <= TK_KEEP          ? launch_select<TK_SEL_KEPT, tk_sel_v(TK_KEEP)>
+                   : a.keep <= TK_KEEP_MAX[0] ? launch_select<TK_SEL_KEPT, tk_sel_v(TK_KEEP_MAX[0])>
+                   : a.keep <= TK_KEEP_MAX[1] ? launch_select<TK_SEL_KEPT, tk_sel_v(TK_KEEP_MAX[1])>
+                                              : launch_select<TK_SEL_KEPT, tk_sel_v(TK_KEEP_MAX[2])>;
+    CR_RET(select(a, out_d, out_ids, s));
     if (a.cand_off) return CR_OK;
     TkArgs g = a;  // the candidates' queries are the moved ones
     g.queries = a.qc;
@@ -2094,30 +2096,41 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
                                  ? std::min<uint64_t>(n_base, filter->total_cardinality + filter->n_containers)
                                  : n_base;
 
+    // Rows whose estimates are all kept: two launches over every estimate are
+    // less than the sample, its bound, the candidates and the choice, as long as
+    // the estimates are few.  us kept / by candidates, 128 dimensions (64 where
+    // said): 65 queries, 17000 rows 26 / 46, 65000 rows 50 / 56 (64 dimensions,
+    // 50000 rows 41 / 39); 300 queries, 32000 rows 60 / 71, 45000 rows 77 / 76; 700
+    // queries, 24500 rows 61 / 86, 32000 rows 97 / 90.
+    const uint32_t limit = g_topk_small.load();
+    const uint32_t most = n_q <= 256 ? (dim > 64 ? 65536 : 40960) : n_q <= 512 ? 40960 : 24576;
+    a.keep = TK_KEEP;
+    for (uint32_t m : TK_KEEP_MAX)
+        if (rows_ub > a.keep && rows_ub <= most && m <= most) a.keep = m;
+    auto fit = [&](uint32_t q_rows) { return TK_SCRATCH / (4ull * q_rows) / TK_ROWS * TK_ROWS; };  // estimates within the scratch limit
+    const uint64_t fit64 = fit((n_q + 63) / 64 * 64);
+    a.keep = static_cast<uint32_t>(std::min<uint64_t>(std::min(limit, a.keep), fit64));
+    a.cand_off = rows_ub <= a.keep;
+
     // The estimate path: 256 queries a workgroup, or 64 for the few that read
-    // the rows only once anyway.
-    const bool few = n_q <= 64;
+    // the rows only once anyway and for kept rows, whose tiles are too few to share
+    // the queries' preparation (12000 rows: 65 queries 24.1 us with 256, 23.1 with 64;
+    // 256 queries 32.3 and 28.1; 1024 queries 54.4 and 51.6).
+    const bool few = n_q <= 64 || a.cand_off;
     const uint32_t est_qb = few ? 64 : 256;
     const uint32_t n_qb = (n_q + est_qb - 1) / est_qb;
     a.q_rows = n_qb * est_qb;
     a.est_qb = est_qb;
     a.n_cw = std::min<uint32_t>(TK_SEL_LISTS, std::max<uint32_t>(1, (few ? 2 : 1) * cus / n_qb));
-    const uint32_t limit = g_topk_small.load();
-    const uint64_t fit = TK_SCRATCH / (4ull * a.q_rows) / TK_ROWS * TK_ROWS;  // estimate rows within the scratch limit
-    // For few queries and up to TK_KEEP_MAX rows, two launches over every estimate
-    // are less than the sample, its bound, the candidates and the choice: 24000
-    // rows, 6 and 40 queries 26.7 and 31.9 us against 38.1 and 45.4; 40000 rows 32.2
-    // and 39.0 against 40.8 and 49.9.  With 300 queries it is 49.8 against 45.5.
-    const uint32_t most = few && rows_ub > TK_KEEP && rows_ub <= TK_KEEP_MAX ? TK_KEEP_MAX : TK_KEEP;
-    a.keep = static_cast<uint32_t>(std::min<uint64_t>(std::min(limit, most), fit));
     a.sample_lg = 14;
     static_assert(TK_KEEP == 1u << 14, "the sample is at most the kept rows");
-    while ((1ull << a.sample_lg) > fit && a.sample_lg > 0) --a.sample_lg;
+    while ((1ull << a.sample_lg) > fit(a.q_rows) && a.sample_lg > 0) --a.sample_lg;
     a.sample = 1u << a.sample_lg;
     // limit 0 turns it off; so does a batch of queries too large for a sample
     // that bounds the k-th distance.
     a.gate = limit > 0 && a.sample >= std::max<uint32_t>(1024, 8 * k);
     if (!a.gate) a.keep = 0;
+    else a.keep = static_cast<uint32_t>(std::min<uint64_t>(a.keep, fit(a.q_rows)));
     a.pd_stride = std::max((a.keep + 63u) / 64u * 64u, a.sample);
     a.cand_off = a.gate && rows_ub <= a.keep;
     // Lists that hold every row a workgroup sees need no list path behind them.

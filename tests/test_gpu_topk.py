@@ -198,8 +198,8 @@ def test_topk_multi_and_filter(gpu, path):
 @pytest.mark.parametrize("rows", [16384, 16385, 24003, 40960, 40961])
 @pytest.mark.parametrize("filtered", [False, True])
 def test_topk_kept_estimates(gpu, rows, filtered):
-    """Every estimate is kept up to 16384 rows, and for at most 64 queries up to
-    40960; otherwise the sample and candidate lists answer."""
+    """Every estimate is kept up to 40960 rows here (64 dimensions or fewer, at most
+    256 queries); past it the sample and candidate lists answer."""
     _say("topk kept estimates", rows, filtered)
     n_base = rows + 9000 if filtered else rows
     mask = np.ones(n_base, np.uint8)
@@ -212,6 +212,18 @@ def test_topk_kept_estimates(gpu, rows, filtered):
         check_topk(base, queries[:n_q], k, mask, got_d, got_i)
     if filtered:
         gpu.free(g)
+
+
+@pytest.mark.parametrize("n_q,dim,rows", [(4, 128, 65536), (4, 128, 65537), (256, 65, 65536), (257, 65, 40960),
+                                          (257, 64, 40961), (512, 32, 24577), (513, 32, 24576), (513, 96, 24577)])
+def test_topk_kept_limits(gpu, n_q, dim, rows):
+    """Both sides of the limits of the kept rows: 65536 (up to 256 queries of more
+    than 64 dimensions), 40960 (up to 512 queries), 24576."""
+    _say("topk kept limits", n_q, dim, rows)
+    base, queries = _data(rows, n_q, dim, rows + n_q)
+    got_d, got_i = _run(gpu, base, queries, 33, None)
+    pick = np.arange(0, n_q, 1 + n_q // 20)
+    check_topk(base, queries[pick], 33, None, got_d[pick], got_i[pick])
 
 
 def test_topk_understated_cardinality(gpu):
