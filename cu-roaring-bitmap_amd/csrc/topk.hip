@@ -124,7 +124,7 @@ struct TkArgs {
     float* qc;           // [n_q][dim] the queries about their blocks' centres
     float* centre;       // [blocks][128]
     uint32_t* moved;     // [blocks] the centre is not the origin
-    uint2* cand;         // [n_cw][q_rows][cap] (estimate bits, id)
+    uint2* cand;         // [n_cw][n_q][cap] (estimate bits, id)
     uint32_t* cand_n;    // [n_cw][q_rows] candidates found, beyond cap too
     uint32_t* q_over;    // [n_q] the query's lists overflowed: tk_dist and tk_merge answer it
     uint32_t* qb_over;   // [n_qb] ... any query of the block's
@@ -931,7 +931,11 @@ __global__ __launch_bounds__(TK_MERGE_NT) void tk_merge(TkArgs a, const float* l
 constexpr uint32_t TK_KEEP = 16384;         // rows whose estimates are all kept, and the sample, at most ...
 constexpr uint32_t TK_KEEP_MAX[] = {24576, 40960, 65536};  // ... rows kept where that is all of a call's rows
 constexpr uint32_t TK_SCRATCH = 1u << 30;   // bytes of estimates, and of candidate lists, at most
-constexpr uint32_t TK_CAND_CAP = 2048;      // candidates a list holds where it cannot hold every row
+// Candidates a query's lists hold together: every row up to TK_CAND_WHOLE, else TK_CAND_MANY (or eight times those
+// expected) and at most TK_CAND_CAP a list.
+constexpr uint32_t TK_CAND_WHOLE = 1u << 21;
+constexpr uint32_t TK_CAND_MANY = 1u << 18;
+constexpr uint32_t TK_CAND_CAP = 2048;
 constexpr double TK_TWO_STAGE = 1024;       // expected candidates of a query, and of all of them, above which a
 constexpr double TK_TWO_STAGE_ALL = 1 << 17;  // second bound pays
 // |q.x - hi.hi| <= (2 x 2^-11 + 2^-22) |q||x|, and 2 |q||x| <= |q|^2 + |x|^2: the
@@ -1291,7 +1295,7 @@ __global__ __launch_bounds__((TkEst<KS, QW, QG>::NT)) __attribute__((amdgpu_wave
     __syncthreads();
 
     // The workgroup's lists (TK_SCRATCH bounds them: 32-bit offsets).
-    uint2* cand = GATE ? a.cand + (static_cast<size_t>(chunk) * a.q_rows + qb * C::QB) * a.cap : nullptr;
+    uint2* cand = GATE ? a.cand + (static_cast<size_t>(chunk) * a.n_q + qb * C::QB) * a.cap : nullptr;
     uint32_t held = 0;  // candidates in the wave's buffer (uniform)
     auto drain = [&]() {
         wave_lds_fence();
@@ -1644,7 +1648,7 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
     float4 v[V];
     uint32_t C = 0;  // candidates in the lists
     const uint2* lists = a.cand + static_cast<size_t>(q) * a.cap;
-    const size_t list_step = static_cast<size_t>(a.q_rows) * a.cap;
+    const size_t list_step = static_cast<size_t>(a.n_q) * a.cap;
     float lo = __builtin_inff(), hi = -__builtin_inff();
     auto load = [&]() {
         const float* row = a.pd + static_cast<size_t>(q) * a.pd_stride;
@@ -2136,9 +2140,17 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
     // Lists that hold every row a workgroup sees need no list path behind them.
     const uint64_t list_rows = ((rows_ub + TK_ROWS - 1) / TK_ROWS + a.n_cw - 1) / a.n_cw * TK_ROWS +
                                TK_ROWS;  // two stages may give a workgroup one tile more
-    const uint64_t lists_fit = TK_SCRATCH / (8ull * a.q_rows * a.n_cw);
-    a.cap = static_cast<uint32_t>(list_rows <= lists_fit ? list_rows : std::min<uint64_t>(TK_CAND_CAP, lists_fit));
-    a.list_off = a.gate && (a.cand_off || a.cap == list_rows);
+    const uint64_t lists_fit = TK_SCRATCH / (8ull * n_q * a.n_cw);
+    const bool whole = list_rows <= std::min<uint64_t>(lists_fit, TK_CAND_WHOLE / a.n_cw);
+    // One bound from the sample lets about k rows / sample candidates a query
+    // through.  A second bound, from the first 16th of the tiles, costs two
+    // launches; it saves most of the lists, and of the cross products (a fragment
+    // computes them for any candidate it may hold).
+    const double expected = static_cast<double>(k) * static_cast<double>(rows_ub) / a.sample;
+    const bool two_stages = expected > TK_TWO_STAGE || expected * n_q > TK_TWO_STAGE_ALL;
+    const uint64_t many = std::max<uint64_t>(TK_CAND_MANY, static_cast<uint64_t>(8 * expected / (two_stages ? TK_STAGE : 1)));
+    a.cap = static_cast<uint32_t>(whole ? list_rows : std::min<uint64_t>({TK_CAND_CAP, lists_fit, many / a.n_cw}));
+    a.list_off = a.gate && (a.cand_off || whole);
 
     // The list path: enough (chunk, query block) workgroups to cover every CU once.
     const uint32_t list_qb = (n_q + TK_QB - 1) / TK_QB;
@@ -2159,7 +2171,7 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
     const size_t o_taum = cv.add(a.list_off ? 0 : static_cast<size_t>(n_chunks) * n_q * 4);
     const size_t o_pd = cv.add(a.gate ? static_cast<size_t>(a.q_rows) * a.pd_stride * 4 : 0);
     const bool cands = a.gate && !a.cand_off;
-    const size_t o_cand = cv.add(cands ? static_cast<size_t>(a.q_rows) * a.n_cw * a.cap * 8 : 0);
+    const size_t o_cand = cv.add(cands ? static_cast<size_t>(n_q) * a.n_cw * a.cap * 8 : 0);
     const size_t o_qc = cv.add(cands ? static_cast<size_t>(n_q) * dim * 4 : 0);
     const size_t o_centre = cv.add(cands ? static_cast<size_t>(n_qb) * 128 * 4 : 0);
     const size_t o_moved = cv.add(cands ? static_cast<size_t>(n_qb) * 4 : 0);
@@ -2208,12 +2220,6 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
         CR_LAUNCH_CHECK();
     }
     if (a.gate) {
-        // One bound from the sample lets about k rows / sample candidates a
-        // query through.  A second bound, from the first 16th of the tiles,
-        // costs two launches; it saves most of the lists, and of the cross
-        // products (a fragment computes them for any candidate it may hold).
-        const double cands = static_cast<double>(k) * static_cast<double>(rows_ub) / a.sample;
-        const bool two_stages = cands > TK_TWO_STAGE || cands * n_q > TK_TWO_STAGE_ALL;
         const int rc = few ? launch_gated_dim<1, 2>(a, n_qb, two_stages, d_out_dist, d_out_ids, s)
                            : launch_gated_dim<2, 4>(a, n_qb, two_stages, d_out_dist, d_out_ids, s);
         CR_RET(rc);

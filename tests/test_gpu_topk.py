@@ -214,6 +214,25 @@ def test_topk_kept_estimates(gpu, rows, filtered):
         gpu.free(g)
 
 
+@pytest.mark.parametrize("n_q,most", [(1, 80), (20, 160)])
+def test_topk_scratch_of_few_queries(gpu, n_q, most):
+    """The candidate lists are sized for the queries there are and the candidates to
+    expect: 2 MB a query, beside 4 MB of estimates (512 MB when 64 queries' lists of
+    2048 each were taken for any number)."""
+    _say("topk scratch", n_q)
+    torch = _torch()
+    base = torch.randn(3_000_000, 32, device="cuda")
+    q = torch.randn(n_q, 32, device="cuda")
+    d = torch.empty(n_q, 10, device="cuda")
+    i = torch.empty(n_q, 10, dtype=torch.int64, device="cuda")
+    torch.cuda.synchronize()
+    gpu.load().cr_mempool_trim(-1, 0)
+    before = torch.cuda.mem_get_info()[0]
+    gpu.topk_filtered(base, q, 10, None, d, i)
+    torch.cuda.synchronize()
+    assert before - torch.cuda.mem_get_info()[0] < most << 20
+
+
 @pytest.mark.parametrize("n_q,dim,rows", [(4, 128, 65536), (4, 128, 65537), (256, 65, 65536), (257, 65, 40960),
                                           (257, 64, 40961), (512, 32, 24577), (513, 32, 24576), (513, 96, 24577)])
 def test_topk_kept_limits(gpu, n_q, dim, rows):
