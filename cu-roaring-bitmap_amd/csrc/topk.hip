@@ -126,6 +126,11 @@ struct TkArgs {
     uint32_t* moved;     // [blocks] the centre is not the origin
     uint2* cand;         // [n_cw][n_q][cap] (estimate bits, id)
     uint32_t* cand_n;    // [n_cw][q_rows] candidates found, beyond cap too
+    // Up to 64 queries: a query with many candidates is answered by `parts`
+    // workgroups, each its part of them; the last one to finish merges.
+    uint32_t parts;
+    uint64_t* part_key;   // [n_q][parts][k] each part's best, ascending
+    uint32_t* part_done;  // [n_q] parts finished
     uint32_t* q_over;    // [n_q] the query's lists overflowed: tk_dist and tk_merge answer it
     uint32_t* qb_over;   // [n_qb] ... any query of the block's
     // What the host launched, from the passing count it knew: with no
@@ -1476,6 +1481,10 @@ constexpr uint32_t TK_SEL_RANK = 512;  // ... ranked by counting (one a thread) 
 // 16-byte loads a thread that hold `rows` kept estimates
 constexpr int tk_sel_v(uint32_t rows) { return static_cast<int>(rows / (4 * TK_SEL_NT)); }
 constexpr uint32_t TK_SEL_LISTS = 512;  // candidate lists a query has at most
+// Candidates from which a query's selection is split: 64 queries among 300K rows,
+// four of them so far away that every row is a candidate, 7730 us without,
+// 958 us with; below, the parts' start and merge would be most of it.
+constexpr uint32_t TK_SEL_SPLIT = 16384;
 constexpr int TK_SEL_ROUNDS = 4;        // histograms beyond the first
 constexpr uint64_t TK_NOKEY = ~0ull;    // no candidate: after every (distance, id) key
 // Limit of the small-set path's rows (cr_topk_set_small_limit).
@@ -1616,7 +1625,8 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
     __shared__ TkSelLds L;
     const uint64_t n_rows = tk_rows(a);
     const bool small = n_rows <= a.keep;
-    const uint32_t q = blockIdx.x;
+    const uint32_t q = MODE == TK_SEL_CAND ? blockIdx.x % a.n_q : blockIdx.x;
+    const uint32_t share = MODE == TK_SEL_CAND ? blockIdx.x / a.n_q : 0u;  // of the query's workgroups
     const uint32_t t = threadIdx.x;
     if (MODE != TK_SEL_KEPT && small) return;
     // More rows than kept with no candidate kernels launched, or lists that
@@ -1646,7 +1656,8 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
     // candidate lists' through the running counts.
     const uint32_t S = MODE == TK_SEL_KEPT ? static_cast<uint32_t>(small || n_rows < a.sample ? n_rows : a.sample) : 0u;
     float4 v[V];
-    uint32_t C = 0;  // candidates in the lists
+    uint32_t from = 0, C = 0;  // the workgroup's candidates in the lists: [from, C)
+    bool split = false;      // the query has other workgroups
     const uint2* lists = a.cand + static_cast<size_t>(q) * a.cap;
     const size_t list_step = static_cast<size_t>(a.n_q) * a.cap;
     float lo = __builtin_inff(), hi = -__builtin_inff();
@@ -1685,6 +1696,12 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
         if (t == 0) L.off[TK_SEL_LISTS] = C;
         __syncthreads();
         if constexpr (MODE == TK_SEL_CAND) {
+            split = a.parts > 1 && C > TK_SEL_SPLIT && !over;
+            if (share > 0 && !split) return;
+            if (split) {
+                from = static_cast<uint32_t>(static_cast<uint64_t>(C) * share / a.parts);
+                C = static_cast<uint32_t>(static_cast<uint64_t>(C) * (share + 1) / a.parts);
+            }
             if (!a.list_off) {
                 if (t == 0) {
                     a.q_over[q] = over ? 1u : 0u;
@@ -1707,7 +1724,7 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
         return lists[c * list_step + (i - L.off[c])];
     };
     if constexpr (MODE != TK_SEL_KEPT) {
-        for (uint32_t i = t; i < C; i += TK_SEL_NT) {
+        for (uint32_t i = from + t; i < C; i += TK_SEL_NT) {
             const float e = __uint_as_float(cand_at(i).x);
             if (tk_finite(e)) lo = fminf(lo, e), hi = fmaxf(hi, e);
         }
@@ -1724,7 +1741,7 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
                 if (tk_finite(e[c])) atomicAdd(&L.hist[tk_bin(e[c], lo, scale)], 1u);
         }
     } else {
-        for (uint32_t i = t; i < C; i += TK_SEL_NT) {
+        for (uint32_t i = from + t; i < C; i += TK_SEL_NT) {
             const float e = __uint_as_float(cand_at(i).x);
             if (tk_finite(e)) atomicAdd(&L.hist[tk_bin(e, lo, scale)], 1u);
         }
@@ -1748,7 +1765,7 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
         scale = hi > lo ? static_cast<float>(TK_SEL_BINS) / (hi - lo) : 0.f;
         again = true;
 #pragma unroll 4
-        for (uint32_t i = t; i < (MODE == TK_SEL_KEPT ? S : C); i += TK_SEL_NT) {
+        for (uint32_t i = from + t; i < (MODE == TK_SEL_KEPT ? S : C); i += TK_SEL_NT) {
             const float e = MODE == TK_SEL_KEPT ? a.pd[static_cast<size_t>(q) * a.pd_stride + i] : __uint_as_float(cand_at(i).x);
             if (tk_finite(e) && e <= hi) atomicAdd(&L.hist[tk_bin(e, lo, scale)], 1u);
         }
@@ -1773,7 +1790,7 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
     auto write_bound = [&]() {
         if (t == 0) {
             a.tau[q] = __float_as_uint(MODE == TK_SEL_KEPT ? bound : fminf(bound, gate));
-            if (MODE == TK_SEL_KEPT) a.tau_first[q] = __float_as_uint(bound);
+            if (MODE == TK_SEL_KEPT) a.tau_first[q] = __float_as_uint(bound), a.part_done[q] = 0;
             if (MODE == TK_SEL_KEPT && !a.list_off && q % TK_QB == 0) a.qb_over[q / TK_QB] = 0;
         }
     };
@@ -1786,6 +1803,22 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
     // Candidates in batches: fp32 direct distances, an order by (distance, id),
     // and a merge into the running best k.
     uint32_t nb = 0, cur = 0;
+    auto sort = [&](uint32_t n) {  // key[0, n), ascending
+        uint32_t P = 2;
+        while (P < n) P <<= 1;
+        for (uint32_t i = n + t; i < P; i += TK_SEL_NT) L.key[i] = TK_NOKEY;
+        __syncthreads();
+        for (uint32_t size = 2; size <= P; size <<= 1) {
+            for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+                for (uint32_t i = t; i < P / 2; i += TK_SEL_NT) {
+                    const uint32_t l = 2 * i - (i & (stride - 1));
+                    const uint64_t x = L.key[l], y = L.key[l + stride];
+                    if ((y < x) == ((l & size) == 0)) L.key[l] = y, L.key[l + stride] = x;
+                }
+                __syncthreads();
+            }
+        }
+    };
     auto flush = [&](uint32_t nbatch, bool rows) {  // the batch's ids (or rows of the set) are in key
         for (uint32_t c0 = 0; c0 < nbatch; c0 += TK_SEL_NT / 8) {  // eight threads (of one wave) per candidate
             const uint32_t c = c0 + t / 8, part = t % 8;
@@ -1836,20 +1869,7 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
                 for (uint32_t i = 0; i < nbatch; ++i) r += L.key[i] < mine ? 1u : 0u;
             if (mine != TK_NOKEY && r < a.k) L.best[cur ^ 1][r] = mine;
         } else {
-            uint32_t P = 2;
-            while (P < nbatch) P <<= 1;
-            for (uint32_t i = nbatch + t; i < P; i += TK_SEL_NT) L.key[i] = TK_NOKEY;
-            __syncthreads();
-            for (uint32_t size = 2; size <= P; size <<= 1) {
-                for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-                    for (uint32_t i = t; i < P / 2; i += TK_SEL_NT) {
-                        const uint32_t l = 2 * i - (i & (stride - 1));
-                        const uint64_t x = L.key[l], y = L.key[l + stride];
-                        if ((y < x) == ((l & size) == 0)) L.key[l] = y, L.key[l + stride] = x;
-                    }
-                    __syncthreads();
-                }
-            }
+            sort(nbatch);
             // Merge: an entry's rank is its index plus the number of entries of
             // the other list before it (all keys but TK_NOKEY are distinct).
             auto below = [](const uint64_t* p, uint32_t n, uint64_t y) {
@@ -1913,7 +1933,7 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
             }
             if (t == 0) L.n = total;
         } else {
-            for (uint32_t i = t; i < C; i += TK_SEL_NT) {
+            for (uint32_t i = from + t; i < C; i += TK_SEL_NT) {
                 const uint2 e = cand_at(i);
                 if (!(__uint_as_float(e.x) <= edge)) continue;
                 const uint32_t at = atomicAdd(&L.n, 1u);
@@ -1959,7 +1979,7 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
             }
         }
     } else {
-        for (uint32_t i0 = 0; i0 < C; i0 += TK_SEL_NT) {
+        for (uint32_t i0 = from; i0 < C; i0 += TK_SEL_NT) {
             room();
             if (i0 + t < C) {
                 const uint2 e = cand_at(i0 + t);
@@ -1970,6 +1990,23 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
     __syncthreads();
     const uint32_t left = L.n;
     if (left) flush(left, MODE == TK_SEL_KEPT || all_rows);
+    if (MODE == TK_SEL_CAND && split) {
+        uint64_t* mine = a.part_key + (static_cast<size_t>(q) * a.parts + share) * a.k;
+        for (uint32_t r = t; r < a.k; r += TK_SEL_NT) mine[r] = r < nb ? L.best[cur][r] : TK_NOKEY;
+        __threadfence();  // each thread's keys before its workgroup's count
+        __syncthreads();
+        if (t == 0) L.n = atomicAdd(&a.part_done[q], 1u);
+        __syncthreads();
+        if (L.n != a.parts - 1u) return;
+        __threadfence();
+        const uint32_t n = a.parts * a.k;  // at most TK_SEL_CB
+        const uint64_t* all = a.part_key + static_cast<size_t>(q) * n;
+        for (uint32_t i = t; i < n; i += TK_SEL_NT)
+            L.key[i] = __hip_atomic_load(all + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        sort(n);  // (a barrier first)
+        for (uint32_t r = t; r < a.k; r += TK_SEL_NT) L.best[cur][r] = L.key[r];
+        nb = a.k;
+    }
     for (uint32_t r = t; r < a.k; r += TK_SEL_NT) {
         const uint64_t x = r < nb ? L.best[cur][r] : TK_NOKEY;
         const bool ok = x != TK_NOKEY;
@@ -2005,7 +2042,7 @@ template <int MODE, int V = 1>
 int launch_select(const TkArgs& a, float* out_d, int64_t* out_ids, hipStream_t s)
 {
     CR_TIMED("tk_select", s);
-    tk_select<MODE, V><<<a.n_q, TK_SEL_NT, 0, s>>>(a, out_d, out_ids);
+    tk_select<MODE, V><<<MODE == TK_SEL_CAND ? a.n_q * a.parts : a.n_q, TK_SEL_NT, 0, s>>>(a, out_d, out_ids);
     CR_LAUNCH_CHECK();
     return CR_OK;
 }
@@ -2175,6 +2212,9 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
     const size_t o_qc = cv.add(cands ? static_cast<size_t>(n_q) * dim * 4 : 0);
     const size_t o_centre = cv.add(cands ? static_cast<size_t>(n_qb) * 128 * 4 : 0);
     const size_t o_moved = cv.add(cands ? static_cast<size_t>(n_qb) * 4 : 0);
+    a.parts = n_q <= 64 ? std::max<uint32_t>(1, std::min<uint32_t>({64, 4 * cus / n_q, TK_SEL_CB / k})) : 1;
+    const size_t o_pkey = cv.add(cands ? static_cast<size_t>(n_q) * a.parts * k * 8 : 0);
+    const size_t o_pdone = cv.add(cands ? static_cast<size_t>(n_q) * 4 : 0);
     const size_t o_tau_first = cv.add(cands ? static_cast<size_t>(n_q) * 4 : 0);
     const size_t o_candn = cv.add(cands ? static_cast<size_t>(a.q_rows) * a.n_cw * 4 : 0);
     const size_t o_qover = cv.add(cands ? static_cast<size_t>(n_q) * 4 : 0);
@@ -2192,6 +2232,8 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
     a.qc = sc.at<float>(o_qc);
     a.centre = sc.at<float>(o_centre);
     a.moved = sc.at<uint32_t>(o_moved);
+    a.part_key = sc.at<uint64_t>(o_pkey);
+    a.part_done = sc.at<uint32_t>(o_pdone);
     a.tau_first = sc.at<uint32_t>(o_tau_first);
     a.cand_n = sc.at<uint32_t>(o_candn);
     a.q_over = sc.at<uint32_t>(o_qover);

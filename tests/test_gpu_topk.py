@@ -214,6 +214,22 @@ def test_topk_kept_estimates(gpu, rows, filtered):
         gpu.free(g)
 
 
+@pytest.mark.parametrize("n_q,k", [(2, 10), (9, 256), (64, 33), (70, 10)])
+@pytest.mark.parametrize("n_base", [100000, 2200000])
+def test_topk_two_far_modes(gpu, n_base, n_q, k):
+    """Half of the rows and every second query 4000 away from the others: one
+    point is a centre for one half only, and every near row is a candidate of the
+    other half's queries, whose selection is split over several workgroups (up to 64
+    queries; the larger set's lists cannot hold every row)."""
+    _say("topk two modes", n_base, n_q, k)
+    base, queries = _data(n_base, n_q, 16, 59)
+    base[1::2] += 1000
+    queries[1::2] += 1000
+    got_d, got_i = _run(gpu, base, queries, k, None)
+    pick = np.arange(0, n_q, 1 + n_q // 6)
+    check_topk(base, queries[pick], k, None, got_d[pick], got_i[pick])
+
+
 @pytest.mark.parametrize("n_q,most", [(1, 80), (20, 160)])
 def test_topk_scratch_of_few_queries(gpu, n_q, most):
     """The candidate lists are sized for the queries there are and the candidates to
