@@ -28,7 +28,7 @@ struct BsTotals {
 // A workgroup's chunks together: their popcount, and how many are kept
 // (non-empty) as they are and inverted.
 struct alignas(16) BsPart {
-    uint32_t total;  // at most 32 chunks of 65536
+    uint32_t total;  // at most BS_PER chunks of 65536
     uint32_t kept, kept_inv;
 };
 
@@ -252,7 +252,7 @@ int upload_from_device_bitset_impl(const uint32_t* d_words, uint32_t n_words, ui
     g.tail_mask = tail_bits ? ((1u << tail_bits) - 1u) : ~0u;
 
     const uint32_t want = std::max(1u, std::min<uint32_t>(BS_GROUPS, num_cus() * 8u));  // workgroups
-    g.per = std::max((g.n_chunks + want - 1) / want, (g.n_chunks + BS_GROUPS - 1) / BS_GROUPS);
+    g.per = (g.n_chunks + want - 1) / want;
     if (g.per > BS_PER) g.per = BS_PER;  // (65536 chunks in BS_PER each are 1024 workgroups)
     const unsigned grid = (g.n_chunks + g.per - 1) / g.per;
 
