@@ -1487,7 +1487,7 @@ constexpr uint32_t TK_SEL_LISTS = 512;  // candidate lists a query has at most
 constexpr uint32_t TK_SEL_SPLIT = 16384;
 constexpr int TK_SEL_ROUNDS = 4;        // histograms beyond the first
 constexpr uint64_t TK_NOKEY = ~0ull;    // no candidate: after every (distance, id) key
-// Limit of the small-set path's rows (cr_topk_set_small_limit).
+// The largest limit that cr_topk_set_small_limit records (any from the last of TK_KEEP_MAX on is no limit).
 constexpr uint32_t TK_SMALL = 1u << 18;
 std::atomic<uint32_t> g_topk_small{TK_SMALL};
 

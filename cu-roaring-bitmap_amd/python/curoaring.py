@@ -331,8 +331,9 @@ def contains_batch(g: GpuRoaring, d_ids, d_out, mode: int = QUERY_CONTAINS, stre
 
 def topk_set_small_limit(rows: int) -> int:
     """Rows at or below which the top-k may keep every estimate and select per
-    query (capped at 262144; 0 turns the estimates off: sorted lists answer).
-    Returns the previous limit."""
+    query (it does so up to 65536 rows at most, so larger limits, recorded up to
+    262144, are alike; 0 turns the estimates off: sorted lists answer).  Returns
+    the previous limit."""
     return int(load().cr_topk_set_small_limit(rows))
 
 

@@ -244,12 +244,14 @@ int cr_topk_filtered(const float* d_base, uint64_t n_base, const float* d_querie
                      const cr_gpu_roaring* filter, uint32_t k, float* d_out_dist, int64_t* d_out_ids,
                      cr_stream_t stream);
 /* Tuning of cr_topk_filtered (no counterpart in the reference).  A set of at
- * most `rows` passing vectors (capped at 262144, the default) may have every
- * distance estimate kept and one workgroup per query select its k from them;
- * larger sets, and those past 16384 rows or 1 GiB of estimates whatever the
- * limit, get candidate lists under a bound from a sample.  0 turns both off:
- * sorted per-chunk lists answer.  Every path gives the same answer.
- * Process-wide; returns the previous limit. */
+ * most `rows` passing vectors may have every distance estimate kept and one
+ * workgroup per query select its k from them: up to 65536 rows for at most 256
+ * queries (40960 for 64 dimensions or fewer), 40960 for at most 512 queries and
+ * 24576 for more, while the estimates fit 1 GiB.  Larger sets, and those past
+ * `rows`, get candidate lists under a bound from a sample.  The default, which
+ * is also the most that is recorded, is 262144: limits of 65536 and more all do
+ * the same.  0 turns both off: sorted per-chunk lists answer.  Every path gives
+ * the same answer.  Process-wide; returns the previous limit. */
 uint32_t cr_topk_set_small_limit(uint32_t rows);
 
 /* ---- conversions --------------------------------------------------------
