@@ -5,6 +5,7 @@
 #include <condition_variable>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <unordered_map>
@@ -81,7 +82,8 @@ void host_slot_release(HostSlot* slot)
 
 // Pages grow by blocks of 16 to the most that were ever in use at once.
 static std::mutex g_page_mu;
-static std::vector<void*> g_page_free;
+static std::vector<void*> g_page_free;  // its capacity is at least the pages there are: giving one back allocates nothing
+static size_t g_pages = 0;
 
 int HostPageGuard::acquire()
 {
@@ -89,12 +91,19 @@ int HostPageGuard::acquire()
         std::lock_guard<std::mutex> lk(g_page_mu);
         if (g_page_free.empty()) {
             constexpr int N = 16;
+            try {
+                g_page_free.reserve(g_pages + N);
+            } catch (const std::bad_alloc&) {
+                set_error("out of host memory for %zu page records", g_pages + N);
+                return CR_ERR_ALLOC;
+            }
             void* blk = nullptr;
             if (hipHostMalloc(&blk, N * HOST_PAGE_BYTES, hipHostMallocDefault) != hipSuccess || !blk) {
                 set_error("hipHostMalloc of %d pages failed", N);
                 return CR_ERR_ALLOC;
             }
             for (int i = N; i-- > 0;) g_page_free.push_back(static_cast<char*>(blk) + i * HOST_PAGE_BYTES);
+            g_pages += N;
         }
         host = g_page_free.back();
         g_page_free.pop_back();

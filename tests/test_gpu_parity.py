@@ -948,3 +948,29 @@ def test_multi_and_inputs_per_pass(gpu, count, misaligned):
     gs[0].bitmap_data = own
     for g in [*gs, out]:
         gpu.free(g)
+
+
+def test_small_host_uploads_from_many_threads(gpu):
+    """Small host uploads at the same time, more of them than a block of the pinned
+    pages that they read holds: each gets its own result."""
+    import threading
+    _say("small host uploads, 40 threads")
+    U, got = 3_000_000, [None] * 40
+    sets = [np.random.default_rng(900 + i).integers(0, U, 1000, dtype=np.uint32) for i in range(40)]
+    start = threading.Barrier(40)
+
+    def work(i):
+        start.wait(30)
+        for _ in range(5):
+            if got[i] is not None:
+                gpu.free(got[i])
+            got[i] = gpu.upload_from_ids(sets[i], U, orc.PROMOTE_ALL)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(40)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    for i in range(40):
+        assert_same(gpu.download(got[i]), orc.upload_from_ids(sets[i], U, orc.PROMOTE_ALL), strict=True, what=f"thread {i}")
+        gpu.free(got[i])
