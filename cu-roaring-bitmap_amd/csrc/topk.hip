@@ -1560,6 +1560,7 @@ struct TkSelLds {
     uint32_t hist[TK_SEL_BINS];
     uint32_t off[TK_SEL_LISTS + 1];
     float qv[128];
+    float qc[128];  // (candidates) the query about its block's centre
     uint32_t lds[TK_SEL_W];
     float redf[2][TK_SEL_W];
     float redc[8];
@@ -1635,18 +1636,18 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
     // candidate (exact, slower; no estimate is read).
     bool all_rows = MODE == TK_SEL_KEPT && !small && a.cand_off;
     const bool bound_only = MODE == TK_SEL_BOUND || (MODE == TK_SEL_KEPT && !small && !all_rows);
-    for (uint32_t c = t; c < 128; c += TK_SEL_NT) L.qv[c] = c < a.dim ? a.queries[static_cast<size_t>(q) * a.dim + c] : 0.f;
+    for (uint32_t c = t; c < 128; c += TK_SEL_NT) {
+        const size_t at = static_cast<size_t>(q) * a.dim + c;
+        L.qv[c] = c < a.dim ? a.queries[at] : 0.f;
+        if (MODE != TK_SEL_KEPT) L.qc[c] = c < a.dim ? a.qc[at] : 0.f;
+    }
     for (uint32_t i = t; i < TK_SEL_BINS; i += TK_SEL_NT) L.hist[i] = 0;
     if (t == 0) L.n = 0;
     __syncthreads();
     float qn = 0.f;  // |q|^2 as the estimates have it, each wave by itself
     {
-        float x = L.qv[t & 63u], y = L.qv[64u + (t & 63u)];
-        if constexpr (MODE != TK_SEL_KEPT) {
-            const float* c = a.qc + static_cast<size_t>(q) * a.dim;
-            x = (t & 63u) < a.dim ? c[t & 63u] : 0.f;
-            y = 64u + (t & 63u) < a.dim ? c[64u + (t & 63u)] : 0.f;
-        }
+        const float* v = MODE == TK_SEL_KEPT ? L.qv : L.qc;
+        const float x = v[t & 63u], y = v[64u + (t & 63u)];
         qn = x * x + y * y;
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) qn += __shfl_xor(qn, o, 64);
