@@ -13,13 +13,14 @@
 //      them.  A larger one runs it twice: over a strided sample, from which
 //      tk_select bounds each query's k-th distance, and then over every row,
 //      where each (query, row) whose estimate could lie at or below that bound
-//      is appended to the query's candidate lists.
+//      is appended to the query's candidate lists.  The second run takes rows
+//      and queries about a centre of the query block.
 //   3. tk_select: the candidates that can be in the answer get their fp32
 //      distance sum((q - x)^2), are ranked by (distance, id), and the first k
 //      are written.  Every returned distance is the direct one.
 // The estimates only ever gate, with a bound on their error, so the answer does
 // not depend on them.  When a query's candidate lists overflow (or the
-// small-set path is turned off), tk_dist and tk_merge answer: per-chunk sorted
+// estimates are turned off), tk_dist and tk_merge answer: per-chunk sorted
 // lists under an fp32 MFMA gate, merged by one wave per query.
 #include <algorithm>
 #include <atomic>
@@ -923,13 +924,15 @@ __global__ __launch_bounds__(TK_MERGE_NT) void tk_merge(TkArgs a, const float* l
 // counts take 256 queries a workgroup (QW 2, QG 4, eight waves, one a CU): the
 // tile's split and its reads are then shared by 256.  Up to 64 queries are bound
 // by reading the rows (QW 1, QG 2, four waves): two workgroups a CU, which do
-// not wait for each other's loads.
-// Measured (128 dimensions, 1024 queries): 483 us for a tenth of 10M rows, 1435 us
-// for 4M unfiltered ones, against 2505 us and ~9.5 ms of fp32 MFMA with sorted
-// lists; with all three products for every pair 706 us (the MFMAs alone 480 us:
-// 1.6 PFLOP/s, where the clock gives way to power).  Without the loads, 4M rows
-// take 980 us.  64 queries: 4M rows 315 us (6.1 TB/s of rows; 306 us with one
-// 128-row workgroup a CU), 300K x 100 33 us (36 us).
+// not wait for each other's loads; so are sets whose estimates are all kept.
+// Of the variants, QW 1's candidates of 97 to 128 dimensions with scalar row loads
+// spill (5 to 13 registers, compiler's report).
+// Measured (128 dimensions, 1024 queries, k 10, both stages of candidates): 543 us
+// for 822K of 10M rows, 1854 us for 4M unfiltered ones, against 2505 us and ~9.5 ms
+// of fp32 MFMA with sorted lists.  All three products for every pair took 706 us
+// of 1M rows when the test on hi.hi came in at 483 (the MFMAs alone 480: 1.6
+// PFLOP/s, where the clock gives way to power).  64 queries: 4M rows 372 us (5.5
+// TB/s of rows), 300K x 100 36 us.
 // The estimate's error against fp64, 32 x 32 blocks of 17 to 128 dimensions
 // (normal, positive, and over 2^20 of magnitudes), rms of |q|^2 + |x|^2:
 // 5.5e-8 to 1.45e-7, with fp32 MFMA 6.4e-8 to 1.73e-7 (lower in each block).
