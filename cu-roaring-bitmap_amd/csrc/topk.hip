@@ -1192,9 +1192,9 @@ __global__ __launch_bounds__((TkEst<KS, QW, QG>::NT)) __attribute__((amdgpu_wave
         moved = a.moved[qb] != 0;
         c_t = a.centre[qb * 128u + min(threadIdx.x, C::DP - 1u)];  // (written to LDS once the rows are on their way)
     }
-    // Candidates rarely need the queries' lo halves: they stay in LDS where
-    // registers are short.
-    constexpr bool QL_LDS = GATE && QW == 2;
+    // The queries' lo halves stay in LDS where registers are short (held there,
+    // the sample's kernel of 97 to 128 dimensions spilled 5 to 8, with scalar row loads 46).
+    constexpr bool QL_LDS = QW == 2;
     __shared__ alignas(16) _Float16 s_ql[QL_LDS ? C::QB * C::RS : 8];
     using Gate = TkGateLds<GATE ? C::QB : 1, GATE ? C::WAVES : 1>;
     __shared__ Gate G;
@@ -1302,6 +1302,11 @@ __global__ __launch_bounds__((TkEst<KS, QW, QG>::NT)) __attribute__((amdgpu_wave
     }
     __syncthreads();
 
+    auto lo_half = [&](int f, int s) -> f16x8 {  // of query fragment f, step s
+        if constexpr (QL_LDS) return *reinterpret_cast<const f16x8*>(&s_ql[(lq0 + 32u * f + j) * C::RS + 16u * s + 8u * h]);
+        else return ql[f][s];
+    };
+
     // The workgroup's lists (TK_SCRATCH bounds them: 32-bit offsets).
     uint2* cand = GATE ? a.cand + (static_cast<size_t>(chunk) * a.n_q + qb * C::QB) * a.cap : nullptr;
     uint32_t held = 0;  // candidates in the wave's buffer (uniform)
@@ -1355,13 +1360,18 @@ __global__ __launch_bounds__((TkEst<KS, QW, QG>::NT)) __attribute__((amdgpu_wave
                 const int s = GATE ? i : CROSS_FIRST ? (last ? i - 2 * KS : i / 2) : i / 3;
                 const int what = GATE || last ? 0 : CROSS_FIRST ? 1 + i % 2 : i % 3;  // hi.hi, lo.hi, hi.lo
                 f16x8& x = xh[!GATE && CROSS_FIRST ? s : 0];
+                f16x8 l8[QW];
+                if (what == 1) {
+#pragma unroll
+                    for (int f = 0; f < QW; ++f) l8[f] = lo_half(f, s);
+                }
                 if (GATE || (!last && (CROSS_FIRST ? i % 2 : i % 3) == 0)) {
                     x = *reinterpret_cast<const f16x8*>(H + 16 * s);
                     if (!GATE) xl = *reinterpret_cast<const f16x8*>(W + 16 * s);
                 }
 #pragma unroll
                 for (int f = 0; f < QW; ++f)
-                    acc[f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(what == 1 ? ql[QL_LDS ? 0 : f][QL_LDS ? 0 : s] : qh[f][s],
+                    acc[f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(what == 1 ? l8[f] : qh[f][s],
                                                                      what == 2 ? xl : x, acc[f], 0, 0, 0);
                 const int end = (i + 1) * TkSplit<C, VEC>::PIECES / PRODUCTS;
 #pragma unroll
@@ -1393,10 +1403,7 @@ __global__ __launch_bounds__((TkEst<KS, QW, QG>::NT)) __attribute__((amdgpu_wave
                     for (int s = 0; s < KS; ++s) {
                         const f16x8 x = *reinterpret_cast<const f16x8*>(H + 16 * s);
                         const f16x8 y = *reinterpret_cast<const f16x8*>(W + 16 * s);
-                        f16x8 l8;
-                        if constexpr (QL_LDS) l8 = *reinterpret_cast<const f16x8*>(&s_ql[(lq0 + 32u * f + j) * C::RS + 16u * s + 8u * h]);
-                        else l8 = ql[f][s];
-                        cross = __builtin_amdgcn_mfma_f32_32x32x16_f16(l8, x, cross, 0, 0, 0);
+                        cross = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo_half(f, s), x, cross, 0, 0, 0);
                         cross = __builtin_amdgcn_mfma_f32_32x32x16_f16(qh[f][s], y, cross, 0, 0, 0);
                     }
 #pragma unroll
