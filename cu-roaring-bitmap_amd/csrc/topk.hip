@@ -927,8 +927,8 @@ __global__ __launch_bounds__(TK_MERGE_NT) void tk_merge(TkArgs a, const float* l
 // not wait for each other's loads; so are sets whose estimates are all kept.
 // Of the variants, QW 1's candidates of 97 to 128 dimensions with scalar row loads
 // spill (5 to 13 registers, compiler's report).
-// Measured (128 dimensions, 1024 queries, k 10, both stages of candidates): 543 us
-// for 822K of 10M rows, 1854 us for 4M unfiltered ones, against 2505 us and ~9.5 ms
+// Measured (128 dimensions, 1024 queries, k 10, both stages of candidates): 550 us
+// for 822K of 10M rows, 1814 us for 4M unfiltered ones, against 2505 us and ~9.5 ms
 // of fp32 MFMA with sorted lists.  All three products for every pair took 706 us
 // of 1M rows when the test on hi.hi came in at 483 (the MFMAs alone 480: 1.6
 // PFLOP/s, where the clock gives way to power).  64 queries: 4M rows 372 us (5.5
