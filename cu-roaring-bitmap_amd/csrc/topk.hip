@@ -20,7 +20,8 @@
 //      are written.  Every returned distance is the direct one.
 // The estimates only ever gate, with a bound on their error, so the answer does
 // not depend on them.  When a query's candidate lists overflow (or the
-// estimates are turned off), tk_dist and tk_merge answer: per-chunk sorted
+// estimates are turned off, or its sample says that they would bound little),
+// tk_dist and tk_merge answer: per-chunk sorted
 // lists under an fp32 MFMA gate, merged by one wave per query.
 #include <algorithm>
 #include <atomic>
@@ -132,7 +133,7 @@ struct TkArgs {
     uint32_t parts;
     uint64_t* part_key;   // [n_q][parts][k] each part's best, ascending
     uint32_t* part_done;  // [n_q] parts finished
-    uint32_t* q_over;    // [n_q] the query's lists overflowed: tk_dist and tk_merge answer it
+    uint32_t* q_over;    // [n_q] the query's lists overflowed, or would: tk_dist and tk_merge answer it
     uint32_t* qb_over;   // [n_qb] ... any query of the block's
     // What the host launched, from the passing count it knew: with no
     // candidate kernels (or no list path), tk_select answers a set too large
@@ -926,7 +927,7 @@ __global__ __launch_bounds__(TK_MERGE_NT) void tk_merge(TkArgs a, const float* l
 // by reading the rows (QW 1, QG 2, four waves): two workgroups a CU, which do
 // not wait for each other's loads; so are sets whose estimates are all kept.
 // Of the variants, QW 1's candidates of 97 to 128 dimensions with scalar row loads
-// spill (5 to 13 registers, compiler's report).
+// spill (24 to 28 registers, compiler's report).
 // Measured (128 dimensions, 1024 queries, k 10, both stages of candidates): 550 us
 // for 822K of 10M rows, 1814 us for 4M unfiltered ones, against 2505 us and ~9.5 ms
 // of fp32 MFMA with sorted lists.  All three products for every pair took 706 us
@@ -1204,7 +1205,7 @@ __global__ __launch_bounds__((TkEst<KS, QW, QG>::NT)) __attribute__((amdgpu_wave
     const uint32_t h = lane >> 5, j = lane & 31u;
     const uint32_t lq0 = qg * 32u * QW;  // the wave's first query within the workgroup
     const uint32_t q0 = qb * C::QB + lq0;
-    const bool busy = q0 < a.n_q;  // wave-uniform
+    bool busy = q0 < a.n_q;  // wave-uniform
 
     // Tile t's rows are in set t & 1 of pre, with their ids.
     float pre[2][C::P][C::V];
@@ -1222,12 +1223,15 @@ __global__ __launch_bounds__((TkEst<KS, QW, QG>::NT)) __attribute__((amdgpu_wave
 
     // A operand: the wave's queries, split, positions 16 s + 8 h .. + 7 a lane.
     f16x8 qh[QW][KS], ql[QL_LDS ? 1 : QW][QL_LDS ? 1 : KS];
+    bool any = false;
     float vw[QW], vc[QW];  // the rank-2 product's query factors: sq (lanes 0-31), (gate - |q|^2) sq / 2 (lanes 32-63)
 #pragma unroll
     for (int f = 0; f < QW; ++f) {
         const uint32_t q = q0 + 32u * f + j;
-        const bool ok = q < a.n_q;
-        const float* src = a.queries + static_cast<size_t>(ok ? q : 0u) * a.dim;
+        const float* src = a.queries + static_cast<size_t>(q < a.n_q ? q : 0u) * a.dim;
+        // (a query that the list path is to answer takes no part)
+        const bool ok = q < a.n_q && !(GATE && !a.list_off && a.q_over[q]);
+        any = any || ok;
         float x[8 * KS];
         if (a.qvec) {
 #pragma unroll
@@ -1265,7 +1269,7 @@ __global__ __launch_bounds__((TkEst<KS, QW, QG>::NT)) __attribute__((amdgpu_wave
                 ql[f][s] = l8;
             }
         }
-        const float gate = GATE && ok ? __uint_as_float(a.tau[q]) : 0.f;
+        const float gate = GATE && q < a.n_q ? __uint_as_float(a.tau[q]) : 0.f;
         const bool pass = odd || !(gate < __builtin_inff());  // every row is a candidate
         const float qgn = (1.f - TK_EST_ERR) * ss;
         vw[f] = h == 0 ? (ok ? sq : 0.f) : !ok ? -__builtin_inff() : pass ? __builtin_inff() : 0.5f * (gate - qgn) * sq;
@@ -1300,7 +1304,12 @@ __global__ __launch_bounds__((TkEst<KS, QW, QG>::NT)) __attribute__((amdgpu_wave
 #pragma unroll
         for (int i = 0; i < TkSplit<C, VEC>::PIECES; ++i) split.piece(i, T0, pre[0], id[0], valid, a.dim);
     }
-    __syncthreads();
+    if (GATE && !a.list_off) {
+        busy = __ballot(any) != 0;
+        if (!__syncthreads_or(busy)) return;  // the list path answers the whole block
+    } else {
+        __syncthreads();
+    }
 
     auto lo_half = [&](int f, int s) -> f16x8 {  // of query fragment f, step s
         if constexpr (QL_LDS) return *reinterpret_cast<const f16x8*>(&s_ql[(lq0 + 32u * f + j) * C::RS + 16u * s + 8u * h]);
@@ -1495,6 +1504,11 @@ constexpr uint32_t TK_SEL_LISTS = 512;  // candidate lists a query has at most
 // four of them so far away that every row is a candidate, 7730 us without,
 // 958 us with; below, the parts' start and merge would be most of it.
 constexpr uint32_t TK_SEL_SPLIT = 16384;
+// The share of the sample in the gate from which a query goes to the list path.
+// 1024 queries in ten modes, as candidates / from 1/20 on / 1/50 / 1/100: 300K rows,
+// modes 30 deviations apart 562, 569, 559, 1385 us; 60 apart 2546, 1810, 1495, 1355;
+// 100 apart 2945, 1447, 1447, 1446.
+constexpr float TK_SEL_LIST = 1.f / 50;
 constexpr int TK_SEL_ROUNDS = 4;        // histograms beyond the first
 constexpr uint64_t TK_NOKEY = ~0ull;    // no candidate: after every (distance, id) key
 // The largest limit that cr_topk_set_small_limit records (any from the last of TK_KEEP_MAX on is no limit).
@@ -1551,13 +1565,15 @@ struct TkCentre {
     }
 
     // After a barrier: query q about the centre, and the block's by its first query.
-    __device__ __forceinline__ void write(const TkArgs& a, uint32_t q, const float* red, const float* qv)
+    __device__ __forceinline__ void write(const TkArgs& a, uint32_t q, const float* red, const float* qv, float* qc)
     {
         const uint32_t t = threadIdx.x;
         if (t >= 128) return;
         const bool moved = red[0] + red[1] + red[2] + red[3] > 0.0625f * (red[4] + red[5] + red[6] + red[7]);
         const float c = moved ? med : 0.f;
-        if (t < a.dim) a.qc[static_cast<size_t>(q) * a.dim + t] = qv[t] - c;
+        const float x = qv[t] - c;
+        qc[t] = t < a.dim ? x : 0.f;
+        if (t < a.dim) a.qc[static_cast<size_t>(q) * a.dim + t] = x;
         if (q % a.est_qb) return;
         a.centre[q / a.est_qb * 128u + t] = c;
         if (t == 0) a.moved[q / a.est_qb] = moved ? 1u : 0u;
@@ -1570,7 +1586,7 @@ struct TkSelLds {
     uint32_t hist[TK_SEL_BINS];
     uint32_t off[TK_SEL_LISTS + 1];
     float qv[128];
-    float qc[128];  // (candidates) the query about its block's centre
+    float qc[128];  // the query about its block's centre (where candidates are found)
     uint32_t lds[TK_SEL_W];
     float redf[2][TK_SEL_W];
     float redc[8];
@@ -1645,7 +1661,8 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
     // cardinality understates its set does that, and every row is then a
     // candidate (exact, slower; no estimate is read).
     bool all_rows = MODE == TK_SEL_KEPT && !small && a.cand_off;
-    const bool bound_only = MODE == TK_SEL_BOUND || (MODE == TK_SEL_KEPT && !small && !all_rows);
+    // (More than TK_KEEP rows are kept only where they are all there are.)
+    const bool bound_only = MODE == TK_SEL_BOUND || (MODE == TK_SEL_KEPT && V == tk_sel_v(TK_KEEP) && !small && !all_rows);
     for (uint32_t c = t; c < 128; c += TK_SEL_NT) {
         const size_t at = static_cast<size_t>(q) * a.dim + c;
         L.qv[c] = c < a.dim ? a.queries[at] : 0.f;
@@ -1699,8 +1716,10 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
                 if (tk_finite(e[c])) lo = fminf(lo, e[c]), hi = fmaxf(hi, e[c]);
         }
     } else {
-        uint32_t n = t < a.n_cw ? a.cand_n[static_cast<size_t>(t) * a.q_rows + q] : 0u;
-        const bool over = __syncthreads_or(n > a.cap);
+        const bool lists = !a.list_off && a.q_over[q];  // (nothing wrote its counts)
+        if (MODE == TK_SEL_BOUND && lists) return;
+        uint32_t n = t < a.n_cw && !lists ? a.cand_n[static_cast<size_t>(t) * a.q_rows + q] : 0u;
+        const bool over = __syncthreads_or(n > a.cap) || lists;
         n = min(n, a.cap);
         const uint32_t e = block_excl_scan<TK_SEL_NT>(n, L.lds, C);
         L.off[t] = e;
@@ -1741,7 +1760,7 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
         }
     }
     tk_block_range(L, lo, hi);
-    if (MODE == TK_SEL_KEPT && bound_only) centre.write(a, q, L.redc, L.qv);
+    if (MODE == TK_SEL_KEPT && bound_only) centre.write(a, q, L.redc, L.qv, L.qc);
     float scale = hi > lo ? static_cast<float>(TK_SEL_BINS) / (hi - lo) : 0.f;
     if constexpr (MODE == TK_SEL_KEPT) {
 #pragma unroll
@@ -1798,15 +1817,16 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
     // 3590 -> 1790 and 15.4 -> 3.6 ms.
     const bool near_first = MODE != TK_SEL_BOUND && !all_rows && bound < __builtin_inff() &&
                             ((again && bound > hi) || L.hist[tk_bin(bound, lo, scale)] > (bound_only ? 2 * a.k + 32u : few));
-    auto write_bound = [&]() {
+    auto write_bound = [&](bool lists) {
         if (t == 0) {
+            if (MODE == TK_SEL_KEPT) a.q_over[q] = lists ? 1u : 0u;
             a.tau[q] = __float_as_uint(MODE == TK_SEL_KEPT ? bound : fminf(bound, gate));
             if (MODE == TK_SEL_KEPT) a.tau_first[q] = __float_as_uint(bound), a.part_done[q] = 0;
             if (MODE == TK_SEL_KEPT && !a.list_off && q % TK_QB == 0) a.qb_over[q / TK_QB] = 0;
         }
     };
     if (bound_only && !near_first) {
-        write_bound();
+        write_bound(false);
         return;
     }
     if (all_rows) bound = __builtin_inff();
@@ -1919,6 +1939,22 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
         __syncthreads();  // every thread has read the count
         if (n > TK_SEL_CB - TK_SEL_NT) flush(n, MODE == TK_SEL_KEPT || all_rows);
     };
+    // Whether the list path is the better one from the start: of the sampled rows,
+    // more than TK_SEL_LIST pass the candidates' gate, or so many that the lists
+    // would overflow.  An estimate here lies about 2 E |q|^2 under the distance (the
+    // near rows' norms are the query's), the gate's about the centre 2 E |q'|^2.
+    auto too_many = [&]() -> bool {
+        float x = L.qc[t & 63u], y = L.qc[64u + (t & 63u)];
+        float qm = x * x + y * y;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) qm += __shfl_xor(qm, o, 64);
+        const float top = bound + 2.f * TK_EST_ERR * (qm - qn);
+        uint32_t n = 0;
+#pragma unroll 4
+        for (uint32_t i = t; i < S; i += TK_SEL_NT) n += a.pd[static_cast<size_t>(q) * a.pd_stride + i] <= top ? 1u : 0u;
+        n = block_sum<TK_SEL_NT>(n, L.lds);
+        return n > S * TK_SEL_LIST || static_cast<float>(n) * static_cast<float>(n_rows) > 0.7f * S * a.cap * a.n_cw;
+    };
     if (__builtin_expect(near_first, 0)) {
         // The rows up to the edge, TK_SEL_CB of them where ties make them more,
         // which bound the k-th distance as well.  They are taken again below.
@@ -1954,7 +1990,7 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
         __syncthreads();
         flush(min(L.n, TK_SEL_CB), MODE == TK_SEL_KEPT);
         if (bound_only) {
-            write_bound();
+            write_bound(MODE == TK_SEL_KEPT && !a.list_off && too_many());
             return;
         }
         nb = 0;
@@ -2183,6 +2219,7 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
     a.gate = limit > 0 && a.sample >= std::max<uint32_t>(1024, 8 * k);
     if (!a.gate) a.keep = 0;
     else a.keep = static_cast<uint32_t>(std::min<uint64_t>(a.keep, fit(a.q_rows)));
+    if (rows_ub > a.keep) a.keep = std::min(a.keep, TK_KEEP);
     a.pd_stride = std::max((a.keep + 63u) / 64u * 64u, a.sample);
     a.cand_off = a.gate && rows_ub <= a.keep;
     // Lists that hold every row a workgroup sees need no list path behind them.

@@ -230,6 +230,21 @@ def test_topk_two_far_modes(gpu, n_base, n_q, k):
     check_topk(base, queries[pick], k, None, got_d[pick], got_i[pick])
 
 
+def test_topk_four_far_modes(gpu):
+    """Rows and queries in four modes, none near the block's centre: every query goes
+    from the sample to the list path, but for a block whose queries share one mode."""
+    _say("topk four modes")
+    n_base, n_q = 600000, 300
+    base, queries = _data(n_base, n_q, 16, 60)
+    for m in range(4):
+        base[m::4, 4 * m:4 * m + 4] += 1000
+        queries[m:256:4, 4 * m:4 * m + 4] += 1000
+    queries[256:, :4] += 1000
+    got_d, got_i = _run(gpu, base, queries, 10, None)
+    pick = np.arange(0, n_q, 23)
+    check_topk(base, queries[pick], 10, None, got_d[pick], got_i[pick])
+
+
 @pytest.mark.parametrize("n_q,most", [(1, 80), (20, 160)])
 def test_topk_scratch_of_few_queries(gpu, n_q, most):
     """The candidate lists are sized for the queries there are and the candidates to
