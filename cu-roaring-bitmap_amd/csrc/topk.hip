@@ -105,6 +105,7 @@ struct TkArgs {
     uint32_t* list_id;  // the same two planes
     size_t plane;       // elements per plane
     uint32_t* list_n;   // [n_chunks][n_q]: list length | (plane holding the list << 31)
+    float* gate_at;       // [n_q] the candidates' gate: tau, or -inf for a query that the list path is to answer
     uint32_t* tau_first;  // [n_q] the sample's bound, at which the first candidates are rounded (tau may fall since)
     uint32_t* tau;      // [n_q] bits of the smallest k-th distance any chunk has reached
     uint32_t* tau_m;    // [n_chunks][n_q] bits of each chunk's m_rank-th distance (+inf: fewer entries)
@@ -927,7 +928,7 @@ __global__ __launch_bounds__(TK_MERGE_NT) void tk_merge(TkArgs a, const float* l
 // by reading the rows (QW 1, QG 2, four waves): two workgroups a CU, which do
 // not wait for each other's loads; so are sets whose estimates are all kept.
 // Of the variants, QW 1's candidates of 97 to 128 dimensions with scalar row loads
-// spill (24 to 28 registers, compiler's report).
+// spill (5 to 13 registers, compiler's report).
 // Measured (128 dimensions, 1024 queries, k 10, both stages of candidates): 550 us
 // for 822K of 10M rows, 1814 us for 4M unfiltered ones, against 2505 us and ~9.5 ms
 // of fp32 MFMA with sorted lists.  All three products for every pair took 706 us
@@ -1173,6 +1174,11 @@ __global__ __launch_bounds__((TkEst<KS, QW, QG>::NT)) __attribute__((amdgpu_wave
     const uint32_t pidx = (blockIdx.x % 8u) * (gridDim.x / 8u) + blockIdx.x / 8u;
     const uint32_t chunk = pidx / n_qb, qb = pidx % n_qb;
     if (chunk >= a.n_cw) return;
+    if (GATE && !a.list_off) {
+        const uint32_t q = qb * C::QB + threadIdx.x;
+        if (!__syncthreads_or(threadIdx.x < C::QB && q < a.n_q && a.gate_at[q] > -__builtin_inff()))
+            return;  // the list path answers the whole block
+    }
     const uint64_t all = (sp.n + C::T - 1) / C::T;
     const uint64_t first = (all + TK_STAGE - 1) / TK_STAGE;  // tiles of stage 1
     const uint64_t part = stage == 0 ? all : stage == 1 ? first : all - first;
@@ -1205,7 +1211,7 @@ __global__ __launch_bounds__((TkEst<KS, QW, QG>::NT)) __attribute__((amdgpu_wave
     const uint32_t h = lane >> 5, j = lane & 31u;
     const uint32_t lq0 = qg * 32u * QW;  // the wave's first query within the workgroup
     const uint32_t q0 = qb * C::QB + lq0;
-    bool busy = q0 < a.n_q;  // wave-uniform
+    const bool busy = q0 < a.n_q;  // wave-uniform
 
     // Tile t's rows are in set t & 1 of pre, with their ids.
     float pre[2][C::P][C::V];
@@ -1223,15 +1229,12 @@ __global__ __launch_bounds__((TkEst<KS, QW, QG>::NT)) __attribute__((amdgpu_wave
 
     // A operand: the wave's queries, split, positions 16 s + 8 h .. + 7 a lane.
     f16x8 qh[QW][KS], ql[QL_LDS ? 1 : QW][QL_LDS ? 1 : KS];
-    bool any = false;
     float vw[QW], vc[QW];  // the rank-2 product's query factors: sq (lanes 0-31), (gate - |q|^2) sq / 2 (lanes 32-63)
 #pragma unroll
     for (int f = 0; f < QW; ++f) {
         const uint32_t q = q0 + 32u * f + j;
         const float* src = a.queries + static_cast<size_t>(q < a.n_q ? q : 0u) * a.dim;
-        // (a query that the list path is to answer takes no part)
-        const bool ok = q < a.n_q && !(GATE && !a.list_off && a.q_over[q]);
-        any = any || ok;
+        const bool ok = q < a.n_q;
         float x[8 * KS];
         if (a.qvec) {
 #pragma unroll
@@ -1269,8 +1272,8 @@ __global__ __launch_bounds__((TkEst<KS, QW, QG>::NT)) __attribute__((amdgpu_wave
                 ql[f][s] = l8;
             }
         }
-        const float gate = GATE && q < a.n_q ? __uint_as_float(a.tau[q]) : 0.f;
-        const bool pass = odd || !(gate < __builtin_inff());  // every row is a candidate
+        const float gate = GATE && ok ? a.gate_at[q] : 0.f;  // (-inf: the list path answers the query, and no row passes)
+        const bool pass = (odd && gate > -__builtin_inff()) || !(gate < __builtin_inff());  // every row is a candidate
         const float qgn = (1.f - TK_EST_ERR) * ss;
         vw[f] = h == 0 ? (ok ? sq : 0.f) : !ok ? -__builtin_inff() : pass ? __builtin_inff() : 0.5f * (gate - qgn) * sq;
         vc[f] = h == 0 || !ok || pass ? vw[f] : 0.5f * (gate - qgn * TK_COARSE) * sq;
@@ -1304,12 +1307,7 @@ __global__ __launch_bounds__((TkEst<KS, QW, QG>::NT)) __attribute__((amdgpu_wave
 #pragma unroll
         for (int i = 0; i < TkSplit<C, VEC>::PIECES; ++i) split.piece(i, T0, pre[0], id[0], valid, a.dim);
     }
-    if (GATE && !a.list_off) {
-        busy = __ballot(any) != 0;
-        if (!__syncthreads_or(busy)) return;  // the list path answers the whole block
-    } else {
-        __syncthreads();
-    }
+    __syncthreads();
 
     auto lo_half = [&](int f, int s) -> f16x8 {  // of query fragment f, step s
         if constexpr (QL_LDS) return *reinterpret_cast<const f16x8*>(&s_ql[(lq0 + 32u * f + j) * C::RS + 16u * s + 8u * h]);
@@ -1820,7 +1818,9 @@ __global__ __launch_bounds__(TK_SEL_NT) void tk_select(TkArgs a, float* out_d, i
     auto write_bound = [&](bool lists) {
         if (t == 0) {
             if (MODE == TK_SEL_KEPT) a.q_over[q] = lists ? 1u : 0u;
-            a.tau[q] = __float_as_uint(MODE == TK_SEL_KEPT ? bound : fminf(bound, gate));
+            const float at = MODE == TK_SEL_KEPT ? bound : fminf(bound, gate);
+            a.tau[q] = __float_as_uint(at);
+            a.gate_at[q] = lists ? -__builtin_inff() : at;
             if (MODE == TK_SEL_KEPT) a.tau_first[q] = __float_as_uint(bound), a.part_done[q] = 0;
             if (MODE == TK_SEL_KEPT && !a.list_off && q % TK_QB == 0) a.qb_over[q / TK_QB] = 0;
         }
@@ -2263,6 +2263,7 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
     a.parts = n_q <= 64 ? std::max<uint32_t>(1, std::min<uint32_t>({64, 4 * cus / n_q, TK_SEL_CB / k})) : 1;
     const size_t o_pkey = cv.add(cands ? static_cast<size_t>(n_q) * a.parts * k * 8 : 0);
     const size_t o_pdone = cv.add(cands ? static_cast<size_t>(n_q) * 4 : 0);
+    const size_t o_gate_at = cv.add(cands ? static_cast<size_t>(n_q) * 4 : 0);
     const size_t o_tau_first = cv.add(cands ? static_cast<size_t>(n_q) * 4 : 0);
     const size_t o_candn = cv.add(cands ? static_cast<size_t>(a.q_rows) * a.n_cw * 4 : 0);
     const size_t o_qover = cv.add(cands ? static_cast<size_t>(n_q) * 4 : 0);
@@ -2282,6 +2283,7 @@ extern "C" int cr_topk_filtered(const float* d_base, uint64_t n_base, const floa
     a.moved = sc.at<uint32_t>(o_moved);
     a.part_key = sc.at<uint64_t>(o_pkey);
     a.part_done = sc.at<uint32_t>(o_pdone);
+    a.gate_at = sc.at<float>(o_gate_at);
     a.tau_first = sc.at<uint32_t>(o_tau_first);
     a.cand_n = sc.at<uint32_t>(o_candn);
     a.q_over = sc.at<uint32_t>(o_qover);
