@@ -230,6 +230,21 @@ def test_topk_two_far_modes(gpu, n_base, n_q, k):
     check_topk(base, queries[pick], k, None, got_d[pick], got_i[pick])
 
 
+@pytest.mark.parametrize("n_base,n_q", [(9000, 5), (24576, 70), (60000, 5), (60000, 300), (300000, 9)])
+@pytest.mark.parametrize("shift", [0.0, 300.0])
+def test_topk_equal_rows(gpu, shift, n_base, n_q):
+    """Every row the same: all estimates fall into one bin, more rows than a batch
+    holds lie at the edge, and the smallest ids are the answer."""
+    _say("topk equal rows", shift, n_base, n_q)
+    row, queries = _data(1, n_q, 40, 61)
+    base = np.repeat(row + np.float32(shift), n_base, axis=0)
+    got_d, got_i = _run(gpu, base, queries + np.float32(shift), 20, None)
+    assert np.array_equal(got_i, np.broadcast_to(np.arange(20), (n_q, 20)))
+    assert np.all(got_d == got_d[:, :1])
+    exact = ((base[0].astype(np.float64) - (queries + np.float32(shift)).astype(np.float64)) ** 2).sum(axis=1)
+    assert np.allclose(got_d[:, 0], exact, rtol=RTOL, atol=0)
+
+
 def test_topk_four_far_modes(gpu):
     """Rows and queries in four modes, none near the block's centre: every query goes
     from the sample to the list path, but for a block whose queries share one mode."""
